@@ -31,39 +31,96 @@ __device__ __forceinline__ T stream_load(const T* p) {
   return __builtin_nontemporal_load(p);
 }
 
-// ---- CSR, one lane per row ------------------------------------------------------
+// Workgroup of the CSR kernels in the order their rows are taken: workgroups are dealt to the
+// XCDs round-robin, so on grids of whole chunks (csr_grid) each XCD takes chunks of consecutive
+// workgroups (the mapping of bundle_walk) and neighbouring rows' x-gathers meet in its L2.
+__device__ __forceinline__ int csr_block() {
+  constexpr int C = (int)kXcdChunk;
+  if (gridDim.x % (unsigned)(kXcds * C) != 0) return (int)blockIdx.x;
+  const int p = blockIdx.x, i = p / kXcds;
+  return (i / C) * (kXcds * C) + (p % kXcds) * C + i % C;
+}
+
+// ---- CSR, one lane per row, products staged through LDS ----------------------------
+// A workgroup's rows are one contiguous run of entries: the lanes load it coalesced, kCsrUnroll
+// values, columns and gathers each in flight at once, and leave the rounded products in LDS; then
+// each lane adds its own row's products from there, left to right. The sum is the sequential one
+// bit for bit (product and add are separate roundings anyway). Walking a row per lane instead
+// makes every load of a wavefront touch 64 rows and waits for each entry in turn. Bound by HBM:
+// the 7-point 160^3 matrix (424 MB) takes 78 us, 5.5 TB/s (walk: 221 us, 1.9 TB/s); FP32 60 us.
+// kCsrStageRow: runs of more than this many entries a row on average keep the walk: with rows that
+// long a tile holds few of them, so most lanes would wait while a few add.
+constexpr int kCsrUnroll = 8;
+constexpr int kCsrTile = kCsrUnroll * kBlock;
+constexpr int kCsrStageRow = 64;
+
+// Row sum of row r0 + threadIdx.x (r0: the workgroup's first row, < n). Every lane of the
+// workgroup calls it.
+template <typename T>
+__device__ __forceinline__ T csr_row_sum(unsigned n, unsigned r0, const int* __restrict__ ro, const int* __restrict__ cols,
+                                         const T* __restrict__ vals, const T* __restrict__ x, T* prod) {
+  // unsigned: a tile's end may pass the largest int
+  const unsigned tid = threadIdx.x;
+  const unsigned kb = ro[min(r0 + tid, n)], ke = ro[min(r0 + tid + 1, n)];
+  const unsigned first = ro[r0], last = ro[min(r0 + kBlock, n)];
+  T acc = 0;
+  if (last - first > kCsrStageRow * kBlock) {
+    for (unsigned k = kb; k < ke; ++k) acc = acc + vals[k] * x[cols[k]];
+    return acc;
+  }
+  for (unsigned t0 = first; t0 < last; t0 += kCsrTile) {
+    int c[kCsrUnroll];
+    T v[kCsrUnroll];
+#pragma unroll
+    for (int u = 0; u < kCsrUnroll; ++u) {
+      const unsigned k = min(t0 + u * kBlock + tid, last - 1); // clamped: every load in bounds, none conditional
+      c[u] = stream_load(cols + k);
+      v[u] = stream_load(vals + k);
+    }
+#pragma unroll
+    for (int u = 0; u < kCsrUnroll; ++u) prod[u * kBlock + tid] = v[u] * x[c[u]];
+    __syncthreads();
+    const unsigned e = min(ke, t0 + kCsrTile);
+    for (unsigned k = max(kb, t0); k < e; ++k) acc = acc + prod[k - t0];
+    __syncthreads();
+  }
+  return acc;
+}
+
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_spmv_csr(int n, const int* __restrict__ ro,
                                                       const int* __restrict__ cols,
                                                       const T* __restrict__ vals,
                                                       const T* __restrict__ x, T* __restrict__ y) {
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  T acc = 0;
-  const int e = ro[i + 1];
-  for (int k = ro[i]; k < e; ++k) acc = acc + vals[k] * x[cols[k]];
-  y[i] = acc;
+  __shared__ T prod[kCsrTile];
+  const unsigned r0 = (unsigned)csr_block() * kBlock;
+  if (r0 >= (unsigned)n) return;
+  const T acc = csr_row_sum<T>(n, r0, ro, cols, vals, x, prod);
+  if (r0 + threadIdx.x < (unsigned)n) y[r0 + threadIdx.x] = acc;
 }
 
-// y = A x and out = y . x
+// y = A x and out = y . x (partials in row order, whatever the workgroups' order)
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_spmv_dot_csr(int n, const int* __restrict__ ro,
                                                           const int* __restrict__ cols,
                                                           const T* __restrict__ vals,
                                                           const T* __restrict__ x, T* __restrict__ y,
                                                           RedWork w) {
+  __shared__ T prod[kCsrTile];
   __shared__ double lds4[4];
+  const int block = csr_block();
+  const unsigned r0 = (unsigned)block * kBlock;
   double s = 0.0;
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i < n) {
-    T acc = 0;
-    const int e = ro[i + 1];
-    for (int k = ro[i]; k < e; ++k) acc = acc + vals[k] * x[cols[k]];
-    y[i] = acc;
-    s = (double)acc * (double)x[i];
+  if (r0 < (unsigned)n) {
+    const T acc = csr_row_sum<T>(n, r0, ro, cols, vals, x, prod);
+    const unsigned i = r0 + threadIdx.x;
+    if (i < (unsigned)n) {
+      y[i] = acc;
+      s = (double)acc * (double)x[i];
+    }
   }
-  double v[1] = {block_sum(s, lds4)};
-  store_partials<1>(v, w);
+  const double v = block_sum(s, lds4);
+  if (threadIdx.x == 0) w.partial[block] = v;
 }
 
 // ---- RB-CSR / RB-DIA --------------------------------------------------------------
@@ -359,6 +416,16 @@ struct Vec4<double> { typedef double4 type; typedef double2 half; };
 template <>
 struct Vec4<float> { typedef float4 type; typedef float2 half; };
 
+// kBsrRows block rows per workgroup, two lanes a block row (one per scalar row), the four rounded
+// products of each block staged through LDS as in csr_row_sum: the blocks' run is loaded coalesced
+// (32 bytes a lane in FP64), and each lane adds its own scalar row's products in the reference's
+// order (block by block, column 0 then 1): the sequential sum bit for bit. Bound by HBM: 97 x 93 x
+// 101 cells, 7 blocks a row (260 MB), 46 us, 5.6 TB/s (one lane a block row walking: 133 us, 2.0 TB/s). Runs of more than
+// kBsrStageRow blocks a block row keep the walk, one lane a block row.
+constexpr int kBsrRows = kBlock / 2;
+constexpr int kBsrUnroll = 4;
+constexpr int kBsrTile = kBsrUnroll * kBlock;
+constexpr int kBsrStageRow = 64;
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_spmv_bsr2(int nb, const int* __restrict__ ro,
                                                        const int* __restrict__ cols,
@@ -366,23 +433,64 @@ __global__ void __launch_bounds__(kBlock) k_spmv_bsr2(int nb, const int* __restr
                                                        const T* __restrict__ x, T* __restrict__ y) {
   typedef typename Vec4<T>::type V4;
   typedef typename Vec4<T>::half V2;
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= nb) return;
-  T y0 = 0, y1 = 0;
-  const int e = ro[i + 1];
-  for (int k = ro[i]; k < e; ++k) {
-    const V4 m = reinterpret_cast<const V4*>(vals)[k];
-    const V2 xv = reinterpret_cast<const V2*>(x)[cols[k]];
-    // row ieq = 0 then 1, columns iu = 0 then 1: m[ieq + 2 iu]
-    y0 = y0 + m.x * xv.x;
-    y0 = y0 + m.z * xv.y;
-    y1 = y1 + m.y * xv.x;
-    y1 = y1 + m.w * xv.y;
+  __shared__ V2 prod[2 * kBsrTile]; // block k of the tile: scalar row 0's products at 2 k, row 1's at 2 k + 1
+  const unsigned n = nb, r0 = (unsigned)csr_block() * kBsrRows;
+  if (r0 >= n) return;
+  const unsigned tid = threadIdx.x;
+  const unsigned first = ro[r0], last = ro[min(r0 + kBsrRows, n)];
+  if (last - first > kBsrStageRow * kBsrRows) {
+    const unsigned i = r0 + tid;
+    if (tid >= kBsrRows || i >= n) return;
+    T y0 = 0, y1 = 0;
+    const unsigned e = ro[i + 1];
+    for (unsigned k = ro[i]; k < e; ++k) {
+      const V4 m = reinterpret_cast<const V4*>(vals)[k];
+      const V2 xv = reinterpret_cast<const V2*>(x)[cols[k]];
+      // row ieq = 0 then 1, columns iu = 0 then 1: m[ieq + 2 iu]
+      y0 = y0 + m.x * xv.x;
+      y0 = y0 + m.z * xv.y;
+      y1 = y1 + m.y * xv.x;
+      y1 = y1 + m.w * xv.y;
+    }
+    V2 out;
+    out.x = y0;
+    out.y = y1;
+    reinterpret_cast<V2*>(y)[i] = out;
+    return;
   }
-  V2 out;
-  out.x = y0;
-  out.y = y1;
-  reinterpret_cast<V2*>(y)[i] = out;
+  const unsigned i = r0 + tid / 2, half = tid & 1;
+  const unsigned kb = ro[min(i, n)], ke = ro[min(i + 1, n)];
+  T acc = 0;
+  for (unsigned t0 = first; t0 < last; t0 += kBsrTile) {
+    int c[kBsrUnroll];
+    V4 m[kBsrUnroll];
+#pragma unroll
+    for (int u = 0; u < kBsrUnroll; ++u) {
+      const unsigned k = min(t0 + u * kBlock + tid, last - 1);
+      c[u] = stream_load(cols + k);
+      m[u] = reinterpret_cast<const V4*>(vals)[k];
+    }
+#pragma unroll
+    for (int u = 0; u < kBsrUnroll; ++u) {
+      const V2 xv = reinterpret_cast<const V2*>(x)[c[u]];
+      V2 p0, p1;
+      p0.x = m[u].x * xv.x;
+      p0.y = m[u].z * xv.y;
+      p1.x = m[u].y * xv.x;
+      p1.y = m[u].w * xv.y;
+      prod[2 * (u * kBlock + tid)] = p0;
+      prod[2 * (u * kBlock + tid) + 1] = p1;
+    }
+    __syncthreads();
+    const unsigned e = min(ke, t0 + kBsrTile);
+    for (unsigned k = max(kb, t0); k < e; ++k) {
+      const V2 p = prod[2 * (k - t0) + half];
+      acc = acc + p.x;
+      acc = acc + p.y;
+    }
+    __syncthreads();
+  }
+  if (i < n) y[2 * (size_t)i + half] = acc;
 }
 
 // ---- row-bundled 2x2 block CSR ("RB-BSR2") -------------------------------------------------
@@ -532,9 +640,15 @@ __global__ void __launch_bounds__(kBlock) k_invdiag_bellpack(int n, int slice, c
 // ---- launchers ---------------------------------------------------------------------------
 static inline dim3 rows_grid(long n) { return dim3((unsigned)((n + kBlock - 1) / kBlock)); }
 
+// Workgroups of the CSR kernels at `rows` rows each: whole XCD chunks (csr_block) once the rounding
+// adds at most a fourth.
+static inline dim3 csr_grid(long n, int rows) {
+  const long g = (n + rows - 1) / rows;
+  return dim3((unsigned)(g >= 4 * kXcds * kXcdChunk ? round_chunks(g) : g));
+}
 template <typename T>
 void launch_spmv_csr(hipStream_t st, int n, const int* ro, const int* cols, const T* vals, const T* x, T* y) {
-  if (n > 0) hipLaunchKernelGGL(k_spmv_csr<T>, rows_grid(n), dim3(kBlock), 0, st, n, ro, cols, vals, x, y);
+  if (n > 0) hipLaunchKernelGGL(k_spmv_csr<T>, csr_grid(n, kBlock), dim3(kBlock), 0, st, n, ro, cols, vals, x, y);
 }
 template <typename T>
 void launch_spmv_dot_csr(hipStream_t st, RedWork w, int n, const int* ro, const int* cols, const T* vals,
@@ -543,8 +657,8 @@ void launch_spmv_dot_csr(hipStream_t st, RedWork w, int n, const int* ro, const 
     launch_finalize(st, w, 0, 1, kFinStore, out, nullptr);
     return;
   }
-  hipLaunchKernelGGL(k_spmv_dot_csr<T>, rows_grid(n), dim3(kBlock), 0, st, n, ro, cols, vals, x, y, w);
-  launch_finalize(st, w, rows_grid(n).x, 1, kFinStore, out, nullptr);
+  hipLaunchKernelGGL(k_spmv_dot_csr<T>, csr_grid(n, kBlock), dim3(kBlock), 0, st, n, ro, cols, vals, x, y, w);
+  launch_finalize(st, w, rows_grid(n).x, 1, kFinStore, out, nullptr); // partials past the last row's are not read
 }
 template <typename T>
 void launch_spmv_rb(hipStream_t st, int n, RBMat<T> A, const T* x, T* y) {
@@ -706,7 +820,7 @@ void launch_addmult_csr(hipStream_t st, int n, int upper, double alpha, const in
 }
 template <typename T>
 void launch_spmv_bsr2(hipStream_t st, int nb, const int* ro, const int* cols, const T* vals, const T* x, T* y) {
-  if (nb > 0) hipLaunchKernelGGL(k_spmv_bsr2<T>, rows_grid(nb), dim3(kBlock), 0, st, nb, ro, cols, vals, x, y);
+  if (nb > 0) hipLaunchKernelGGL(k_spmv_bsr2<T>, csr_grid(nb, kBsrRows), dim3(kBlock), 0, st, nb, ro, cols, vals, x, y);
 }
 template <typename T>
 void launch_spmv_rbbsr2(hipStream_t st, int nbr, const int* bo, const int* bc, const T* bv, const T* x, T* y) {
