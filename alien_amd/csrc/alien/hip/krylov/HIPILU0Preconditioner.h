@@ -4,7 +4,8 @@
 // (src/core/alien/expression/krylov/ILU0Preconditioner.h:50-323), which work
 // on host pointers (y.data()) and so cannot run on device vectors. Here the
 // factorisation and both triangular sweeps run on the GPU over level-set
-// schedules built once on the host; the results are bit-exact with the
+// schedules built once on the host, or on pencils of grid lines where the
+// matrix is a full 7-point one; the results are bit-exact with the
 // sequential reference because each row performs the same operations in the
 // same order, after all the rows it reads are final.
 #pragma once
@@ -54,6 +55,7 @@ class ILU0Preconditioner<HIPInternalLinearAlgebra> {
       buildLevelSweeps(st, false); // the colour classes as the levels
       return;
     }
+    if (buildPencils(st)) return;
     std::vector<int> level(n);
     m_nl = alien_hip::host_levels(n, m_A.kcol(), m_A.cols(), m_A.dcol(), 0, level.data());
     m_lptr.resize(m_nl + 1);
@@ -69,7 +71,9 @@ class ILU0Preconditioner<HIPInternalLinearAlgebra> {
   }
   void update() {}
   void solve(AlgebraType& alg, const VectorType& y, VectorType& x) const {
-    if (levelOrdered())
+    if (m_pencil)
+      alien_hip::launch_pencil_apply<double>(alg.stream(), m_pen, y.data(), x.data());
+    else if (levelOrdered())
       alien_hip::launch_ilu0_solve_lev<double>(alg.stream(), m_nl, m_lptr.data(), d_lptr.data(), m_lsw, m_nu,
                                                m_uptr.data(), d_uptr.data(), m_usw, y.data(),
                                                const_cast<double*>(m_t.data()), x.data(), nullptr, sfWork());
@@ -121,9 +125,70 @@ class ILU0Preconditioner<HIPInternalLinearAlgebra> {
   // the level pointers on the device (the sweeps merge runs of small levels)
   const int* lowerPtrDevice() const { return d_lptr.data(); }
   const int* upperPtrDevice() const { return d_uptr.data(); }
-  const double* luValues() const { return d_lu.data(); }
+  // the factor in CSR order
+  const double* luValues() const {
+    if (m_pencil && d_lu.empty()) {
+      hipStream_t st = m_alg.stream();
+      d_lu.resize(m_A.getNnz());
+      ALIEN_HIP_CHECK(hipMemcpyAsync(d_lu.data(), m_A.d_vals.data(), sizeof(double) * m_A.getNnz(),
+                                     hipMemcpyDeviceToDevice, st));
+      alien_hip::launch_pencil_to_csr(st, m_A.getNRows(), m_pen, m_A.d_ro.data(), d_lu.data());
+      alien_hip::check_launch("ilu0 pencils to CSR");
+    }
+    return d_lu.data();
+  }
+  // Full 7-point matrices of lexicographic grids: the factor and its sweeps in pencils of grid lines
+  // (kernels/pencil.hip); no level sets are built then
+  bool pencils() const { return m_pencil; }
+  const alien_hip::PencilFactor<double>& pencilFactor() const { return m_pen; }
+  // the same factor in FP32, with its own faces and tickets
+  alien_hip::PencilFactor<float> pencilF32(hipStream_t st, alien_hip::DeviceArray<float>& vals,
+                                           alien_hip::DeviceArray<int>& work) const {
+    const alien_hip::PencilGrid& g = m_pen.g;
+    vals.resize(8 * g.positions() + 2 * g.halo());
+    work.resize(alien_hip::kPencilWork);
+    alien_hip::PencilFactor<float> F{g, vals.data(), vals.data() + 7 * g.positions(),
+                                     vals.data() + 8 * g.positions(), d_order.data(), work.data()};
+    alien_hip::launch_pencil_init<float>(st, F);
+    alien_hip::launch_pencil_demote(st, m_pen, F.base);
+    alien_hip::check_launch("ilu0 pencils (FP32)");
+    return F;
+  }
 
  private:
+  bool buildPencils(hipStream_t st) {
+    const int n = m_A.getNRows();
+    alien_hip::PencilGrid g;
+    m_pencil = false;
+    d_lu.reset();
+    if (!alien_hip::g_ilu_sync_free || !alien_hip::pencil_grid(n, m_A.kcol(), m_A.cols(), g)) return false;
+    const int zero[alien_hip::kPencilWork] = {0, 0, 0};
+    int bad[alien_hip::kPencilWork];
+    d_penwork.upload(zero, alien_hip::kPencilWork, st);
+    alien_hip::launch_pencil_check(st, n, g, m_A.d_ro.data(), m_A.d_cols.data(), d_penwork.data());
+    alien_hip::check_launch("ilu0 pencils check");
+    auto read = [&] {
+      ALIEN_HIP_CHECK(hipMemcpyAsync(bad, d_penwork.data(), sizeof(bad), hipMemcpyDeviceToHost, st));
+      ALIEN_HIP_CHECK(hipStreamSynchronize(st));
+    };
+    read();
+    if (bad[0]) return false;
+    const std::vector<int> order = alien_hip::pencil_order(g);
+    d_order.upload(order.data(), order.size(), st);
+    d_pen.resize(8 * g.positions() + 2 * g.halo());
+    m_pen = {g, d_pen.data(), d_pen.data() + 7 * g.positions(), d_pen.data() + 8 * g.positions(), d_order.data(),
+             d_penwork.data()};
+    alien_hip::DeviceArray<double> trans(3 * g.positions());
+    alien_hip::launch_pencil_init<double>(st, m_pen);
+    alien_hip::launch_pencil_factor(st, m_pen, m_A.d_ro.data(), m_A.d_vals.data(), trans.data(), false);
+    alien_hip::check_launch("ilu0 pencils factor");
+    read();
+    if (bad[2]) alien_hip::launch_pencil_factor(st, m_pen, m_A.d_ro.data(), m_A.d_vals.data(), trans.data(), true);
+    alien_hip::check_launch("ilu0 pencils factor");
+    ALIEN_HIP_CHECK(hipStreamSynchronize(st));
+    m_pencil = true;
+    return true;
+  }
   void factorize(hipStream_t st) {
     d_lptr.upload(m_lptr.data(), m_lptr.size(), st);
     d_uptr.upload(m_uptr.data(), m_uptr.size(), st);
@@ -190,8 +255,12 @@ class ILU0Preconditioner<HIPInternalLinearAlgebra> {
   int m_nl = 0, m_nu = 0;
   std::vector<int> m_lptr, m_uptr, m_colours;
   alien_hip::DeviceArray<int> d_lrows, d_urows, d_lptr, d_uptr;
-  alien_hip::DeviceArray<double> d_lu;
+  mutable alien_hip::DeviceArray<double> d_lu;
   VectorType m_t;
+  bool m_pencil = false;
+  alien_hip::PencilFactor<double> m_pen;
+  alien_hip::DeviceArray<double> d_pen;
+  alien_hip::DeviceArray<int> d_order, d_penwork;
 };
 
 } // namespace Alien

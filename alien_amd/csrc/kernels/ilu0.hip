@@ -14,6 +14,7 @@
 #include "../alien/hip/HIPContext.h"
 #include "device_common.h"
 #include "launch.h"
+#include "sync_free.h"
 
 namespace alien_hip {
 
@@ -374,20 +375,6 @@ void level_sf_shape(long n, long nlev, int& rpl, int& blocks) {
     blocks = (int)std::min(256L, std::max(64L, (b + kXcds - 1) / kXcds * kXcds));
   }
 }
-
-template <typename T> struct SfBits;
-template <> struct SfBits<double> {
-  typedef unsigned long long U;
-  static constexpr U kSentinel = 0x7ff4deadbeef0001ull; // a signalling NaN: never an arithmetic result
-  static __device__ __forceinline__ U bits(double v) { return (U)__double_as_longlong(v); }
-  static __device__ __forceinline__ double value(U b) { return __longlong_as_double((long long)b); }
-};
-template <> struct SfBits<float> {
-  typedef unsigned int U;
-  static constexpr U kSentinel = 0x7fa5deadu;
-  static __device__ __forceinline__ U bits(float v) { return __float_as_uint(v); }
-  static __device__ __forceinline__ float value(U b) { return __uint_as_float(b); }
-};
 
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_level_sf_fill(int n, T* out, int* work, const int* __restrict__ done) {

@@ -195,6 +195,48 @@ template <typename T>
 void launch_ilu0_solve_lev(hipStream_t, int nl, const int* lptr_host, const int* lptr_dev, LevelSweep<T> L, int nu,
                            const int* uptr_host, const int* uptr_dev, LevelSweep<T> U, const T* y, T* t, T* x,
                            const int* done = nullptr, int* sf_work = nullptr);
+// ILU(0) of a full 7-point matrix (every row holds exactly its in-grid neighbours) on an nx x ny x nz
+// lexicographic grid, in pencils of 8 x 8 lines (pencil.hip).
+struct PencilGrid {
+  int nx = 0, ny = 0, nz = 0;
+  int py = 0, pz = 0; // pencils in y and z
+  int steps = 0;      // steps of a pencil: nx + 14 rounded up
+  __host__ __device__ int pencils() const { return py * pz; }
+  __host__ __device__ long positions() const { return (long)py * pz * steps * 64; }
+  __host__ __device__ long halo() const { return 2L * py * pz * steps * 8; } // face values of one sweep
+  __host__ __device__ long position(int x, int y, int z) const {
+    const int yl = y % 8, zl = z % 8;
+    return ((long)(z / 8 * py + y / 8) * steps + x + yl + zl) * 64 + zl * 8 + yl;
+  }
+};
+constexpr int kPencilWork = 3; // tickets of the two sweeps, error flag
+template <typename T>
+struct PencilFactor {
+  PencilGrid g;
+  T* base = nullptr;            // 7 arrays of positions() entries: z-, y-, x-, diagonal, x+, y+, z+
+  T* t = nullptr;               // positions() entries: the lower sweep's result
+  T* halo = nullptr;            // 2 * halo() entries
+  const int* order = nullptr;   // pencils, each after those its lower sweep reads
+  int* work = nullptr;          // kPencilWork
+};
+// the grid of a host CSR whose first row and entry count are those of a full 7-point matrix, or
+// false; launch_pencil_check (*bad = 0 on entry) then compares every row
+bool pencil_grid(int n, const int* ro, const int* cols, PencilGrid& g);
+std::vector<int> pencil_order(const PencilGrid& g);
+void launch_pencil_check(hipStream_t, int n, const PencilGrid& g, const int* ro, const int* cols, int* bad);
+// empty faces, tickets and flag: before the first factorisation or apply
+template <typename T> void launch_pencil_init(hipStream_t, const PencilFactor<T>& F);
+// F.base from A's values, factorised; trans: 3 * positions() of workspace. F.work[2] is set
+// afterwards if a wait ran out of polls: call again with redo.
+void launch_pencil_factor(hipStream_t, const PencilFactor<double>& F, const int* ro, const double* vals,
+                          double* trans, bool redo);
+void launch_pencil_demote(hipStream_t, const PencilFactor<double>& F, float* base);
+// the factor in CSR order; lu: A's values on entry
+void launch_pencil_to_csr(hipStream_t, int n, const PencilFactor<double>& F, const int* ro, double* lu);
+// x = (LU)^-1 y; returns early once *done; may be captured
+template <typename T>
+void launch_pencil_apply(hipStream_t, const PencilFactor<T>& F, const T* y, T* x, const int* done = nullptr);
+
 template <typename T>
 void launch_ilu0_solve(hipStream_t, int nl, const int* lptr_host, const int* lrows, int nu,
                        const int* uptr_host, const int* urows, const int* ro, const int* cols, const int* dcol,

@@ -169,6 +169,10 @@ enum PrecKind {
 // Natural-order ILU(0) on its level-set schedules (the reference's ILU0 bit for bit):
 // one launch per level and sweep over the CSR of A and the factor in CSR order.
 struct LevelILU {
+  // a full 7-point matrix: the sweeps run in pencils (kernels/pencil.hip), the rest is unset
+  bool pencils = false;
+  PencilFactor<double> pen64;
+  PencilFactor<float> pen32;
   int nl = 0, nu = 0;
   const int* lptr = nullptr; // host
   const int* uptr = nullptr; // host
@@ -189,7 +193,7 @@ struct LevelILU {
 };
 // The sweeps run sync-free (a few launches per apply, no host call): a solve may capture them.
 inline bool level_sync_free(const LevelILU& L) {
-  return L.ordered && L.sf_work && g_ilu_sync_free && L.l64.nchunks > 0 && L.u64.nchunks > 0;
+  return L.pencils || (L.ordered && L.sf_work && g_ilu_sync_free && L.l64.nchunks > 0 && L.u64.nchunks > 0);
 }
 struct PrecondSpec {
   PrecKind kind = kPrecDiag;
@@ -283,6 +287,11 @@ template <> RBMat<float> PrecondSpec::g<float>() const { return g32; }
 template <> RBMat<float> PrecondSpec::gt<float>() const { return gt32; }
 template <typename T>
 void level_ilu_apply(hipStream_t s, const LevelILU& L, const T* y, T* t, T* x, const int* done) {
+  if (L.pencils) {
+    if constexpr (std::is_same<T, float>::value) launch_pencil_apply<float>(s, L.pen32, y, x, done);
+    else launch_pencil_apply<double>(s, L.pen64, y, x, done);
+    return;
+  }
   if (L.ordered) {
     if constexpr (std::is_same<T, float>::value)
       launch_ilu0_solve_lev<float>(s, L.nl, L.lptr, L.lptr_dev, L.l32, L.nu, L.uptr, L.uptr_dev, L.u32, y, t, x, done,
@@ -1275,6 +1284,7 @@ void solve_on(alien_hip_ctx* ctx, const alien_hip_solve_params* p, HIPMatrix& A,
       q.lu64 = lus.fill<double>(ctx->stream, A, ilu->luValues(), lus.lbv64, lus.ubv64, lus.d64);
     };
     DeviceArray<float> lev_lu32, lev_l32, lev_u32, lev_d32;
+    DeviceArray<int> lev_work32;
     if (p->precond == ALIEN_HIP_PREC_ILU0 && !(colours && !colours->empty())) {
       // natural order: the level-set factor and sweeps of the REFERENCE mode
       ilu.reset(new Alien::ILU0Preconditioner<Alg>(alg, A));
@@ -1282,30 +1292,36 @@ void solve_on(alien_hip_ctx* ctx, const alien_hip_solve_params* p, HIPMatrix& A,
       phase("ILU0 level-set factorisation");
       ps.kind = kPrecILU0Level;
       LevelILU& L = ps.lev;
-      L.nl = ilu->lowerLevels();
-      L.nu = ilu->upperLevels();
-      L.lptr = ilu->lowerPtr();
-      L.uptr = ilu->upperPtr();
-      L.lrows = ilu->lowerRows();
-      L.urows = ilu->upperRows();
-      L.lptr_dev = ilu->lowerPtrDevice();
-      L.uptr_dev = ilu->upperPtrDevice();
-      L.ro = A.d_ro.data();
-      L.cols = A.d_cols.data();
-      L.dcol = A.d_dcol.data();
-      L.lu64 = ilu->luValues();
-      L.ordered = ilu->levelOrdered();
-      if (L.ordered) {
-        L.l64 = ilu->lowerSweep();
-        L.u64 = ilu->upperSweep();
-        L.sf_work = ilu->sfWork();
-      }
-      if (mixed && L.ordered) {
-        ilu->fillSweepsF32(ctx->stream, lev_l32, lev_u32, lev_d32, L.l32, L.u32);
-      } else if (mixed) {
-        lev_lu32.resize(A.getNnz());
-        launch_demote(ctx->stream, A.getNnz(), ilu->luValues(), lev_lu32.data());
-        L.lu32 = lev_lu32.data();
+      L.pencils = ilu->pencils();
+      if (L.pencils) {
+        L.pen64 = ilu->pencilFactor();
+        if (mixed) L.pen32 = ilu->pencilF32(ctx->stream, lev_l32, lev_work32);
+      } else {
+        L.nl = ilu->lowerLevels();
+        L.nu = ilu->upperLevels();
+        L.lptr = ilu->lowerPtr();
+        L.uptr = ilu->upperPtr();
+        L.lrows = ilu->lowerRows();
+        L.urows = ilu->upperRows();
+        L.lptr_dev = ilu->lowerPtrDevice();
+        L.uptr_dev = ilu->upperPtrDevice();
+        L.ro = A.d_ro.data();
+        L.cols = A.d_cols.data();
+        L.dcol = A.d_dcol.data();
+        L.lu64 = ilu->luValues();
+        L.ordered = ilu->levelOrdered();
+        if (L.ordered) {
+          L.l64 = ilu->lowerSweep();
+          L.u64 = ilu->upperSweep();
+          L.sf_work = ilu->sfWork();
+        }
+        if (mixed && L.ordered) {
+          ilu->fillSweepsF32(ctx->stream, lev_l32, lev_u32, lev_d32, L.l32, L.u32);
+        } else if (mixed) {
+          lev_lu32.resize(A.getNnz());
+          launch_demote(ctx->stream, A.getNnz(), ilu->luValues(), lev_lu32.data());
+          L.lu32 = lev_lu32.data();
+        }
       }
     } else if (p->precond == ALIEN_HIP_PREC_ILU0) {
       ilu.reset(new Alien::ILU0Preconditioner<Alg>(alg, A));
