@@ -504,16 +504,25 @@ class HIPMatrix
   // for FP32 only (q = A p 100 us against 125 us).
   alien_hip::RBMat<double> rb64() const {
     if (m_fused_ell) return ellMat<double>(d_bellv.data());
-    return alien_hip::RBMat<double>{d_bo.data(), m_rbdia ? nullptr : d_bc.data(), d_bv.data(),
-                                    m_rbdia ? d_doff.data() : nullptr, m_rbdia ? d_dmask.data() : nullptr,
-                                    m_pair ? 1 : 0};
+    alien_hip::RBMat<double> a{d_bo.data(), m_rbdia ? nullptr : d_bc.data(), d_bv.data(),
+                               m_rbdia ? d_doff.data() : nullptr, m_rbdia ? d_dmask.data() : nullptr, m_pair ? 1 : 0};
+    setWidth(a);
+    return a;
   }
   alien_hip::RBMat<float> rb32() const {
     if (m_fused_ell) return ellMat<float>(d_bellv32.data());
     alien_hip::RBMat<float> a{d_bo.data(), m_rbdia ? nullptr : d_bc.data(), d_bv32.data(),
                               m_rbdia ? d_doff.data() : nullptr, m_rbdia ? d_dmask.data() : nullptr, m_pair ? 1 : 0};
     setUniform(a);
+    setWidth(a);
     return a;
+  }
+  // the widest bundle, for the matrices the resident CG may take (others keep the default)
+  template <typename T>
+  void setWidth(alien_hip::RBMat<T>& a) const {
+    if (m_n > alien_hip::kResidentMaxRows) return;
+    a.wmax = 0;
+    for (size_t b = 1; b < m_bo.size(); ++b) a.wmax = std::max(a.wmax, m_bo[b] - m_bo[b - 1]);
   }
   int uniformSlots() const { return m_uni; }
   template <typename T>

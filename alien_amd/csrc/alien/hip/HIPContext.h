@@ -171,6 +171,14 @@ struct alien_hip_ctx {
   alien_hip::DeviceArray<double> scalars; // device-resident scalar slots
   // zeroed CG state (done = 0, never written): the fused iteration's kernels launched on their own
   alien_hip::DeviceArray<alien_hip::CGState> idle_cg;
+  // slots and head of the grid-wide sums of the resident CG (cg_resident.hip), zeroed on first use
+  alien_hip::DeviceArray<unsigned long long> grid_slots;
+  alien_hip::DeviceArray<int> grid_head;
+  int device = 0, cus = 0; // the context's device and its compute units
+  // resident CG (cg_resident.hip): on / off (ALIEN_HIP_CG_RESIDENT at creation), polls of a wait
+  // before it gives up (ALIEN_HIP_CG_RESIDENT_SPINS)
+  bool cg_resident = true;
+  long resident_spins = 1L << 20;
   double* host_scalars = nullptr;          // pinned mirror of `scalars`
   // Pinned 512-byte blocks for the fused solvers' host state mirrors, allocated once per context
   // (pinned allocation and release cost far more than a solve's own host work); a solver takes a

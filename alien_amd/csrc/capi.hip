@@ -40,6 +40,12 @@ alien_hip_ctx* make_ctx(void* stream) {
     ALIEN_HIP_CHECK(hipMemsetAsync(c->scalars.data(), 0, sizeof(double) * alien_hip_ctx::kSlots, c->stream));
     c->idle_cg.resize(1);
     ALIEN_HIP_CHECK(hipMemsetAsync(c->idle_cg.data(), 0, sizeof(CGState), c->stream));
+    c->grid_slots.resize(kResidentWords);
+    c->grid_head.resize(2);
+    ALIEN_HIP_CHECK(hipMemsetAsync(c->grid_slots.data(), 0, sizeof(unsigned long long) * kResidentWords, c->stream));
+    ALIEN_HIP_CHECK(hipMemsetAsync(c->grid_head.data(), 0, 2 * sizeof(int), c->stream));
+    ALIEN_HIP_CHECK(hipGetDevice(&c->device));
+    ALIEN_HIP_CHECK(hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, c->device));
     ALIEN_HIP_CHECK(hipHostMalloc((void**)&c->host_scalars, sizeof(double) * alien_hip_ctx::kSlots,
                                   hipHostMallocDefault));
     ALIEN_HIP_CHECK(hipStreamSynchronize(c->stream));
@@ -56,6 +62,8 @@ void destroy_ctx(alien_hip_ctx* c) {
   c->partials.reset();
   c->scalars.reset();
   c->idle_cg.reset();
+  c->grid_slots.reset();
+  c->grid_head.reset();
   if (c->host_scalars) (void)hipHostFree(c->host_scalars);
   if (c->pinned_blocks) (void)hipHostFree(c->pinned_blocks);
   if (c->own_stream && c->stream) (void)hipStreamDestroy(c->stream);
@@ -138,6 +146,9 @@ int alien_hip_ctx_create(void* stream, alien_hip_ctx** out) {
   if (const char* e = std::getenv("ALIEN_HIP_ILU_SF_SPINS"))
     g_ilu_sf_spins = std::max(0L, std::strtol(e, nullptr, 10));
   *out = make_ctx(stream);
+  if (const char* e = std::getenv("ALIEN_HIP_CG_RESIDENT")) (*out)->cg_resident = std::atoi(e) != 0;
+  if (const char* e = std::getenv("ALIEN_HIP_CG_RESIDENT_SPINS"))
+    (*out)->resident_spins = std::max(0L, std::strtol(e, nullptr, 10));
   if (const char* e = std::getenv("ALIEN_HIP_TRACE")) (*out)->trace = std::atoi(e) != 0;
   API_END
 }

@@ -37,6 +37,7 @@ struct RBMat {
   int uni = 0;
   int nrows = 0;
   int uoff[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  int wmax = 1 << 30; // row-bundled: at least the widest bundle's slots
 };
 constexpr int kUniMaxSlots = 8;
 
@@ -146,6 +147,35 @@ void launch_factor_p(hipStream_t, RedWork w, int n, RBMat<T, V> G, RBMat<T, V> G
 template <typename T>
 void launch_factor_apply(hipStream_t, RedWork w, int n, RBMat<T> G, RBMat<T> GT, const T* r, T* tmp, T* z,
                          CGState* st);
+// CG iterations in one launch (cg_resident.hip), for systems of row-bundled diagonal offsets whose
+// rows the compute units hold in registers; Diag preconditioner, or Chebyshev of an order > 0.
+constexpr int kResidentMaxSlots = 7;    // entries per row
+constexpr int kResidentMaxBlocks = 256; // workgroups, one per compute unit
+constexpr int kResidentMaxRows = kResidentMaxBlocks * 2048;
+constexpr int kResidentSlots = kResidentMaxRows / 256; // workgroups of a row kernel, whose partials are summed
+constexpr int kResidentWords = 2 * kResidentSlots * 4;
+constexpr int kResidentMaxOrder = 8;
+struct ResidentCheb {
+  int order = 0;
+  double a[kResidentMaxOrder] = {}, b[kResidentMaxOrder] = {};
+};
+struct ResidentPlan {
+  int rows = 0;            // per lane
+  bool pairs = false;      // p.q is summed over pairs of bundles
+  bool one = false;        // one workgroup, its exchange in LDS
+  size_t lds = 0;
+  int exchange = 0; // vectors of workspace (none of memory with `one`)
+};
+// false: the system is not one of these
+template <typename T>
+bool resident_plan(int n, const RBMat<T>& A, int cus, int cheb_order, ResidentPlan& P);
+// ex: P.exchange vectors of n entries; slots: kResidentWords words and head: two ints, 0 before the
+// first launch; head[1] is set when a wait ran out of polls: x, r, z and p may then be a mixture,
+// the state is the one before. spins: polls of a wait. false: not launched.
+template <typename T>
+bool launch_cg_resident(hipStream_t, const ResidentPlan& P, int n, RBMat<T> A, const T* invd, T* x, T* r, T* z, T* p,
+                        T* ex, CGState* st, unsigned long long* slots, int* head, const ResidentCheb& cheb, int iters,
+                        int check, double below, long spins);
 void launch_fold_increment(hipStream_t, int n, float* x32, double* x);
 void launch_demote(hipStream_t, int n, const double* a, float* b);
 

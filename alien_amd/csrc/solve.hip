@@ -9,6 +9,7 @@
 #include <cmath>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <numeric>
 #include <type_traits>
 #include <vector>
@@ -341,6 +342,13 @@ struct ProgressWatch {
   }
 };
 
+// One resident launch at a time per device: two that each hold half of the compute units would wait
+// for each other. Held from the launch to the read of the state.
+std::mutex& resident_mutex(int device) {
+  static std::mutex m[64];
+  return m[device & 63];
+}
+
 template <typename T>
 struct FusedCG {
   alien_hip_ctx* ctx;
@@ -370,6 +378,53 @@ struct FusedCG {
     static_assert(sizeof(CGState) <= alien_hip_ctx::kPinnedBytes, "state mirror exceeds a pinned block");
     h_st = static_cast<CGState*>(ctx->take_pinned());
     if (!h_st) ALIEN_HIP_CHECK(hipHostMalloc((void**)&h_st, sizeof(CGState), hipHostMallocDefault));
+    const bool cheb = P.kind == kPrecCheb;
+    if ((cheb || P.kind == kPrecDiag) && ctx->cg_resident && !ctx->step_timing)
+      resident = resident_plan<T>(n, A, ctx->cus, cheb ? P.order : 0, res);
+    if (resident && cheb) {
+      res_cheb.order = P.order;
+      std::copy_n(P.a.begin(), P.order, res_cheb.a);
+      std::copy_n(P.b.begin(), P.order, res_cheb.b);
+    }
+    if (resident && !res.one) ex.resize((size_t)n * res.exchange);
+  }
+  // Small and middle-sized systems: the iterations run in one launch (cg_resident.hip) instead of
+  // being launched one by one or from a graph
+  bool resident = false;
+  ResidentPlan res;
+  ResidentCheb res_cheb;
+  DeviceArray<T> ex;
+  bool lost = false; // a resident launch gave up: x is valid, the recurrence is not (see restart)
+  // iterations until the device stop flag is raised, or to a multiple of `check` iterations with r.r
+  // below `below`; then the state
+  CGState advance_resident(T* x, int check, double below) {
+    const CGState before = *h_st;
+    const std::lock_guard<std::mutex> alone(resident_mutex(ctx->device));
+    if (!launch_cg_resident<T>(ctx->stream, res, n, A, invd, x, r.data(), z.data(), p.data(), ex.data(),
+                               st.data(), ctx->grid_slots.data(), ctx->grid_head.data(), res_cheb,
+                               kResidentIters, check, below, ctx->resident_spins)) {
+      resident = false;
+      return before;
+    }
+    const CGState cur = read_state();
+    if (!cur.done && cur.it == before.it) {
+      lost = true;
+      resident = false;
+      ALIEN_HIP_CHECK(hipMemsetAsync(ctx->grid_head.data() + 1, 0, sizeof(int), ctx->stream));
+    }
+    return cur;
+  }
+  // one launch at most runs this many iterations (tens of milliseconds)
+  static constexpr int kResidentIters = 4096;
+  // r holds the residual of x: begin a recurrence from it, the count going on
+  CGState restart(T* x, CGState h) {
+    lost = false;
+    h.done = 0;
+    h.status = 0;
+    write_state(h);
+    iteration(x, true);
+    check_launch("fused CG restart");
+    return read_state();
   }
   ~FusedCG() {
     release_graph();
@@ -493,10 +548,10 @@ struct FusedCG {
     return *h_st;
   }
 
+  // (the mirror is written again only after a read_state, which waits for this copy)
   void write_state(const CGState& h) {
     *h_st = h;
     ALIEN_HIP_CHECK(hipMemcpyAsync(st.data(), h_st, sizeof(CGState), hipMemcpyHostToDevice, ctx->stream));
-    ALIEN_HIP_CHECK(hipStreamSynchronize(ctx->stream));
   }
 
   // k loop iterations captured once in a hipGraph (re-captured if x changes)
@@ -525,7 +580,12 @@ struct FusedCG {
   // k more iterations (fewer if the device stop flag is raised), then the state. With step
   // timing on, the iterations are launched directly (events recorded by a graph's nodes carry
   // no timestamps here): the same kernels in the same order on the same stream.
-  CGState advance(T* x, bool graph, int k) {
+  // A resident system runs on, to the stop or to a multiple of k iterations with r.r below `below`.
+  CGState advance(T* x, bool graph, int k, double below = 0) {
+    if (resident) {
+      const CGState cur = advance_resident(x, k, below);
+      if (resident || lost) return cur;
+    }
     const bool timed = ctx->step_timing;
     const int it0 = h_st->it; // the state last read or written
     if (timed) ensure_timing_events(k);
@@ -569,6 +629,10 @@ struct FusedCG {
     ProgressWatch watch{stall_window};
     while (!cur.done) {
       cur = advance(x, graph, k);
+      if (lost) {
+        launch_residual<T>(s, ctx->red(), n, A, x, b, r.data(), ctx->dslot(slot));
+        cur = restart(x, cur);
+      }
       if (stall_window <= 0) continue;
       if (!std::isfinite(cur.rr) || (watch.stalled(cur.rr, cur.it) && !cur.done)) {
         *stalled = true;
@@ -687,6 +751,16 @@ MixedResult mixed_reliable_cg(alien_hip_ctx* ctx, int n, RBMat<double> A64, RBMa
   const int k = graph ? std::max(1, poll_every) : 1;
   ProgressWatch watch{stall_window};
   watch.stalled(rr64, 0);
+  auto advance = [&]() {
+    CGState c = F.advance(x32.data(), graph, k, d2 * rr_last);
+    if (!F.lost) return c;
+    // the increment is kept, its recurrence begun again from the true residual
+    launch_fold_increment(s, n, x32.data(), x);
+    launch_residual<double>(s, ctx->red(), n, A64, x, b, r64.data(), ctx->dslot(rslot));
+    c.rr = rr_last = ctx->read_slot(rslot);
+    launch_demote(s, n, r64.data(), F.r.data());
+    return F.restart(x32.data(), c);
+  };
   for (;;) {
     if (!std::isfinite(cur.rr)) {
       // the increment is lost; x holds the last reliable update
@@ -698,7 +772,7 @@ MixedResult mixed_reliable_cg(alien_hip_ctx* ctx, int n, RBMat<double> A64, RBMa
     const bool stall = stall_window > 0 && watch.stalled(cur.rr, cur.it);
     const bool update = cur.done || cur.rr < d2 * rr_last || stall;
     if (!update) {
-      cur = F.advance(x32.data(), graph, k);
+      cur = advance();
       continue;
     }
     // reliable update: x64 += x32, x32 = 0, r64 = b - A x64 in FP64
@@ -729,7 +803,7 @@ MixedResult mixed_reliable_cg(alien_hip_ctx* ctx, int n, RBMat<double> A64, RBMa
     F.write_state(cur);
     if (inside) F.resume_inside_step(x32.data());
     else F.residual_replaced();
-    cur = F.advance(x32.data(), graph, k);
+    cur = advance();
   }
   out.it = cur.it;
   return out;
