@@ -16,7 +16,7 @@
 // the device (resident_mutex); what else might hold one back too long runs the waits out of polls.
 // Bound by the latency of the sums, about 3 us each. An iteration of Jacobi-CG in FP64 against the
 // graph of launches: 14 x 11 x 9 cells 3.9 us (16), 32^3 5.6 (18), 64^3 8.5 (21), 80^3 (two rows per
-// lane, which spill) 21 (30); FP32 in the mixed solver 9.4 (19) at 64^3; Chebyshev of degree 3 17
+// lane, which spill) 21 (30); FP32 in the mixed solver 9.4 (19) at 64^3; Chebyshev of degree 3 16
 // (39) at 32^3. One sum per workgroup, with a tree of its own, took 7.7 us at 64^3, but its iterates
 // are not the launches'. Exchanging through barriers (stores settled, then a sum, then loads) took 10.4.
 #include "../alien_hip_internal.h"
@@ -317,6 +317,9 @@ __global__ void __launch_bounds__(kResBlock) k_cg_resident(int n, RBMat<T> A, co
 #pragma unroll
       for (int j = 0; j < K; ++j) there = there && u[j] != SfBits<T>::kSentinel;
       if (there || !(on[q] >> 31) || give_up(g, spins, &lds.failed)) break;
+      // (reads repeated at once hold up the very stores they wait for: Chebyshev steps of 6,000 to
+      // 18,000 rows took up to three times as long)
+      __builtin_amdgcn_s_sleep(16);
     }
 #pragma unroll
     for (int j = 0; j < K; ++j) out[j] = SfBits<T>::value(u[j]);
