@@ -174,6 +174,20 @@ struct alien_hip_ctx {
   // slots and head of the grid-wide sums of the resident CG (cg_resident.hip), zeroed on first use
   alien_hip::DeviceArray<unsigned long long> grid_slots;
   alien_hip::DeviceArray<int> grid_head;
+  // pivots (one per row) and ticket, flag of the ILU(0) kernels of ilu0_sync.hip
+  alien_hip::DeviceArray<double> ilu_piv;
+  alien_hip::DeviceArray<int> ilu_work;
+  // room for them; false where that would take an allocation inside a stream capture
+  bool reserve_ilu(size_t rows) {
+    if (ilu_work.size() == 2 && ilu_piv.size() >= rows) return true;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    ALIEN_HIP_CHECK(hipStreamIsCapturing(stream, &cap));
+    if (cap != hipStreamCaptureStatusNone) return false;
+    ALIEN_HIP_CHECK(hipStreamSynchronize(stream));
+    if (ilu_work.size() != 2) ilu_work.resize(2);
+    if (ilu_piv.size() < rows) ilu_piv.resize(rows);
+    return true;
+  }
   int device = 0, cus = 0; // the context's device and its compute units
   // resident CG (cg_resident.hip): on / off (ALIEN_HIP_CG_RESIDENT at creation), polls of a wait
   // before it gives up (ALIEN_HIP_CG_RESIDENT_SPINS)

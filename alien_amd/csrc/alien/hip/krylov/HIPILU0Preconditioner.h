@@ -195,8 +195,18 @@ class ILU0Preconditioner<HIPInternalLinearAlgebra> {
     d_lu.resize(m_A.getNnz());
     ALIEN_HIP_CHECK(hipMemcpyAsync(d_lu.data(), m_A.d_vals.data(), sizeof(double) * m_A.getNnz(),
                                    hipMemcpyDeviceToDevice, st));
-    alien_hip::launch_ilu0_factor<double>(st, m_nl, m_lptr.data(), d_lrows.data(), m_A.d_ro.data(),
-                                          m_A.d_cols.data(), m_A.d_dcol.data(), d_lu.data());
+    const int n = m_A.getNRows();
+    alien_hip::DeviceArray<double> piv;
+    alien_hip::DeviceArray<int> work;
+    if (alien_hip::sync_levels(n, m_nl)) {
+      piv.resize(n);
+      work.resize(2);
+      alien_hip::launch_sync_factor(st, n, m_nl, d_lrows.data(), m_A.d_ro.data(), m_A.d_cols.data(),
+                                    m_A.d_dcol.data(), d_lu.data(), piv.data(), work.data());
+    } else {
+      alien_hip::launch_ilu0_factor<double>(st, m_nl, m_lptr.data(), d_lrows.data(), m_A.d_ro.data(),
+                                            m_A.d_cols.data(), m_A.d_dcol.data(), d_lu.data());
+    }
     alien_hip::check_launch("ilu0_factor");
     m_alg.allocate(AlgebraType::resource(m_A), m_t);
     ALIEN_HIP_CHECK(hipStreamSynchronize(st));

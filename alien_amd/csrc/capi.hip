@@ -64,6 +64,8 @@ void destroy_ctx(alien_hip_ctx* c) {
   c->idle_cg.reset();
   c->grid_slots.reset();
   c->grid_head.reset();
+  c->ilu_piv.reset();
+  c->ilu_work.reset();
   if (c->host_scalars) (void)hipHostFree(c->host_scalars);
   if (c->pinned_blocks) (void)hipHostFree(c->pinned_blocks);
   if (c->own_stream && c->stream) (void)hipStreamDestroy(c->stream);
@@ -954,7 +956,10 @@ int alien_hip_ilu0_factor_f64(alien_hip_ctx* ctx, int n, const int* ro, const in
           "ilu0_factor_f64: bad arguments");
   REQUIRE(nlevels == 0 || (lptr_host[0] == 0 && lptr_host[nlevels] == n), "ilu0_factor_f64: schedule must cover the rows");
   API_BEGIN
-  launch_ilu0_factor<double>(ctx->stream, nlevels, lptr_host, lrows, ro, cols, dcol, lu);
+  if (sync_levels(n, nlevels) && ctx->reserve_ilu(n))
+    launch_sync_factor(ctx->stream, n, nlevels, lrows, ro, cols, dcol, lu, ctx->ilu_piv.data(), ctx->ilu_work.data());
+  else
+    launch_ilu0_factor<double>(ctx->stream, nlevels, lptr_host, lrows, ro, cols, dcol, lu);
   LAUNCHED("ilu0_factor_f64");
   API_END
 }
@@ -969,7 +974,11 @@ int alien_hip_ilu0_solve_f64(alien_hip_ctx* ctx, int n, const int* ro, const int
   REQUIRE(nl == 0 || (lptr[0] == 0 && lptr[nl] == n), "ilu0_solve_f64: lower schedule must cover the rows");
   REQUIRE(nu == 0 || (uptr[0] == 0 && uptr[nu] == n), "ilu0_solve_f64: upper schedule must cover the rows");
   API_BEGIN
-  launch_ilu0_solve<double>(ctx->stream, nl, lptr, lrows, nu, uptr, urows, ro, cols, dcol, lu, y, t, x);
+  const bool apart = std::abs(y - t) >= n && std::abs(x - t) >= n; // a sweep that overwrites its input goes level by level
+  if (apart && sync_levels(n, nl) && sync_levels(n, nu) && ctx->reserve_ilu(0))
+    launch_sync_solve(ctx->stream, n, nl, lrows, nu, urows, ro, cols, dcol, lu, y, t, x, ctx->ilu_work.data());
+  else
+    launch_ilu0_solve<double>(ctx->stream, nl, lptr, lrows, nu, uptr, urows, ro, cols, dcol, lu, y, t, x);
   LAUNCHED("ilu0_solve_f64");
   API_END
 }

@@ -195,6 +195,15 @@ template <typename T>
 void launch_ilu0_solve_lev(hipStream_t, int nl, const int* lptr_host, const int* lptr_dev, LevelSweep<T> L, int nu,
                            const int* uptr_host, const int* uptr_dev, LevelSweep<T> U, const T* y, T* t, T* x,
                            const int* done = nullptr, int* sf_work = nullptr);
+// ILU(0) over CSR arrays and level schedules in one launch each (ilu0_sync.hip), where sync_levels
+// says so: small levels. piv: n doubles, work: two ints of workspace. The sweeps write their results
+// over sentinels, so a sweep's output may not be its input (x may be y).
+bool sync_levels(int n, int nlevels);
+void launch_sync_factor(hipStream_t, int n, int nlevels, const int* rows, const int* ro, const int* cols,
+                        const int* dcol, double* lu, double* piv, int* work);
+void launch_sync_solve(hipStream_t, int n, int nl, const int* lrows, int nu, const int* urows, const int* ro,
+                       const int* cols, const int* dcol, const double* lu, const double* y, double* t, double* x,
+                       int* work);
 // ILU(0) of a full 7-point matrix (every row holds exactly its in-grid neighbours) on an nx x ny x nz
 // lexicographic grid, in pencils of 8 x 8 lines (pencil.hip).
 struct PencilGrid {
