@@ -22,6 +22,7 @@
 #include "device_common.h"
 #include "gnn.h"
 #include "launch.h"
+#include "wave_total.h"
 
 namespace alien_hip {
 namespace gnn {
@@ -383,50 +384,324 @@ __global__ void k_grad_ghat(int n, const int* __restrict__ ro, const int* __rest
 struct Coef4 {
   float c[4];
 };
-// per-column dot products X_c . Y_c into 4 partial slots
-__global__ void __launch_bounds__(256) k_dot4(int n, const float* __restrict__ X, const float* __restrict__ Y,
-                                              RedWork w) {
-  __shared__ double lds[4];
-  double a[4] = {0.0, 0.0, 0.0, 0.0};
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < n) {
+
+// Three launches a step forward, three in the reverse pass. One lane per row, its four columns in one 16-byte value.
+// Each element is computed by the operations and in the order of the separate products, dots and combinations it
+// stands for, a neighbour's element that has not been stored yet by the same operations again: the results do not
+// depend on the fusion. Step scalars stay on the device: a kernel that needs a dot product finalizes the partials of
+// the launch before (up to one wavefront's lanes of them; larger systems launch the finalize and read one total), and
+// its first workgroup keeps the value for later steps. When the host read every dot product back (64 of them on a
+// 16^3 system with 16 steps) and a step took 23 launches, that gradient took 3.70 ms; now 1.04. Dependent loads and
+// launch latency bound a launch: 3.9 us (products alone) to 6.5 (with a scalar to finalize first).
+struct Dot4 {
+  const double* p; // value c's partials at p[c * n ..)
+  int n;           // at most kWave
+};
+// the total of column lane % 4 (every lane of the wavefront calls it)
+__device__ __forceinline__ double dot_value(Dot4 d) {
+  const int lane = threadIdx.x & (kWave - 1);
+  double in[4], v[4];
 #pragma unroll
-    for (int c = 0; c < 4; ++c) a[c] = (double)X[(long)i * 4 + c] * (double)Y[(long)i * 4 + c];
-  }
-  double v[4];
+  for (int c = 0; c < 4; ++c) in[c] = lane < d.n ? 0.0 + d.p[c * d.n + lane] : 0.0;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) v[c] = 0.0 + wave_total(in[c]);
+  return lane & 2 ? (lane & 1 ? v[3] : v[2]) : (lane & 1 ? v[1] : v[0]);
+}
+// column lane % 4 of a kept scalar
+__device__ __forceinline__ double kept(const double* s) { return s[threadIdx.x & 3]; }
+__device__ __forceinline__ void keep(double* to, double v) {
+  if (blockIdx.x == 0 && threadIdx.x < 4) to[threadIdx.x] = v;
+}
+// the four columns' values of v, held by lanes 0..3
+__device__ __forceinline__ void columns(double v, float (&to)[4]) {
+  const int f = __float_as_int((float)v);
+#pragma unroll
+  for (int c = 0; c < 4; ++c) to[c] = __int_as_float(__builtin_amdgcn_readlane(f, c));
+}
+// per-column partials of X . Y of this workgroup's rows at part[c * stride + workgroup] (block_sum's tree,
+// the four columns in one pass); lds: 16 doubles, not read or written by the workgroup otherwise
+__device__ __forceinline__ void dot_partials(bool in, const float4& X, const float4& Y, double* part, int stride,
+                                             double* lds) {
+  const float x[4] = {X.x, X.y, X.z, X.w}, y[4] = {Y.x, Y.y, Y.z, Y.w};
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
-    v[c] = block_sum(a[c], lds);
-    __syncthreads();
+    const double s = wave_total(in ? (double)x[c] * (double)y[c] : 0.0);
+    if (lane == 0) lds[c * 4 + wave] = s;
   }
-  store_partials<4>(v, w);
-}
-// Y_c = a_c X_c + b_c Z_c (Z may be NULL; Y may alias X or Z)
-__global__ void k_lin4(int n, Coef4 a, const float* X, Coef4 b, const float* Z, float* Y) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long)n * 4) return;
-  const int c = (int)(t & 3);
-  float v = a.c[c] * X[t];
-  if (Z) v += b.c[c] * Z[t];
-  Y[t] = v;
-}
-// dL/dGhat_il += sum_c U_ic V_lc (+ W_ic X_lc) over the lower pattern (l <= i)
-__global__ void k_edge_acc4(int n, const int* __restrict__ ro, const int* __restrict__ cols,
-                            const int* __restrict__ dcol, const float* __restrict__ U, const float* __restrict__ V,
-                            const float* __restrict__ W, const float* __restrict__ X, float* __restrict__ gg) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  for (int k = ro[i]; k <= dcol[i]; ++k) {
-    const int l = cols[k];
-    float s = 0.f;
+  __syncthreads();
+  if (threadIdx.x < 4) {
+    double r = 0.0;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      s += U[(long)i * 4 + c] * V[(long)l * 4 + c];
-      if (W) s += W[(long)i * 4 + c] * X[(long)l * 4 + c];
-    }
-    gg[k] += s;
+    for (int q = 0; q < 4; ++q) r += lds[threadIdx.x * 4 + q];
+    part[(long)threadIdx.x * stride + blockIdx.x] = r;
   }
 }
+__device__ __forceinline__ float4 axpy4(float4 x, const float (&b)[4], float4 z) { // 1 x + b z
+  return make_float4(x.x + b[0] * z.x, x.y + b[1] * z.y, x.z + b[2] * z.z, x.w + b[3] * z.w);
+}
+__device__ __forceinline__ float4 scale4(const float (&a)[4], float4 x) {
+  return make_float4(a[0] * x.x, a[1] * x.y, a[2] * x.z, a[3] * x.w);
+}
+__device__ __forceinline__ float4 add4(float4 x, float4 y) { return make_float4(x.x + y.x, x.y + y.y, x.z + y.z, x.w + y.w); }
+__device__ __forceinline__ void mac4(float4& acc, float g, float4 v) {
+  acc.x += g * v.x;
+  acc.y += g * v.y;
+  acc.z += g * v.z;
+  acc.w += g * v.w;
+}
+struct CgRows { // the system and the factor
+  int n;
+  const int *ro, *cols, *dcol, *tpos;
+  const float *e, *ghat;
+};
+// Sum over the entries [b, e) of a row (b < e), in order, of coefficient(entry, column) * use(load(column)).
+// kBatch entries' columns are loaded together, then their coefficients and vectors; ready() is called
+// once, by every lane, with the first of these loads in flight: it waits for the step's scalars.
+// (One entry after the other, behind the scalars, took two or three round trips to memory an entry.)
+constexpr int kBatch = 8;
+template <typename C, typename L, typename R, typename U>
+__device__ __forceinline__ float4 row_sum(const int* __restrict__ cols, int b, int e, C coef, L load, R ready, U use) {
+  int j[kBatch];
+  float a[kBatch];
+  decltype(load(0)) v[kBatch];
+  float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+  auto fetch = [&] {
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) j[u] = cols[min(b + u, e - 1)];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) a[u] = coef(min(b + u, e - 1), j[u]);
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) v[u] = load(j[u]);
+  };
+  auto add = [&] {
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u)
+      if (b + u < e) mac4(acc, a[u], use(v[u]));
+  };
+  fetch();
+  ready();
+  add();
+  for (b += kBatch; b < e; b += kBatch) {
+    fetch();
+    add();
+  }
+  return acc;
+}
+// rows of Ahat, Ghat and Ghat^T
+template <typename L, typename R, typename U>
+__device__ __forceinline__ float4 ahat_row(const CgRows& A, int i, L load, R ready, U use) {
+  return row_sum(A.cols, A.ro[i], A.ro[i + 1], [&](int k, int j) { return j == i ? 1.f : -A.e[k]; }, load, ready, use);
+}
+template <typename L, typename R, typename U>
+__device__ __forceinline__ float4 ghat_row(const CgRows& A, int i, L load, R ready, U use) {
+  return row_sum(A.cols, A.ro[i], A.dcol[i] + 1, [&](int k, int) { return A.ghat[k]; }, load, ready, use);
+}
+template <typename L, typename R, typename U>
+__device__ __forceinline__ float4 ghat_t_row(const CgRows& A, int i, L load, R ready, U use) {
+  return row_sum(A.cols, A.dcol[i], A.ro[i + 1], [&](int k, int) { return A.ghat[A.tpos[k]]; }, load, ready, use);
+}
+struct Two4 {
+  float4 x, y;
+};
+// this lane's row; lanes past the last one work on it again and store nothing
+struct CgLane {
+  bool in;
+  int i;
+  __device__ __forceinline__ explicit CgLane(int n) {
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    in = t < n;
+    i = min(t, n - 1);
+  }
+};
+#define CG4_PLAIN [] {}, [](float4 v) { return v; }
+
+// T = Ghat^T R with T.T and R.R
+__global__ void __launch_bounds__(256) k_cg4_start(CgRows A, const float4* __restrict__ R, float4* __restrict__ T,
+                                                   double* tt, double* rr, int stride) {
+  __shared__ double lds[32];
+  const CgLane me(A.n);
+  const float4 r = R[me.i];
+  const float4 t = ghat_t_row(A, me.i, [&](int j) { return R[j]; }, CG4_PLAIN);
+  if (me.in) T[me.i] = t;
+  dot_partials(me.in, t, t, tt, stride, lds);
+  dot_partials(me.in, r, r, rr, stride, lds + 16);
+}
+// P = Ghat T, or P = Ghat T + (rho1 / rho) P0; keeps rho1
+__global__ void __launch_bounds__(256) k_cg4_dir(CgRows A, const float4* __restrict__ T, const float4* __restrict__ P0,
+                                                 Dot4 rho1, const double* __restrict__ rho, double* keep_rho1,
+                                                 float4* __restrict__ P) {
+  const CgLane me(A.n);
+  float4 p0 = make_float4(0.f, 0.f, 0.f, 0.f);
+  double r0 = 1.0;
+  if (P0) {
+    p0 = P0[me.i];
+    r0 = kept(rho);
+  }
+  float b[4];
+  const float4 z = ghat_row(A, me.i, [&](int j) { return T[j]; },
+                            [&] {
+                              const double r1 = dot_value(rho1);
+                              keep(keep_rho1, r1);
+                              columns(r1 / r0, b);
+                            },
+                            [](float4 v) { return v; });
+  if (me.in) P[me.i] = P0 ? axpy4(z, b, p0) : z;
+}
+// Q = Ahat P with P.Q
+__global__ void __launch_bounds__(256) k_cg4_ap(CgRows A, const float4* __restrict__ P, float4* __restrict__ Q,
+                                                double* pq, int stride) {
+  __shared__ double lds[16];
+  const CgLane me(A.n);
+  const float4 p = P[me.i];
+  const float4 q = ahat_row(A, me.i, [&](int j) { return P[j]; }, CG4_PLAIN);
+  if (me.in) Q[me.i] = q;
+  dot_partials(me.in, p, q, pq, stride, lds);
+}
+// R1 = R - (rho / sig) Q; T1 = Ghat^T R1 with T1.T1, or (T1 NULL) R1.R1; keeps sig
+__global__ void __launch_bounds__(256) k_cg4_res(CgRows A, const float4* __restrict__ R, const float4* __restrict__ Q,
+                                                 const double* __restrict__ rho, Dot4 sig, double* keep_sig,
+                                                 float4* __restrict__ R1, float4* __restrict__ T1, double* dot,
+                                                 int stride) {
+  __shared__ double lds[16];
+  const CgLane me(A.n);
+  const float4 r0 = R[me.i], q0 = Q[me.i];
+  const double rh = kept(rho);
+  float na[4];
+  auto scalars = [&] {
+    const double sg = dot_value(sig);
+    keep(keep_sig, sg);
+    columns(-(rh / sg), na);
+  };
+  float4 d;
+  if (T1) {
+    d = ghat_t_row(A, me.i, [&](int j) { return Two4{R[j], Q[j]}; }, scalars,
+                   [&](Two4 v) { return axpy4(v.x, na, v.y); });
+    if (me.in) T1[me.i] = d;
+  } else {
+    scalars();
+  }
+  const float4 r = axpy4(r0, na, q0);
+  if (me.in) R1[me.i] = r;
+  if (!T1) d = r;
+  dot_partials(me.in, d, d, dot, stride, lds);
+}
+// reverse: rbar = (2 / (4 rrk)) R with Q.rbar
+__global__ void __launch_bounds__(256) k_cg4_rev_start(int n, Coef4 c0, const float4* __restrict__ R,
+                                                       const float4* __restrict__ Q, float4* __restrict__ rbar,
+                                                       double* qr, int stride) {
+  __shared__ double lds[16];
+  const CgLane me(n);
+  const float4 r = scale4(c0.c, R[me.i]), q = Q[me.i];
+  if (me.in) rbar[me.i] = r;
+  dot_partials(me.in, q, r, qr, stride, lds);
+}
+// z = Ghat t, rho = t.t: tbar = 2 rhobar T + Ghat^T pbar, with rhobar = rhobar_next + betabar / rho (or
+// rhobar_next alone: rho NULL); keeps what rho's own adjoint takes from beta, -betabar rho1 / rho^2
+__global__ void __launch_bounds__(256) k_cg4_rev_t(CgRows A, const float4* __restrict__ pbar, const float4* __restrict__ T,
+                                                   const double* __restrict__ rhobar_next, Dot4 betabar,
+                                                   const double* __restrict__ rho, const double* __restrict__ rho1,
+                                                   double* keep_own, float4* __restrict__ tbar) {
+  const CgLane me(A.n);
+  const float4 own = T[me.i];
+  float two[4];
+  const float4 t = ghat_t_row(A, me.i, [&](int j) { return pbar[j]; },
+                              [&] {
+                                double rb = kept(rhobar_next);
+                                if (rho) {
+                                  const double r = kept(rho), r1 = kept(rho1), bb = dot_value(betabar);
+                                  rb = rb + bb / r;
+                                  keep(keep_own, 0.0 - bb * r1 / (r * r));
+                                }
+                                columns(2.0 * rb, two);
+                              },
+                              [](float4 v) { return v; });
+  if (me.in) tbar[me.i] = add4(scale4(two, own), t);
+}
+// t = Ghat^T r, z = Ghat t: dL/dGhat += pbar T^T + R tbar^T over the lower pattern; rbar += Ghat tbar
+// with Q.rbar (rbar NULL: the first residual, fixed)
+__global__ void __launch_bounds__(256) k_cg4_rev_r(CgRows A, const float4* __restrict__ pbar, const float4* __restrict__ T,
+                                                   const float4* __restrict__ R, const float4* __restrict__ tbar,
+                                                   float* __restrict__ gg, float4* __restrict__ rbar,
+                                                   const float4* __restrict__ Q, double* qr, int stride) {
+  __shared__ double lds[16];
+  constexpr int kHalf = kBatch / 2; // two vectors an entry
+  const CgLane me(A.n);
+  const float4 u = pbar[me.i], w = R[me.i];
+  float4 r = make_float4(0.f, 0.f, 0.f, 0.f), q = r, acc = r;
+  if (rbar) {
+    r = rbar[me.i];
+    q = Q[me.i];
+  }
+  const int e = A.dcol[me.i] + 1;
+  for (int k = A.ro[me.i]; k < e; k += kHalf) {
+    float4 v[kHalf], x[kHalf];
+    float g[kHalf], old[kHalf];
+#pragma unroll
+    for (int m = 0; m < kHalf; ++m) {
+      const int km = min(k + m, e - 1), l = A.cols[km];
+      v[m] = T[l];
+      x[m] = tbar[l];
+      g[m] = A.ghat[km];
+      old[m] = gg[km];
+    }
+#pragma unroll
+    for (int m = 0; m < kHalf; ++m) {
+      if (k + m >= e) continue;
+      float s = 0.f;
+      s += u.x * v[m].x;
+      s += w.x * x[m].x;
+      s += u.y * v[m].y;
+      s += w.y * x[m].y;
+      s += u.z * v[m].z;
+      s += w.z * x[m].z;
+      s += u.w * v[m].w;
+      s += w.w * x[m].w;
+      if (me.in) gg[k + m] = old[m] + s;
+      mac4(acc, g[m], x[m]);
+    }
+  }
+  if (!rbar) return;
+  r = add4(r, acc);
+  if (me.in) rbar[me.i] = r;
+  dot_partials(me.in, q, r, qr, stride, lds);
+}
+// r1 = r - alpha q, q = Ahat p: qbar = -alpha rbar + sigbar P; pbar = (beta pbar + sigbar Q) + Ahat qbar (beta =
+// rho1 / rho; rho1 NULL: no direction follows) with pbar.P0; keeps rhobar = own + alphabar / sig (alphabar = -Q.rbar)
+__global__ void __launch_bounds__(256) k_cg4_rev_p(CgRows A, const float4* __restrict__ rbar, const float4* __restrict__ P,
+                                                   const float4* __restrict__ Q, const double* __restrict__ rho,
+                                                   const double* __restrict__ rho1, const double* __restrict__ sig,
+                                                   Dot4 qr, const double* __restrict__ own, double* keep_rhobar,
+                                                   float4* __restrict__ pbar, const float4* __restrict__ P0,
+                                                   double* betabar, int stride) {
+  __shared__ double lds[16];
+  const CgLane me(A.n);
+  float4 p = make_float4(0.f, 0.f, 0.f, 0.f), p0 = p;
+  const float4 q = Q[me.i];
+  const double r0 = kept(rho), sg = kept(sig);
+  double r1 = 0.0, ow = 0.0;
+  if (rho1) {
+    r1 = kept(rho1);
+    ow = kept(own);
+    p = pbar[me.i];
+  }
+  if (P0) p0 = P0[me.i];
+  float na[4], sb[4], be[4];
+  const float4 t = ahat_row(A, me.i, [&](int j) { return Two4{rbar[j], P[j]}; },
+                            [&] {
+                              const double alphabar = -dot_value(qr);
+                              keep(keep_rhobar, ow + alphabar / sg);
+                              columns(-alphabar * r0 / (sg * sg), sb);
+                              columns(-(r0 / sg), na);
+                              columns(r1 / r0, be);
+                            },
+                            [&](Two4 v) { return add4(scale4(na, v.x), scale4(sb, v.y)); });
+  if (rho1) p = scale4(be, p);
+  p = add4(axpy4(p, sb, q), t);
+  if (me.in) pbar[me.i] = p;
+  if (P0) dot_partials(me.in, p, p0, betabar, stride, lds);
+}
+#undef CG4_PLAIN
 
 // head backward: do_i = g_ii ghat_ii, dc_ij = g_ij e_ij;
 // dh_i = do_i w_d + sum_{j<i} dc_ij w_a + sum_{m>i} dc_mi w_b ; per-row parameter-gradient terms
@@ -465,37 +740,10 @@ __global__ void k_head_bwd(int n, const int* __restrict__ ro, const int* __restr
   pr[3 * kHidden + 1] = sa;            // c_e (each lower edge counted once, in its row)
 }
 
-// dense layer backward: dz = dh * (z > 0) ; du = dz W^T (W bf16-rounded) ;
-// dh_prev = dh + du[:, :32] (the E du[:, 32:] part is added by k_aggregate_add) ; dmsg = du[:, 32:]
-template <int KIN>
-__global__ void k_dense_bwd(int n, const float* __restrict__ dh, const float* __restrict__ Z, const float* __restrict__ W,
-                            int kin, float* __restrict__ dz, float* __restrict__ dh_prev, float* __restrict__ dmsg) {
-  __shared__ float Ws[KIN * kHidden];
-  for (int t = threadIdx.x; t < KIN * kHidden; t += blockDim.x)
-    Ws[t] = (t / kHidden < kin) ? bf16_round(W[t]) : 0.f;
-  __syncthreads();
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  float d[kHidden];
-#pragma unroll
-  for (int q = 0; q < kHidden; ++q) {
-    const long o = (long)i * kHidden + q;
-    d[q] = Z[o] > 0.f ? dh[o] : 0.f;
-    dz[o] = d[q];
-  }
-  if (!dh_prev) return;
-  for (int k = 0; k < kin; ++k) {
-    float s = 0.f;
-#pragma unroll
-    for (int q = 0; q < kHidden; ++q) s += d[q] * Ws[k * kHidden + q];
-    if (k < kHidden) dh_prev[(long)i * kHidden + k] = dh[(long)i * kHidden + k] + s;
-    else dmsg[(long)i * kHidden + (k - kHidden)] = s;
-  }
-}
-
-// The same for the message-passing layers (kin = 64) on MFMA: du = dz W^T is a 32-row x 64 x 32
-// product per wave, 2 output tiles of 16 v_mfma_f32_32x32x2_f32 steps (FP32 operands: dz and the
-// bf16-rounded weights, as in the scalar form; only the summation order of the 32 terms differs).
+// dense layer backward (message-passing layers, kin = 64): dz = dh * (z > 0) ; du = dz W^T (W bf16-rounded) ;
+// dh_prev = dh + du[:, :32] (the E du[:, 32:] part is added by k_aggregate_add) ; dmsg = du[:, 32:].
+// On MFMA: du is a 32-row x 64 x 32 product per wave, 2 output tiles of 16 v_mfma_f32_32x32x2_f32
+// steps (FP32 operands: dz and the bf16-rounded weights).
 // Each wave stages its 32 rows of dh and dz in LDS (16-byte loads), the workgroup the weights.
 __global__ void __launch_bounds__(256) k_dense_bwd_mfma(int n, const float* __restrict__ dh,
                                                         const float* __restrict__ Z, const float* __restrict__ W,
@@ -553,90 +801,193 @@ __global__ void __launch_bounds__(256) k_dense_bwd_mfma(int n, const float* __re
   }
 }
 
-// dh[i] += sum_{j != i} e_ji dmsg[j]   (E^T dmsg; e_ji read at the transpose position)
+// dh[i] += sum_{j != i} e_ji dmsg[j]   (E^T dmsg; e_ji read at the transpose position); lanes, rows and
+// order of the sums as in k_aggregate (one lane per feature took 563 us at 96^3, this 192)
 __global__ void __launch_bounds__(256) k_aggregate_add(int n, const int* __restrict__ ro, const int* __restrict__ cols,
                                                        const int* __restrict__ tpos, const float* __restrict__ e,
                                                        const float* __restrict__ dmsg, float* __restrict__ dh) {
-  const long t = (long)blockIdx.x * 256 + threadIdx.x;
-  const int i = (int)(t >> 5);
-  const int c = (int)(t & 31);
+  const int p = blockIdx.x, q = p / kXcds;
+  const int logical = (q / kAggChunk) * (kXcds * kAggChunk) + (p % kXcds) * kAggChunk + q % kAggChunk;
+  const int i = logical * kAggRows + (threadIdx.x >> 3);
+  const int c4 = threadIdx.x & 7;
   if (i >= n) return;
-  float acc = 0.f;
+  float4 acc = {0.f, 0.f, 0.f, 0.f};
+  const float4* __restrict__ d4 = reinterpret_cast<const float4*>(dmsg);
   for (int k = ro[i]; k < ro[i + 1]; ++k) {
     const float w = e[tpos[k]];
-    if (w != 0.f) acc += w * dmsg[(long)cols[k] * kHidden + c];
+    if (w != 0.f) {
+      const float4 v = d4[(long)cols[k] * (kHidden / 4) + c4];
+      acc.x += w * v.x;
+      acc.y += w * v.y;
+      acc.z += w * v.z;
+      acc.w += w * v.w;
+    }
   }
-  dh[(long)i * kHidden + c] += acc;
+  float4* __restrict__ to = reinterpret_cast<float4*>(dh) + (long)i * (kHidden / 4) + c4;
+  const float4 h = *to;
+  *to = make_float4(h.x + acc.x, h.y + acc.y, h.z + acc.z, h.w + acc.w);
 }
 
-// weight-gradient partials: per workgroup of 256 rows, sum_r bf16(X_r) (x) dz_r  (kin x 32) and sum_r dz_r (32)
-template <int KIN>
+// Weight-gradient partials: per 256 rows, sum_r bf16(X_r) (x) dz_r  (kin x 32) and sum_r dz_r (32), with
+// dz = dz_r where Zm is NULL and dz_r masked by Zm > 0 otherwise.
+// Per output FP32 sums of 32 rows, added in FP64 in row order. A workgroup takes COLS of the input columns; the
+// KGRP workgroups that share the rows' dz run on one XCD, whose L2 serves it. All 256 rows are loaded at once
+// (the loads' latency bounds a small system); then each half-wave sums one chunk of 32 rows, a lane
+// a tile of COLS / 4 columns x 4 outputs (1 + COLS / 16 16-byte LDS reads for COLS multiply-adds: one output
+// a lane read LDS twice for each and was bound by that on large systems).
+// One workgroup for all 64 columns, staging 32 rows at a time, left a 16^3 system's layer on 16 CUs:
+// 55 us, 367 at 96^3; this takes 7.1 us at 20^3 and 190 at 96^3.
+constexpr int kWgChunk = 32;
+// All 64 columns in 8 workgroups of 8 on small systems (latency: 7.2 us against 11.9 at 20^3, 32 row blocks), in 2 of 32 from
+// this many row blocks on (dz read twice, not 8 times); 14.4 against 15.0 us at 128 blocks, 20.8 against 20.2 at 250.
+constexpr long kWgradWide = 256;
+template <int KIN, int COLS>
 __global__ void __launch_bounds__(256) k_wgrad_partials(int n, const float* __restrict__ X0, int ld0, int c0,
                                                         const float* __restrict__ X1, int ld1, int kin,
-                                                        const float* __restrict__ dz, double* __restrict__ part,
-                                                        int cap) {
-  constexpr int NOUT = KIN * kHidden + kHidden;
-  constexpr int CH = 32; // rows staged per chunk
-  __shared__ float xs[CH][KIN];
-  __shared__ float ds[CH][kHidden];
-  const int r0 = blockIdx.x * 256;
-  double acc[(NOUT + 255) / 256];
+                                                        const float* __restrict__ dz, const float* __restrict__ Zm,
+                                                        double* __restrict__ part, int cap) {
+  constexpr int KGRP = (KIN + COLS - 1) / COLS;
+  constexpr int NCH = 256 / kWgChunk;
+  constexpr int KT = COLS / 4;                     // columns of a lane's tile
+  constexpr int DCH = kWgChunk * kHidden + kHidden; // floats per chunk, padded: two chunks of a wave on other banks
+  constexpr int XCH = kWgChunk * COLS + 32;
+  __shared__ __attribute__((aligned(16))) float ds[NCH * DCH];
+  __shared__ __attribute__((aligned(16))) float xs[NCH * XCH];
+  const int q = blockIdx.x / kXcds;
+  const int blk = q / KGRP * kXcds + blockIdx.x % kXcds, k0 = q % KGRP * COLS;
+  const int r0 = blk * 256;
+  if (r0 >= n) return;
+  float4 d[kHidden / 4];
 #pragma unroll
-  for (int q = 0; q < (NOUT + 255) / 256; ++q) acc[q] = 0.0;
-  for (int c = 0; c < 256; c += CH) {
-    for (int t = threadIdx.x; t < CH * KIN; t += 256) {
-      const int rr = t / KIN, k = t % KIN, row = r0 + c + rr;
-      float v = 0.f;
-      if (row < n && k < kin) v = bf16_round((k < c0) ? X0[(long)row * ld0 + k] : X1[(long)row * ld1 + (k - c0)]);
-      xs[rr][k] = v;
+  for (int j = 0; j < kHidden / 4; ++j) {
+    const int t = j * 256 + threadIdx.x, row = r0 + t / (kHidden / 4);
+    const long o = (long)r0 * (kHidden / 4) + t;
+    d[j] = row < n ? reinterpret_cast<const float4*>(dz)[o] : make_float4(0.f, 0.f, 0.f, 0.f);
+    if (Zm && row < n) {
+      const float4 z = reinterpret_cast<const float4*>(Zm)[o];
+      d[j] = make_float4(z.x > 0.f ? d[j].x : 0.f, z.y > 0.f ? d[j].y : 0.f, z.z > 0.f ? d[j].z : 0.f,
+                         z.w > 0.f ? d[j].w : 0.f);
     }
-    for (int t = threadIdx.x; t < CH * kHidden; t += 256) {
-      const int rr = t / kHidden, q = t % kHidden, row = r0 + c + rr;
-      ds[rr][q] = (row < n) ? dz[(long)row * kHidden + q] : 0.f;
-    }
-    __syncthreads();
+  }
+  float x[COLS];
 #pragma unroll
-    for (int q = 0; q < (NOUT + 255) / 256; ++q) {
-      const int o = threadIdx.x + q * 256;
-      if (o < NOUT) {
-        float s = 0.f;
-        if (o < KIN * kHidden) {
-          const int k = o / kHidden, j = o % kHidden;
-          for (int rr = 0; rr < CH; ++rr) s += xs[rr][k] * ds[rr][j];
-        } else {
-          const int j = o - KIN * kHidden;
-          for (int rr = 0; rr < CH; ++rr) s += ds[rr][j];
-        }
-        acc[q] += (double)s;
-      }
-    }
-    __syncthreads();
+  for (int j = 0; j < COLS; ++j) {
+    const int t = j * 256 + threadIdx.x, row = r0 + t / COLS, k = k0 + t % COLS;
+    x[j] = row < n && k < kin ? ((k < c0) ? X0[(long)row * ld0 + k] : X1[(long)row * ld1 + (k - c0)]) : 0.f;
   }
 #pragma unroll
-  for (int q = 0; q < (NOUT + 255) / 256; ++q) {
-    const int o = threadIdx.x + q * 256;
-    if (o < NOUT) part[(long)o * cap + blockIdx.x] = acc[q];
+  for (int j = 0; j < kHidden / 4; ++j) {
+    const int t = j * 256 + threadIdx.x, row = t / (kHidden / 4);
+    *reinterpret_cast<float4*>(&ds[row / kWgChunk * DCH + row % kWgChunk * kHidden + t % (kHidden / 4) * 4]) = d[j];
   }
+#pragma unroll
+  for (int j = 0; j < COLS; ++j) {
+    const int t = j * 256 + threadIdx.x, row = t / COLS;
+    xs[row / kWgChunk * XCH + row % kWgChunk * COLS + t % COLS] = bf16_round(x[j]);
+  }
+  __syncthreads();
+  const int c = threadIdx.x / 32, kq = threadIdx.x % 32 / 8 * KT, jq = threadIdx.x % 8 * 4;
+  float s[KT][4], sb[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int u = 0; u < KT; ++u)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) s[u][v] = 0.f;
+#pragma unroll 4
+  for (int rr = 0; rr < kWgChunk; ++rr) {
+    const float4 w = *reinterpret_cast<const float4*>(&ds[c * DCH + rr * kHidden + jq]);
+    const float y[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+    for (int u = 0; u < KT; ++u) {
+      const float xv = xs[c * XCH + rr * COLS + kq + u];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) s[u][v] += xv * y[v];
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) sb[v] += y[v];
+  }
+  __syncthreads(); // the chunks' sums take the place of dz and X
+#pragma unroll
+  for (int u = 0; u < KT; ++u)
+    *reinterpret_cast<float4*>(&ds[(c * COLS + kq + u) * kHidden + jq]) = make_float4(s[u][0], s[u][1], s[u][2], s[u][3]);
+  if (kq == 0) *reinterpret_cast<float4*>(&xs[c * kHidden + jq]) = make_float4(sb[0], sb[1], sb[2], sb[3]);
+  __syncthreads();
+#pragma unroll
+  for (int o = threadIdx.x; o < COLS * kHidden; o += 256) {
+    double acc = 0.0;
+#pragma unroll
+    for (int h = 0; h < NCH; ++h) acc += (double)ds[h * COLS * kHidden + o];
+    const int k = k0 + o / kHidden;
+    if (k < KIN) part[(long)(k * kHidden + o % kHidden) * cap + blk] = acc;
+  }
+  if (k0 == 0 && threadIdx.x < kHidden) {
+    double acc = 0.0;
+#pragma unroll
+    for (int h = 0; h < NCH; ++h) acc += (double)xs[h * kHidden + threadIdx.x];
+    part[(long)(KIN * kHidden + threadIdx.x) * cap + blk] = acc;
+  }
+}
+template <int KIN, int COLS>
+void wgrad_partials(hipStream_t s, int n, const float* X0, int ld0, int c0, const float* X1, int ld1, int kin,
+                    const float* dz, const float* Zm, double* part, int cap) {
+  static_assert(COLS % 4 == 0 && COLS <= 32, "the chunks' sums fit where dz was");
+  const long g = (cap + kXcds - 1) / kXcds * kXcds * ((KIN + COLS - 1) / COLS);
+  hipLaunchKernelGGL((k_wgrad_partials<KIN, COLS>), dim3((unsigned)g), dim3(256), 0, s, n, X0, ld0, c0, X1, ld1, kin,
+                     dz, Zm, part, cap);
 }
 
-// out[o] (+)= sum_b part[o * cap + b] in block order (one lane per output)
-__global__ void k_colsum(int nout, int nblk, const double* __restrict__ part, int cap, float* __restrict__ out,
-                         int accumulate) {
-  const int o = blockIdx.x * blockDim.x + threadIdx.x;
-  if (o >= nout) return;
-  double s = 0.0;
-  for (int b = 0; b < nblk; ++b) s += part[(long)o * cap + b];
-  out[o] = accumulate ? out[o] + (float)s : (float)s;
+// out[o] (+)= sum_b part[o * cap + b] in block order. A workgroup takes kColOut outputs: tiles of 256 partials of
+// each are loaded coalesced, the next while one lane per output adds the last, so that a tile costs its chain of
+// additions (one lane per output reading 8 bytes of a line at a time took 449 us at 96^3, this 71; at 16^3 both 3.4).
+constexpr int kColOut = 8;
+__global__ void __launch_bounds__(256) k_colsum(int nout, int nblk, const double* __restrict__ part, int cap,
+                                                float* __restrict__ out, int accumulate) {
+  __shared__ double tile[kColOut][256 + 1];
+  const int o0 = blockIdx.x * kColOut, t = threadIdx.x;
+  double v[kColOut], s = 0.0;
+  auto load = [&](int b0) {
+#pragma unroll
+    for (int c = 0; c < kColOut; ++c)
+      v[c] = o0 + c < nout && b0 + t < nblk ? part[(long)(o0 + c) * cap + b0 + t] : 0.0;
+  };
+  load(0);
+  for (int b0 = 0; b0 < nblk; b0 += 256) {
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < kColOut; ++c) tile[c][t] = v[c];
+    __syncthreads();
+    load(b0 + 256);
+    if (t < kColOut) {
+      const int m = min(256, nblk - b0);
+#pragma unroll 16
+      for (int b = 0; b < m; ++b) s += tile[t][b];
+    }
+  }
+  const int o = o0 + t;
+  if (t < kColOut && o < nout) out[o] = accumulate ? out[o] + (float)s : (float)s;
 }
-// per-row head gradient terms (N x kHeadGrads) -> partials per 256 rows
+// per-row head gradient terms (N x kHeadGrads) -> partials per 256 rows. A workgroup takes kRowsumCols of the
+// columns through LDS (every load in flight at once); one lane then adds a column's rows in order.
+// Lanes that walked their column in memory had few loads in flight: 41 us at 16^3, now 5.5.
+constexpr int kRowsumCols = 25;
 __global__ void __launch_bounds__(256) k_rowsum_partials(int n, int ncol, const float* __restrict__ prow,
                                                          double* __restrict__ part, int cap) {
-  const int r0 = blockIdx.x * 256;
-  for (int o = threadIdx.x; o < ncol; o += 256) {
-    double s = 0.0;
-    for (int r = r0; r < min(n, r0 + 256); ++r) s += (double)prow[(long)r * ncol + o];
-    part[(long)o * cap + blockIdx.x] = s;
+  __shared__ float xs[256 * kRowsumCols];
+  const int r0 = blockIdx.x * 256, o0 = blockIdx.y * kRowsumCols, rows = min(256, n - r0);
+  float v[kRowsumCols];
+#pragma unroll
+  for (int q = 0; q < kRowsumCols; ++q) {
+    const int t = q * 256 + threadIdx.x, r = t / kRowsumCols, o = o0 + t % kRowsumCols;
+    v[q] = r < rows && o < ncol ? prow[(long)(r0 + r) * ncol + o] : 0.f;
   }
+#pragma unroll
+  for (int q = 0; q < kRowsumCols; ++q) xs[q * 256 + threadIdx.x] = v[q];
+  __syncthreads();
+  const int o = o0 + threadIdx.x;
+  if (threadIdx.x >= kRowsumCols || o >= ncol) return;
+  double s = 0.0;
+#pragma unroll 16
+  for (int r = 0; r < rows; ++r) s += (double)xs[r * kRowsumCols + threadIdx.x];
+  part[(long)o * cap + blockIdx.x] = s;
 }
 
 // Adam (Kingma & Ba 2015) on the FP32 master weights
@@ -900,8 +1251,8 @@ double Engine::loss_grad(const float* P, const float* V, int K, float beta, int 
                      d_e.data(), d_ghat.data(), gg.data(), d_h[3].data(), P, dh[0].data(), prow.data());
   const int cap = (int)nb;
   DeviceArray<double> part((size_t)(2 * kHidden * kHidden + kHidden) * cap);
-  hipLaunchKernelGGL(k_rowsum_partials, dim3((unsigned)nb), dim3(256), 0, s, n, kHeadGrads, prow.data(), part.data(), cap);
-  hipLaunchKernelGGL(k_colsum, g1(kHeadGrads), dim3(256), 0, s, kHeadGrads, (int)nb, part.data(), cap, grad + kOffWd, 0);
+  hipLaunchKernelGGL(k_rowsum_partials, dim3((unsigned)nb, (kHeadGrads + kRowsumCols - 1) / kRowsumCols), dim3(256), 0, s, n, kHeadGrads, prow.data(), part.data(), cap);
+  hipLaunchKernelGGL(k_colsum, g1(kHeadGrads, kColOut), dim3(256), 0, s, kHeadGrads, (int)nb, part.data(), cap, grad + kOffWd, 0);
   // ---- message-passing layers, last to first
   const int offs[3] = {kOffW1, kOffW2, kOffW3};
   int cur = 0;
@@ -909,20 +1260,22 @@ double Engine::loss_grad(const float* P, const float* V, int K, float beta, int 
     const float* Wl = P + offs[l - 1];
     hipLaunchKernelGGL(k_dense_bwd_mfma, dim3((unsigned)(((n + 31) / 32 + 3) / 4)), dim3(256), 0, s, n, dh[cur].data(),
                        d_z[l].data(), Wl, dz.data(), dh[cur ^ 1].data(), dmsg.data());
-    hipLaunchKernelGGL(k_aggregate_add, g1((long)n * 32), dim3(256), 0, s, n, m_v.d_ro, m_v.d_cols,
+    hipLaunchKernelGGL(k_aggregate_add, aggregate_grid(n), dim3(256), 0, s, n, m_v.d_ro, m_v.d_cols,
                        d_tpos.data(), d_e.data(), dmsg.data(), dh[cur ^ 1].data());
-    hipLaunchKernelGGL(k_wgrad_partials<64>, dim3((unsigned)nb), dim3(256), 0, s, n, d_h[l - 1].data(), kHidden, kHidden,
-                       d_m[l].data(), kHidden, 2 * kHidden, dz.data(), part.data(), cap);
-    hipLaunchKernelGGL(k_colsum, g1(kLayerSize), dim3(256), 0, s, kLayerSize, (int)nb, part.data(), cap,
+    if (nb < kWgradWide)
+      wgrad_partials<2 * kHidden, 8>(s, n, d_h[l - 1].data(), kHidden, kHidden, d_m[l].data(), kHidden, 2 * kHidden,
+                                     dz.data(), nullptr, part.data(), cap);
+    else
+      wgrad_partials<2 * kHidden, 32>(s, n, d_h[l - 1].data(), kHidden, kHidden, d_m[l].data(), kHidden, 2 * kHidden,
+                                      dz.data(), nullptr, part.data(), cap);
+    hipLaunchKernelGGL(k_colsum, g1(kLayerSize, kColOut), dim3(256), 0, s, kLayerSize, (int)nb, part.data(), cap,
                        grad + offs[l - 1], 0);
     cur ^= 1;
   }
   // ---- input layer
-  hipLaunchKernelGGL(k_dense_bwd<kFeat>, g1(n), dim3(256), 0, s, n, dh[cur].data(), d_z[0].data(), P + kOffWin, kFeat,
-                     dz.data(), (float*)nullptr, (float*)nullptr);
-  hipLaunchKernelGGL(k_wgrad_partials<kFeat>, dim3((unsigned)nb), dim3(256), 0, s, n, d_f.data(), kFeat, kFeat,
-                     (const float*)nullptr, 0, kFeat, dz.data(), part.data(), cap);
-  hipLaunchKernelGGL(k_colsum, g1(kFeat * kHidden + kHidden), dim3(256), 0, s, kFeat * kHidden + kHidden, (int)nb,
+  wgrad_partials<kFeat, 8>(s, n, d_f.data(), kFeat, kFeat, nullptr, 0, kFeat, dh[cur].data(), d_z[0].data(),
+                           part.data(), cap);
+  hipLaunchKernelGGL(k_colsum, g1(kFeat * kHidden + kHidden, kColOut), dim3(256), 0, s, kFeat * kHidden + kHidden, (int)nb,
                      part.data(), cap, grad + kOffWin, 0);
   check_launch("gnn backward");
   double hs[4];
@@ -941,135 +1294,90 @@ double Engine::loss_grad(const float* P, const float* V, int K, float beta, int 
 // 4 columns of B as right-hand sides: L = mean_c log(|r_k|^2 / |r_0|^2), rho =
 // |Ghat^T r|^2. Forward keeps r_j, t_j = Ghat^T r_j, p_j, q_j = Ahat p_j; the
 // reverse pass (the adjoint of each step, last to first) accumulates dL/dGhat
-// on the lower pattern into gg. Step scalars live on the host (one dot4
-// readback each), vectors in FP32, dots in FP64.
+// on the lower pattern into gg. Three launches a step each way; the host reads
+// |r_0|^2 and |r_k|^2 once, between the two. Vectors in FP32, dots in FP64.
 double Engine::cg_term(const float* B, int k, float* gg) {
   hipStream_t s = m_ctx->stream;
   const int n = m_n;
-  const size_t nv = (size_t)n * 4;
-  const dim3 gv = g1((long)nv), gr = g1(n);
-  RedWork w = m_ctx->red();
   const long nb = (n + 255) / 256;
-  DeviceArray<double> dsum(4);
-  auto dot4 = [&](const float* X, const float* Y) {
-    std::array<double, 4> h{};
-    hipLaunchKernelGGL(k_dot4, dim3((unsigned)nb), dim3(256), 0, s, n, X, Y, w);
-    launch_finalize(s, w, nb, 4, kFinStore, dsum.data(), nullptr);
-    ALIEN_HIP_CHECK(hipMemcpyAsync(h.data(), dsum.data(), sizeof(double) * 4, hipMemcpyDeviceToHost, s));
-    ALIEN_HIP_CHECK(hipStreamSynchronize(s));
-    return h;
+  const dim3 g((unsigned)nb), t256(256);
+  // vectors: r_0..r_k, t_j, p_j, q_j (j < k) and the adjoints of r, p and t
+  DeviceArray<float4> vec((size_t)n * (4 * (size_t)k + 4));
+  auto at = [&](size_t slot) { return vec.data() + slot * (size_t)n; };
+  auto R = [&](int j) { return at(j); };
+  auto T = [&](int j) { return at((size_t)k + 1 + j); };
+  auto Pv = [&](int j) { return at(2 * (size_t)k + 1 + j); };
+  auto Q = [&](int j) { return at(3 * (size_t)k + 1 + j); };
+  float4 *rbar = at(4 * (size_t)k + 1), *pbar = at(4 * (size_t)k + 2), *tbar = at(4 * (size_t)k + 3);
+  // partials of two dot products in turn (a kernel consumes one and produces the next) and of r_0.r_0,
+  // a total, and the step scalars kept on the device
+  DeviceArray<double> dots(12 * (size_t)nb + 12 + 16 * (size_t)k);
+  double* part[2] = {dots.data(), dots.data() + 4 * nb};
+  double* rr_part = dots.data() + 8 * nb;
+  double* tot = dots.data() + 12 * nb;
+  double *rr = tot + 4, *scal = tot + 12;
+  auto rho = [&](int j) { return scal + 4 * (size_t)j; };
+  auto sig = [&](int j) { return scal + 4 * (size_t)(k + j); };
+  auto own = [&](int j) { return scal + 4 * (size_t)(2 * k + j); };
+  auto rhobar = [&](int j) { return scal + 4 * (size_t)(3 * k + j); };
+  int cur = 0; // part[cur] holds the last dot product's partials
+  auto next = [&] { return part[cur ^= 1]; };
+  // Up to a wavefront's lanes of partials are summed by their consumers; more take the finalize's launch
+  // (4.5 us), which costs less than every wavefront of the consumer reading several rounds of them.
+  auto value = [&]() {
+    if (nb <= kWave) return Dot4{part[cur], (int)nb};
+    launch_finalize(s, RedWork{part[cur], (int)nb}, nb, 4, kFinStore, tot, nullptr);
+    return Dot4{tot, 1};
   };
-  auto lin = [&](std::array<double, 4> a, const float* X, std::array<double, 4> b, const float* Z, float* Y) {
-    Coef4 ca, cb;
-    for (int c = 0; c < 4; ++c) {
-      ca.c[c] = (float)a[c];
-      cb.c[c] = (float)b[c];
-    }
-    hipLaunchKernelGGL(k_lin4, gv, dim3(256), 0, s, n, ca, X, cb, Z, Y);
-  };
-  auto amul = [&](const float* X, float* Y) {
-    hipLaunchKernelGGL((k_ahat_mult<4>), gr, dim3(256), 0, s, n, m_v.d_ro, m_v.d_cols, d_e.data(), X, Y);
-  };
-  auto gmul = [&](const float* X, float* Y) { // Y = Ghat X
-    hipLaunchKernelGGL((k_ghat_mult<4, false>), gr, dim3(256), 0, s, n, m_v.d_ro, m_v.d_cols, m_v.d_dcol,
-                       d_tpos.data(), d_ghat.data(), X, Y);
-  };
-  auto gtmul = [&](const float* X, float* Y) { // Y = Ghat^T X
-    hipLaunchKernelGGL((k_ghat_mult<4, true>), gr, dim3(256), 0, s, n, m_v.d_ro, m_v.d_cols, m_v.d_dcol,
-                       d_tpos.data(), d_ghat.data(), X, Y);
-  };
-  auto acc = [&](const float* U, const float* V, const float* W, const float* X) {
-    hipLaunchKernelGGL(k_edge_acc4, gr, dim3(256), 0, s, n, m_v.d_ro, m_v.d_cols, m_v.d_dcol, U, V, W, X,
-                       gg);
-  };
-  typedef std::array<double, 4> S4;
-  const S4 one{1, 1, 1, 1}, zero{0, 0, 0, 0};
-  std::vector<DeviceArray<float>> R(k + 1), T(k), Pv(k), Q(k);
-  for (auto& a : R) a.resize(nv);
-  for (auto& a : T) a.resize(nv);
-  for (auto& a : Pv) a.resize(nv);
-  for (auto& a : Q) a.resize(nv);
-  DeviceArray<float> z(nv), rbar(nv), pbar(nv), pbar2(nv), qbar(nv), tbar(nv), tmp(nv);
-  std::vector<S4> rho(k), sig(k), alpha(k), beta(k);
+  const CgRows A{n, m_v.d_ro, m_v.d_cols, m_v.d_dcol, d_tpos.data(), d_e.data(), d_ghat.data()};
   // forward
-  ALIEN_HIP_CHECK(hipMemcpyAsync(R[0].data(), B, sizeof(float) * nv, hipMemcpyDeviceToDevice, s));
-  gtmul(R[0].data(), T[0].data());
-  gmul(T[0].data(), Pv[0].data());
-  rho[0] = dot4(T[0].data(), T[0].data());
-  const S4 rr0 = dot4(R[0].data(), R[0].data());
+  ALIEN_HIP_CHECK(hipMemcpyAsync(R(0), B, sizeof(float4) * n, hipMemcpyDeviceToDevice, s));
+  hipLaunchKernelGGL(k_cg4_start, g, t256, 0, s, A, R(0), T(0), next(), rr_part, (int)nb);
   for (int j = 0; j < k; ++j) {
-    amul(Pv[j].data(), Q[j].data());
-    sig[j] = dot4(Pv[j].data(), Q[j].data());
-    S4 na;
-    for (int c = 0; c < 4; ++c) {
-      alpha[j][c] = rho[j][c] / sig[j][c];
-      na[c] = -alpha[j][c];
-    }
-    lin(one, R[j].data(), na, Q[j].data(), R[j + 1].data());
-    if (j < k - 1) {
-      gtmul(R[j + 1].data(), T[j + 1].data());
-      gmul(T[j + 1].data(), z.data());
-      rho[j + 1] = dot4(T[j + 1].data(), T[j + 1].data());
-      for (int c = 0; c < 4; ++c) beta[j][c] = rho[j + 1][c] / rho[j][c];
-      lin(one, z.data(), beta[j], Pv[j].data(), Pv[j + 1].data());
-    }
+    const Dot4 rho1 = value();
+    hipLaunchKernelGGL(k_cg4_dir, g, t256, 0, s, A, T(j), j ? Pv(j - 1) : (const float4*)nullptr, rho1,
+                       j ? rho(j - 1) : (const double*)nullptr, rho(j), Pv(j));
+    hipLaunchKernelGGL(k_cg4_ap, g, t256, 0, s, A, Pv(j), Q(j), next(), (int)nb);
+    const Dot4 pq = value();
+    hipLaunchKernelGGL(k_cg4_res, g, t256, 0, s, A, R(j), Q(j), rho(j), pq, sig(j), R(j + 1),
+                       j < k - 1 ? T(j + 1) : (float4*)nullptr, next(), (int)nb);
   }
-  const S4 rrk = dot4(R[k].data(), R[k].data());
+  launch_finalize(s, RedWork{rr_part, (int)nb}, nb, 4, kFinStore, rr, nullptr);
+  launch_finalize(s, RedWork{part[cur], (int)nb}, nb, 4, kFinStore, rr + 4, nullptr);
+  check_launch("gnn cg loss");
+  double h[8]; // |r_0|^2, |r_k|^2
+  ALIEN_HIP_CHECK(hipMemcpyAsync(h, rr, sizeof(h), hipMemcpyDeviceToHost, s));
+  ALIEN_HIP_CHECK(hipStreamSynchronize(s));
   double L = 0.0;
-  S4 c0;
+  Coef4 c0;
   for (int c = 0; c < 4; ++c) {
-    L += std::log(rrk[c] / rr0[c]) / 4.0;
-    c0[c] = 2.0 / (4.0 * rrk[c]);
+    L += std::log(h[4 + c] / h[c]) / 4.0;
+    c0.c[c] = (float)(2.0 / (4.0 * h[4 + c]));
   }
   if (!std::isfinite(L)) return L;
   // reverse
-  lin(c0, R[k].data(), zero, nullptr, rbar.data());
-  S4 rhobar_next = zero;
+  hipLaunchKernelGGL(k_cg4_rev_start, g, t256, 0, s, n, c0, R(k), Q(k - 1), rbar, next(), (int)nb);
   for (int j = k - 1; j >= 0; --j) {
-    S4 rhobar_j = zero;
-    if (j < k - 1) {
-      // p_{j+1} = z_{j+1} + beta_j p_j ; zbar = pbar_{j+1} (held in pbar)
-      const S4 betabar = dot4(pbar.data(), Pv[j].data());
-      S4 rhobar_jp1, two_rho;
-      for (int c = 0; c < 4; ++c) {
-        rhobar_jp1[c] = rhobar_next[c] + betabar[c] / rho[j][c];
-        rhobar_j[c] -= betabar[c] * rho[j + 1][c] / (rho[j][c] * rho[j][c]);
-        two_rho[c] = 2.0 * rhobar_jp1[c];
-      }
-      // z = Ghat t: dGhat += zbar t^T ; tbar = 2 rhobar t + Ghat^T zbar
-      gtmul(pbar.data(), tmp.data());
-      lin(two_rho, T[j + 1].data(), one, tmp.data(), tbar.data());
-      // t = Ghat^T r: dGhat += r tbar^T ; rbar += Ghat tbar
-      acc(pbar.data(), T[j + 1].data(), R[j + 1].data(), tbar.data());
-      gmul(tbar.data(), tmp.data());
-      lin(one, rbar.data(), one, tmp.data(), rbar.data());
-      lin(beta[j], pbar.data(), zero, nullptr, pbar2.data()); // pbar_j = beta_j pbar_{j+1}
-    } else {
-      ALIEN_HIP_CHECK(hipMemsetAsync(pbar2.data(), 0, sizeof(float) * nv, s)); // p_k is not formed
+    const bool last = j == k - 1; // p_k is not formed
+    if (!last) {
+      const Dot4 betabar = value();
+      hipLaunchKernelGGL(k_cg4_rev_t, g, t256, 0, s, A, pbar, T(j + 1), rhobar(j + 1), betabar, rho(j), rho(j + 1),
+                         own(j), tbar);
+      hipLaunchKernelGGL(k_cg4_rev_r, g, t256, 0, s, A, pbar, T(j + 1), R(j + 1), tbar, gg, rbar, Q(j), next(),
+                         (int)nb);
     }
-    // r_{j+1} = r_j - alpha q_j
-    const S4 qr = dot4(Q[j].data(), rbar.data());
-    S4 na, sigbar;
-    for (int c = 0; c < 4; ++c) {
-      const double alphabar = -qr[c];
-      rhobar_j[c] += alphabar / sig[j][c];
-      sigbar[c] = -alphabar * rho[j][c] / (sig[j][c] * sig[j][c]);
-      na[c] = -alpha[j][c];
-    }
-    lin(na, rbar.data(), sigbar, Pv[j].data(), qbar.data()); // qbar = -alpha rbar + sigbar p
-    lin(one, pbar2.data(), sigbar, Q[j].data(), pbar2.data()); // pbar += sigbar q
-    amul(qbar.data(), tmp.data());
-    lin(one, pbar2.data(), one, tmp.data(), pbar.data()); // pbar_j = ... + Ahat qbar
-    rhobar_next = rhobar_j;
+    const Dot4 qr = value();
+    hipLaunchKernelGGL(k_cg4_rev_p, g, t256, 0, s, A, rbar, Pv(j), Q(j), rho(j),
+                       last ? (const double*)nullptr : rho(j + 1), sig(j), qr, own(j), rhobar(j), pbar,
+                       j ? Pv(j - 1) : (const float4*)nullptr, next(), (int)nb);
   }
   // p_0 = Ghat t_0, rho_0 = t_0.t_0, t_0 = Ghat^T r_0
-  S4 two_rho;
-  for (int c = 0; c < 4; ++c) two_rho[c] = 2.0 * rhobar_next[c];
-  gtmul(pbar.data(), tmp.data());
-  lin(two_rho, T[0].data(), one, tmp.data(), tbar.data());
-  acc(pbar.data(), T[0].data(), R[0].data(), tbar.data());
+  hipLaunchKernelGGL(k_cg4_rev_t, g, t256, 0, s, A, pbar, T(0), rhobar(0), Dot4{nullptr, 0}, (const double*)nullptr,
+                     (const double*)nullptr, (double*)nullptr, tbar);
+  hipLaunchKernelGGL(k_cg4_rev_r, g, t256, 0, s, A, pbar, T(0), R(0), tbar, gg, (float4*)nullptr,
+                     (const float4*)nullptr, (double*)nullptr, (int)nb);
   check_launch("gnn cg loss");
-  ALIEN_HIP_CHECK(hipStreamSynchronize(s));
+  ALIEN_HIP_CHECK(hipStreamSynchronize(s)); // before the vectors are freed
   return L;
 }
 
