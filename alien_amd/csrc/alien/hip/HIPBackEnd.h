@@ -787,13 +787,15 @@ class HIPInternalLinearAlgebra
   }
   double dot(const Vector& x, const Vector& y) const {
     const int s = m_ctx->take_slot();
-    alien_hip::launch_dot<double>(stream(), m_ctx->red(), x.scalarizedLocalSize(), x.data(), y.data(), m_ctx->dslot(s));
+    alien_hip::launch_dot<double>(stream(), m_ctx->red_once(), x.scalarizedLocalSize(), x.data(), y.data(),
+                                  m_ctx->dslot(s), m_ctx->post_slot(s));
     alien_hip::check_launch("dot");
     return m_ctx->read_slot(s);
   }
   void dot(const Vector& x, const Vector& y, FutureType& f) const {
     const int s = m_ctx->take_slot();
-    alien_hip::launch_dot<double>(stream(), m_ctx->red(), x.scalarizedLocalSize(), x.data(), y.data(), m_ctx->dslot(s));
+    alien_hip::launch_dot<double>(stream(), m_ctx->red_once(), x.scalarizedLocalSize(), x.data(), y.data(),
+                                  m_ctx->dslot(s), m_ctx->post_slot(s));
     alien_hip::check_launch("dot(future)");
     f.attach(m_ctx, s);
   }
@@ -854,8 +856,8 @@ class HIPInternalLinearAlgebraExpr
   double norm2(const Matrix& a) const {
     const int s = m_alg.ctx()->take_slot();
     m_alg.ctx()->reserve_for(a.getNnz());
-    alien_hip::launch_dot<double>(m_alg.stream(), m_alg.ctx()->red(), a.getNnz(), a.d_vals.data(), a.d_vals.data(),
-                                  m_alg.ctx()->dslot(s));
+    alien_hip::launch_dot<double>(m_alg.stream(), m_alg.ctx()->red_once(), a.getNnz(), a.d_vals.data(), a.d_vals.data(),
+                                  m_alg.ctx()->dslot(s), m_alg.ctx()->post_slot(s));
     alien_hip::check_launch("norm2(matrix)");
     return std::sqrt(m_alg.ctx()->read_slot(s));
   }

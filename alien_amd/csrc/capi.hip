@@ -46,8 +46,11 @@ alien_hip_ctx* make_ctx(void* stream) {
     ALIEN_HIP_CHECK(hipMemsetAsync(c->grid_head.data(), 0, 2 * sizeof(int), c->stream));
     ALIEN_HIP_CHECK(hipGetDevice(&c->device));
     ALIEN_HIP_CHECK(hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, c->device));
-    ALIEN_HIP_CHECK(hipHostMalloc((void**)&c->host_scalars, sizeof(double) * alien_hip_ctx::kSlots,
-                                  hipHostMallocDefault));
+    c->tickets.resize(kTicketWords);
+    ALIEN_HIP_CHECK(hipMemsetAsync(c->tickets.data(), 0, sizeof(unsigned) * kTicketWords, c->stream));
+    ALIEN_HIP_CHECK(hipHostMalloc((void**)&c->mail, sizeof(unsigned long long) * alien_hip_ctx::kMailWords,
+                                  hipHostMallocCoherent));
+    std::fill_n(c->mail, alien_hip_ctx::kMailWords, 0ull);
     ALIEN_HIP_CHECK(hipStreamSynchronize(c->stream));
   } catch (...) {
     destroy_ctx(c);
@@ -66,7 +69,8 @@ void destroy_ctx(alien_hip_ctx* c) {
   c->grid_head.reset();
   c->ilu_piv.reset();
   c->ilu_work.reset();
-  if (c->host_scalars) (void)hipHostFree(c->host_scalars);
+  c->tickets.reset();
+  if (c->mail) (void)hipHostFree(c->mail);
   if (c->pinned_blocks) (void)hipHostFree(c->pinned_blocks);
   if (c->own_stream && c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
@@ -857,7 +861,7 @@ int alien_hip_dot_f64(alien_hip_ctx* ctx, int n, const double* x, const double* 
   REQUIRE(n >= 0 && result && (n == 0 || (x && y)), "dot_f64: bad arguments");
   API_BEGIN
   ctx->reserve_for(n);
-  launch_dot<double>(ctx->stream, ctx->red(), n, x, y, result);
+  launch_dot<double>(ctx->stream, ctx->red_once(), n, x, y, result);
   LAUNCHED("dot_f64");
   API_END
 }
@@ -866,7 +870,7 @@ int alien_hip_dot_f32(alien_hip_ctx* ctx, int n, const float* x, const float* y,
   REQUIRE(n >= 0 && result && (n == 0 || (x && y)), "dot_f32: bad arguments");
   API_BEGIN
   ctx->reserve_for(n);
-  launch_dot<float>(ctx->stream, ctx->red(), n, x, y, result);
+  launch_dot<float>(ctx->stream, ctx->red_once(), n, x, y, result);
   LAUNCHED("dot_f32");
   API_END
 }
@@ -875,7 +879,7 @@ int alien_hip_axpy_dot_f64(alien_hip_ctx* ctx, int n, double a, const double* x,
   REQUIRE(n >= 0 && result && (n == 0 || (x && y)), "axpy_dot_f64: bad arguments");
   API_BEGIN
   ctx->reserve_for(n);
-  launch_axpy_dot<double>(ctx->stream, ctx->red(), n, a, x, y, result);
+  launch_axpy_dot<double>(ctx->stream, ctx->red_once(), n, a, x, y, result);
   LAUNCHED("axpy_dot_f64");
   API_END
 }

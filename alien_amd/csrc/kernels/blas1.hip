@@ -10,6 +10,7 @@
 #include "../alien_hip_internal.h"
 #include "device_common.h"
 #include "launch.h"
+#include "wave_total.h"
 
 namespace alien_hip {
 
@@ -62,9 +63,41 @@ __global__ void __launch_bounds__(kBlock) k_pmult(int n, const T* x, const T* y,
   }
 }
 
-template <typename T>
+// The launch's total by its last workgroup, by the tree of the finalize (reduce.hip: 1024 lanes, lane t takes
+// partials t, t + 1024, ..). Up to kOneLaunchBlocks workgroups a
+// reduction is finished in its own launch: 1.3 us less a dot product than with the finalize's launch up to 768
+// workgroups (an axpy and two dots: 16.3 -> 13.5 us), as much at 1024 (16.3 against 16.2), where the arrivals take as long.
+constexpr int kOneLaunchBlocks = kTicketGroup * kTicketGroups;
+__device__ __forceinline__ void finish_one(double partial, RedWork w, double* out, HostPost post) {
+  constexpr int kFinLanes = 1024, U = kFinLanes / kBlock;
+  __shared__ double lds[kFinLanes / kWave];
+  if (threadIdx.x == 0) __hip_atomic_store(w.partial + blockIdx.x, partial, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (!last_block(w.ticket)) return;
+  const int nblk = gridDim.x;
+  double p[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int b = u * kBlock + threadIdx.x;
+    p[u] = b < nblk ? 0.0 + __hip_atomic_load(w.partial + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.0;
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const double s = wave_total(p[u]);
+    if ((threadIdx.x & (kWave - 1)) == 0) lds[u * (kBlock / kWave) + threadIdx.x / kWave] = s;
+  }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  double t = 0.0;
+#pragma unroll
+  for (int q = 0; q < kFinLanes / kWave; ++q) t += lds[q];
+  if (post.to) post_double(post, t);
+  out[0] = t;
+}
+
+// ONE: finished by its last workgroup, else the partials are left to a finalize
+template <typename T, bool ONE>
 __global__ void __launch_bounds__(kBlock) k_dot(int n, const T* __restrict__ x, const T* __restrict__ y,
-                                                 RedWork w) {
+                                                 RedWork w, double* out, HostPost post) {
   __shared__ double lds4[4];
   T xv[kEPT], yv[kEPT];
 #pragma unroll
@@ -77,13 +110,14 @@ __global__ void __launch_bounds__(kBlock) k_dot(int n, const T* __restrict__ x, 
 #pragma unroll
   for (int k = 0; k < kEPT; ++k) s += (double)xv[k] * (double)yv[k];
   double v[1] = {block_sum(s, lds4)};
-  store_partials<1>(v, w);
+  if constexpr (ONE) finish_one(v[0], w, out, post);
+  else store_partials<1>(v, w);
 }
 
 // y += a x ; out = y . y
-template <typename T>
+template <typename T, bool ONE>
 __global__ void __launch_bounds__(kBlock) k_axpy_dot(int n, T a, const T* __restrict__ x, T* __restrict__ y,
-                                                      RedWork w) {
+                                                      RedWork w, double* out) {
   __shared__ double lds4[4];
   T xv[kEPT], yv[kEPT];
 #pragma unroll
@@ -103,7 +137,8 @@ __global__ void __launch_bounds__(kBlock) k_axpy_dot(int n, T a, const T* __rest
     }
   }
   double v[1] = {block_sum(s, lds4)};
-  store_partials<1>(v, w);
+  if constexpr (ONE) finish_one(v[0], w, out, HostPost{});
+  else store_partials<1>(v, w);
 }
 
 // ---- launchers --------------------------------------------------------------
@@ -130,13 +165,22 @@ void launch_pmult(hipStream_t st, int n, const T* x, const T* y, T* z) {
   if (n > 0) hipLaunchKernelGGL(k_pmult<T>, ept_grid(n), dim3(kBlock), 0, st, n, x, y, z);
 }
 template <typename T>
-void launch_dot(hipStream_t st, RedWork w, int n, const T* x, const T* y, double* out) {
-  hipLaunchKernelGGL(k_dot<T>, ept_grid(n), dim3(kBlock), 0, st, n, x, y, w);
-  launch_finalize(st, w, ept_blocks(n), 1, kFinStore, out, nullptr);
+void launch_dot(hipStream_t st, RedWork w, int n, const T* x, const T* y, double* out, HostPost post) {
+  if (w.ticket && ept_blocks(n) <= kOneLaunchBlocks) {
+    hipLaunchKernelGGL((k_dot<T, true>), ept_grid(n), dim3(kBlock), 0, st, n, x, y, w, out, post);
+    return;
+  }
+  hipLaunchKernelGGL((k_dot<T, false>), ept_grid(n), dim3(kBlock), 0, st, n, x, y, w, out, post);
+  if (post.to) launch_finalize_post(st, w, ept_blocks(n), out, post);
+  else launch_finalize(st, w, ept_blocks(n), 1, kFinStore, out, nullptr);
 }
 template <typename T>
 void launch_axpy_dot(hipStream_t st, RedWork w, int n, T a, const T* x, T* y, double* out) {
-  hipLaunchKernelGGL(k_axpy_dot<T>, ept_grid(n), dim3(kBlock), 0, st, n, a, x, y, w);
+  if (w.ticket && ept_blocks(n) <= kOneLaunchBlocks) {
+    hipLaunchKernelGGL((k_axpy_dot<T, true>), ept_grid(n), dim3(kBlock), 0, st, n, a, x, y, w, out);
+    return;
+  }
+  hipLaunchKernelGGL((k_axpy_dot<T, false>), ept_grid(n), dim3(kBlock), 0, st, n, a, x, y, w, out);
   launch_finalize(st, w, ept_blocks(n), 1, kFinStore, out, nullptr);
 }
 
@@ -146,7 +190,7 @@ void launch_axpy_dot(hipStream_t st, RedWork w, int n, T a, const T* x, T* y, do
   template void launch_scal<T>(hipStream_t, int, T, T*);                                \
   template void launch_assign<T>(hipStream_t, int, T, T*);                              \
   template void launch_pmult<T>(hipStream_t, int, const T*, const T*, T*);              \
-  template void launch_dot<T>(hipStream_t, RedWork, int, const T*, const T*, double*);  \
+  template void launch_dot<T>(hipStream_t, RedWork, int, const T*, const T*, double*, HostPost); \
   template void launch_axpy_dot<T>(hipStream_t, RedWork, int, T, const T*, T*, double*);
 ALIEN_HIP_INST_BLAS1(double)
 ALIEN_HIP_INST_BLAS1(float)

@@ -4,6 +4,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include "host_post.h"
+
 #include <cstdint>
 
 namespace alien_hip {
@@ -152,7 +154,47 @@ __device__ inline double block_sum(double v, double* lds) {
 struct RedWork {
   double* partial; // kMaxSlots * cap
   int cap;         // workgroups per launch the buffer can hold
+  unsigned* ticket = nullptr; // kTicketWords zeros where the reducing kernel may finalize by itself (last_block)
 };
+// counters of last_block, each on a line of its own: one per kTicketGroup workgroups and one for the groups
+constexpr int kTicketGroup = 32, kTicketGroups = 32, kTicketStride = 32;
+constexpr int kTicketWords = (kTicketGroups + 1) * kTicketStride;
+
+// every vector memory access of this wavefront before it has been performed
+__device__ inline void stores_done() {
+  __asm__ __volatile__("s_waitcnt vmcnt(0)" ::: "memory");
+}
+// Whether this workgroup is the last of the launch (at most kTicketGroup * kTicketGroups of them) to come here,
+// the same answer on every lane. What lane 0 of the others stored before they came, with agent scope, an agent-scope
+// load of this one sees: the stores are complete before the count is raised. (A release at agent scope would also write
+// back what else is dirty in the XCD's L2: 19 us a launch after a vector update.) The counters are zero again when it returns true. Two levels, since every arrival at one word waits for the ones before.
+__device__ inline bool last_block(unsigned* ticket) {
+  __shared__ int last;
+  if (threadIdx.x == 0) {
+    const unsigned nb = gridDim.x, g = blockIdx.x / kTicketGroup, ng = (nb + kTicketGroup - 1) / kTicketGroup;
+    const unsigned in_group = g + 1 < ng ? kTicketGroup : nb - g * kTicketGroup;
+    unsigned* mine = ticket + (1 + g) * kTicketStride;
+    stores_done();
+    int l = __hip_atomic_fetch_add(mine, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == in_group - 1;
+    if (l) {
+      __hip_atomic_store(mine, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      stores_done();
+      l = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == ng - 1;
+      if (l) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    last = l;
+  }
+  __syncthreads();
+  return last != 0;
+}
+__device__ inline void post_word(HostPost p, int i, unsigned w) {
+  __hip_atomic_store(p.to + i, (unsigned long long)p.tag << 32 | w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__device__ inline void post_double(HostPost p, double v) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  post_word(p, 0, (unsigned)b);
+  post_word(p, 1, (unsigned)(b >> 32));
+}
 
 template <int NSLOT>
 __device__ inline void store_partials(const double (&vals)[NSLOT], RedWork w) {

@@ -1346,8 +1346,7 @@ double Engine::cg_term(const float* B, int k, float* gg) {
   launch_finalize(s, RedWork{part[cur], (int)nb}, nb, 4, kFinStore, rr + 4, nullptr);
   check_launch("gnn cg loss");
   double h[8]; // |r_0|^2, |r_k|^2
-  ALIEN_HIP_CHECK(hipMemcpyAsync(h, rr, sizeof(h), hipMemcpyDeviceToHost, s));
-  ALIEN_HIP_CHECK(hipStreamSynchronize(s));
+  m_ctx->read_words(rr, h, 16);
   double L = 0.0;
   Coef4 c0;
   for (int c = 0; c < 4; ++c) {

@@ -9,6 +9,8 @@
 
 #include "krylov_state.h"
 
+#include "host_post.h"
+
 namespace alien_hip {
 
 struct RedWork;
@@ -17,6 +19,11 @@ template <typename T> class DeviceArray;
 // what the second stage of a reduction does with the totals (reduce.hip)
 enum FinOp { kFinStore = 0, kFinRho1 = 1, kFinPQ = 2, kFinXR = 3, kFinXRDiag = 4, kFinRho1B = 5 };
 void launch_finalize(hipStream_t, RedWork w, long nblk, int nslot, int op, double* out, CGState* st);
+// one stored total, handed to the host as well
+void launch_finalize_post(hipStream_t, RedWork w, long nblk, double* out, HostPost post);
+// n (at most kMaxPostWords) 32-bit words of device memory to the host
+constexpr int kMaxPostWords = 64;
+void launch_post_words(hipStream_t, const void* from, int n, HostPost post);
 // the same second stage for the BiCGStab state (reduce.hip)
 enum BFinOp { kBFinAlpha = 0, kBFinS = 1, kBFinOmega = 2, kBFinXR = 3 };
 void launch_finalize_bicg(hipStream_t, RedWork w, long nblk, int nslot, int op, BiCGState* st);
@@ -29,7 +36,9 @@ template <typename T> void launch_axpy(hipStream_t, int n, T a, const T* x, T* y
 template <typename T> void launch_scal(hipStream_t, int n, T a, T* x);
 template <typename T> void launch_assign(hipStream_t, int n, T a, T* x);
 template <typename T> void launch_pmult(hipStream_t, int n, const T* x, const T* y, T* z);
-template <typename T> void launch_dot(hipStream_t, RedWork w, int n, const T* x, const T* y, double* out);
+// the total also goes to the host when post.to is set
+template <typename T>
+void launch_dot(hipStream_t, RedWork w, int n, const T* x, const T* y, double* out, HostPost post = {});
 template <typename T> void launch_axpy_dot(hipStream_t, RedWork w, int n, T a, const T* x, T* y, double* out);
 
 // ---- SpMV (spmv.hip) ----

@@ -543,8 +543,8 @@ struct FusedCG {
     check_launch("learned CG resumed step");
   }
   CGState read_state() {
-    ALIEN_HIP_CHECK(hipMemcpyAsync(h_st, st.data(), sizeof(CGState), hipMemcpyDeviceToHost, ctx->stream));
-    ALIEN_HIP_CHECK(hipStreamSynchronize(ctx->stream));
+    static_assert(sizeof(CGState) <= 4 * kMaxPostWords, "one post");
+    ctx->read_words(st.data(), h_st, (int)(sizeof(CGState) / 4));
     return *h_st;
   }
 
@@ -609,7 +609,7 @@ struct FusedCG {
     hipStream_t s = ctx->stream;
     const int slot = ctx->take_slot();
     // Iteration ctor: (b,b) and the criteria
-    launch_dot<T>(s, ctx->red(), n, b, b, ctx->dslot(slot));
+    launch_dot<T>(s, ctx->red_once(), n, b, b, ctx->dslot(slot), ctx->post_slot(slot));
     const double bb = ctx->read_slot(slot);
     if (bb_out) *bb_out = bb;
     CGState h{};
@@ -663,7 +663,7 @@ void finish_breakdown(FusedCG<T>& F, CGState& s, int* error) {
     return;
   }
   const int slot = F.ctx->take_slot();
-  launch_dot<T>(F.ctx->stream, F.ctx->red(), F.n, F.r.data(), F.r.data(), F.ctx->dslot(slot));
+  launch_dot<T>(F.ctx->stream, F.ctx->red_once(), F.n, F.r.data(), F.r.data(), F.ctx->dslot(slot), F.ctx->post_slot(slot));
   const double rr = F.ctx->read_slot(slot);
   s.rr = rr;
   s.status = rr < s.crit;
@@ -718,7 +718,7 @@ MixedResult mixed_reliable_cg(alien_hip_ctx* ctx, int n, RBMat<double> A64, RBMa
   MixedResult out;
   hipStream_t s = ctx->stream;
   const int slot = ctx->take_slot();
-  launch_dot<double>(s, ctx->red(), n, b, b, ctx->dslot(slot));
+  launch_dot<double>(s, ctx->red_once(), n, b, b, ctx->dslot(slot), ctx->post_slot(slot));
   const double bb = ctx->read_slot(slot);
   if (bb == 0) {
     out.status = 1;
@@ -885,8 +885,8 @@ struct FusedBiCG {
                       st.data());
   }
   BiCGState read_state() {
-    ALIEN_HIP_CHECK(hipMemcpyAsync(h_st, st.data(), sizeof(BiCGState), hipMemcpyDeviceToHost, ctx->stream));
-    ALIEN_HIP_CHECK(hipStreamSynchronize(ctx->stream));
+    static_assert(sizeof(BiCGState) <= 4 * kMaxPostWords, "one post");
+    ctx->read_words(st.data(), h_st, (int)(sizeof(BiCGState) / 4));
     return *h_st;
   }
   void write_state(const BiCGState& h) {
@@ -942,7 +942,7 @@ struct FusedBiCG {
                   int stall_window = 0, bool* stalled = nullptr) {
     hipStream_t s = ctx->stream;
     const int slot = ctx->take_slot();
-    launch_dot<T>(s, ctx->red(), n, b, b, ctx->dslot(slot));
+    launch_dot<T>(s, ctx->red_once(), n, b, b, ctx->dslot(slot), ctx->post_slot(slot));
     const double bb = ctx->read_slot(slot);
     if (bb_out) *bb_out = bb;
     BiCGState h{};
@@ -992,7 +992,7 @@ MixedResult mixed_reliable_bicg(alien_hip_ctx* ctx, int n, RBMat<double> A64, RB
   MixedResult out;
   hipStream_t s = ctx->stream;
   const int slot = ctx->take_slot();
-  launch_dot<double>(s, ctx->red(), n, b, b, ctx->dslot(slot));
+  launch_dot<double>(s, ctx->red_once(), n, b, b, ctx->dslot(slot), ctx->post_slot(slot));
   const double bb = ctx->read_slot(slot);
   if (bb == 0) {
     out.status = 1;
@@ -1017,7 +1017,7 @@ MixedResult mixed_reliable_bicg(alien_hip_ctx* ctx, int n, RBMat<double> A64, RB
   auto restart = [&](int it) {
     launch_demote(s, n, r64.data(), F.r.data());
     const int sl = ctx->take_slot();
-    launch_dot<float>(s, ctx->red(), n, F.r.data(), F.r.data(), ctx->dslot(sl));
+    launch_dot<float>(s, ctx->red_once(), n, F.r.data(), F.r.data(), ctx->dslot(sl), ctx->post_slot(sl));
     F.start(ctx->read_slot(sl), crit, it, max_it);
   };
   restart(0);
@@ -1123,7 +1123,7 @@ MixedResult mixed_reliable_bicg(alien_hip_ctx* ctx, int n, RBMat<double> A64, RB
     // reliable update: r <- b - A x64, rho1 <- r.r0
     launch_demote(s, n, r64.data(), F.r.data());
     const int sl = ctx->take_slot();
-    launch_dot<float>(s, ctx->red(), n, F.r.data(), F.r0.data(), ctx->dslot(sl));
+    launch_dot<float>(s, ctx->red_once(), n, F.r.data(), F.r0.data(), ctx->dslot(sl), ctx->post_slot(sl));
     cur.rho1 = ctx->read_slot(sl);
     cur.rr = rr64;
     cur.rrmax = rr64;
