@@ -5,9 +5,9 @@
 // lane (yl, zl) marches along x with a skew of yl + zl steps, and so meets each neighbour inside
 // the pencil one step behind it: the own line's in a register, the others' by lane exchange. Only
 // the values on two faces travel to the next pencils, ny / 8 + nz / 8 - 2 trips in a row (30 at
-// 128^3). Measured there in FP64, against the sync-free level sweeps: lower sweep 156 us (653),
-// upper 171 us (667), factorisation 258 us (382 launches, 7.5 ms), and no level sets to build on
-// the host (21 ms); BiCGStab to 1e-8, 8 iterations, set-up included: 52.7 -> 10.8 ms.
+// 128^3). Measured there in FP64, against the sync-free level sweeps: lower sweep 115 us (653),
+// upper 133 us (667), factorisation 204 us (382 launches, 7.5 ms), and no level sets to build on
+// the host (21 ms); BiCGStab to 1e-8, 8 iterations, set-up included: 53.1 -> 9.3 ms.
 //
 // Storage ("skewed"): step s of pencil p holds the 64 values of its lanes contiguously at
 // (p * steps + s) * 64 + lane, x = s - yl - zl; a step's operands are coalesced loads, and the
@@ -30,7 +30,6 @@ namespace alien_hip {
 
 constexpr int kPen = 8;         // lines of a pencil per direction
 constexpr int kPenChunk = 8;    // steps whose operands are loaded together
-constexpr int kPenDepth = 1;    // of the sweeps, chunks whose loads are in flight
 constexpr int kPenSkew = 2 * (kPen - 1);
 static_assert(kPen * kPen == kWave && kPen * kPenChunk == kWave, "a face's chunk is one load of the wavefront");
 
@@ -160,9 +159,13 @@ __device__ __forceinline__ double lane_y(double v) {
 // Two sets of faces and tickets: the lower sweep uses set 0 and clears set 1, the upper sweep and
 // the factorisation the other way round, so neither needs a clearing launch before it. Waits are
 // bounded (limit polls); one that runs out raises work[2] and the redo kernel follows.
-// Bound by latency: about 0.19 us a step (dependent instructions of a lone wavefront) and per trip
-// between pencils 15 steps of skew and chunk and 1.6 us from store to load. Fetching 2 or 3 chunks
-// ahead instead of one changed nothing (153 and 151 us lower, 176 and 179 us upper).
+// Bound by the instructions and waits of a lone wavefront, 0.12 us a lower step and 0.17 an upper one (a lane
+// exchange, three dependent subtractions, the upper's division), and per trip between pencils by 15 steps of skew
+// and chunk and 1.6 us from store to load. Operands of a step of the next chunk are loaded during each lane exchange, at
+// a scalar address + lane + constant, into the other of two register sets: nothing waits for a load before its
+// step (copying or polling beside them waited for all: 156 and 171 us). The upper sweep's results go out 8 x of 8 lines
+// a store from LDS (64 lines a store, 8 bytes each: 165 us). Tried: the exchange in the vector unit (row rotation,
+// permlane swaps) in place of ds_bpermute, 142 against 117 us.
 enum PencilSweep { kPenLower = 0, kPenUpper = 1, kPenFactor = 2 };
 template <typename T, int KIND>
 __global__ void __launch_bounds__(kWave) k_pencil_sweep(PencilFactor<T> F, const double* __restrict__ trans,
@@ -176,19 +179,19 @@ __global__ void __launch_bounds__(kWave) k_pencil_sweep(PencilFactor<T> F, const
   const PencilGrid& g = F.g;
   const int np = g.pencils(), S = g.steps;
   const int lane = threadIdx.x, yl = lane % kPen, zl = lane / kPen;
-  __shared__ T face[2][kWave];
+  __shared__ T face[3][kWave], val[C][kWave]; // face[2]: zeros
   int* err = F.work + 2;
 
   int tk = 0;
   if (lane == 0) tk = __hip_atomic_fetch_add(F.work + set, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   tk = __builtin_amdgcn_readfirstlane(tk);
   if (tk >= np) return;
-  const int p = F.order[UP ? np - 1 - tk : tk];
+  const int p = __builtin_amdgcn_readfirstlane(F.order[UP ? np - 1 - tk : tk]);
   const int b = p % g.py, c = p / g.py;
   const int y = b * kPen + yl, z = c * kPen + zl;
   const bool rowok = y < g.ny && z < g.nz;
   const long npos = g.positions();
-  const long base = (long)p * S * kWave + lane;
+  const long base = (long)p * S * kWave; // uniform: a step's operand is at a scalar address + the lane + a constant
   const long line = rowok ? ((long)z * g.ny + y) * g.nx : 0;
   const bool hasy = UP ? y < g.ny - 1 : y > 0, hasz = UP ? z < g.nz - 1 : z > 0;
   // z, y, x neighbour's coefficient (the sweep's own triangle)
@@ -197,6 +200,7 @@ __global__ void __launch_bounds__(kWave) k_pencil_sweep(PencilFactor<T> F, const
   T* ax = F.base + (UP ? 4 : 2) * npos + base;
   T* dd = F.base + 3 * npos + base;
   T* tt = F.t + base;
+  constexpr int dir = UP ? -kWave : kWave; // from step to step
 
   U* halo = reinterpret_cast<U*>(F.halo) + set * g.halo();
   U* hy = halo;                         // y faces
@@ -214,8 +218,11 @@ __global__ void __launch_bounds__(kWave) k_pencil_sweep(PencilFactor<T> F, const
   constexpr int edge = UP ? kPen - 1 : 0, far = kPen - 1 - edge; // lines fed by, and feeding, another pencil
   // this lane's part in a face's chunk: step fj of it, line fk
   const int fj = lane / kPen, fk = lane % kPen;
-  const U* ylo = hy + ((long)(UP ? p + 1 : p - 1) * S) * kPen + fk;
-  const U* zlo = hz + ((long)(UP ? p + g.py : p - g.py) * S) * kPen + fk;
+  const U* yfrom = hy + (long)(fromy ? (UP ? p + 1 : p - 1) : p) * S * kPen; // (a pencil's own where none feeds it: not used)
+  const U* zfrom = hz + (long)(fromz ? (UP ? p + g.py : p - g.py) : p) * S * kPen;
+  U* yto = hy + (long)p * S * kPen;
+  U* zto = hz + (long)p * S * kPen;
+  const bool line_y = fromy && c * kPen + fk < g.nz, line_z = fromz && b * kPen + fk < g.ny; // the fed line exists
   auto step = [&](int s) { return UP ? S - 1 - s : s; };
   // Loads and stores of the march are unconditional (lanes without one use a place of their own):
   // memory operations complete in order, and behind a branch the compiler would wait for all of them.
@@ -224,122 +231,143 @@ __global__ void __launch_bounds__(kWave) k_pencil_sweep(PencilFactor<T> F, const
     bool ny, nz; // needed
   };
   auto face_load = [&](int s0, Face& f) {
-    const int s = step(s0 + fj), x = s - edge - fk;
-    const bool in_x = x >= 0 && x < g.nx;
-    f.ny = fromy && in_x && c * kPen + fk < g.nz;
-    f.nz = fromz && in_x && b * kPen + fk < g.ny;
-    const long o = (long)(s + far - edge) * kPen;
-    const U* none = hy + (long)p * S * kPen + fk;
-    f.y = __hip_atomic_load(f.ny ? ylo + o : none, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    f.z = __hip_atomic_load(f.nz ? zlo + o : none, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int s = step(s0 + fj);
+    const bool in_x = (unsigned)(s - edge - fk) < (unsigned)g.nx;
+    f.ny = line_y && in_x;
+    f.nz = line_z && in_x;
+    const unsigned o = (unsigned)min(max(s + far - edge, 0), S - 1) * kPen + fk;
+    f.y = __hip_atomic_load(yfrom + o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    f.z = __hip_atomic_load(zfrom + o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   };
   struct Ops {
     T z[C], y[C], x[C], r[C], d[C];
     T tz[FAC ? C : 1], ty[FAC ? C : 1], tx[FAC ? C : 1];
   };
-  auto fetch = [&](int s0, Ops& o) {
-#pragma unroll
-    for (int j = 0; j < C; ++j) {
-      const int s = step(s0 + j);
-      const long q = (long)s * kWave;
-      o.z[j] = az[q];
-      o.y[j] = ay[q];
-      o.x[j] = ax[q];
-      if constexpr (KIND == kPenLower) o.r[j] = in[line + min(max(s - yl - zl, 0), g.nx - 1)];
-      if constexpr (UP) o.r[j] = tt[q];
-      if constexpr (UP || FAC) o.d[j] = dd[q];
-      if constexpr (FAC) {
-        o.tz[j] = trans[base + q];
-        o.ty[j] = trans[npos + base + q];
-        o.tx[j] = trans[2 * npos + base + q];
-      }
+  // step s0 + j's operands; u: step(s0) * kWave, xc: the lane's x at s0
+  auto fetch = [&](long u, int xc, int j, Ops& o) {
+    const int q = j * dir;
+    o.z[j] = (az + u + lane)[q];
+    o.y[j] = (ay + u + lane)[q];
+    o.x[j] = (ax + u + lane)[q];
+    if constexpr (KIND == kPenLower) o.r[j] = in[line + min(max(xc + j, 0), g.nx - 1)];
+    if constexpr (UP) o.r[j] = (tt + u + lane)[q];
+    if constexpr (UP || FAC) o.d[j] = (dd + u + lane)[q];
+    if constexpr (FAC) {
+      o.tz[j] = (trans + base + u + lane)[q];
+      o.ty[j] = (trans + npos + base + u + lane)[q];
+      o.tx[j] = (trans + 2 * npos + base + u + lane)[q];
     }
   };
 
   T own = T(0);
   Face fc;
-  // the steps s0 .. s0 + C - 1 on their operands o; refetches o for the chunk `ahead` when there is one
-  auto march = [&](int s0, Ops& o, int ahead) {
-    long spins = 0;
-    while (__any((fc.ny && fc.y == SfBits<T>::kSentinel) || (fc.nz && fc.z == SfBits<T>::kSentinel))) {
-      if (++spins > limit) {
-        if (lane == 0) __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        break;
-      }
-      if ((spins & 255) == 0 && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) break;
-      __builtin_amdgcn_s_sleep(1);
-      face_load(s0, fc);
+  // a lane takes the face's value, or 0 for want of a neighbour, in place of another lane's
+  const bool face_lane_y = yl == edge || !hasy, face_lane_z = zl == edge || !hasz;
+  const T* face_y = &face[yl == edge && hasy ? 0 : 2][zl];
+  const T* face_z = &face[zl == edge && hasz ? 1 : 2][yl];
+  face[2][lane] = T(0);
+  // the steps s0 .. s0 + C - 1 on their operands o; o_next: those of the chunk at `ahead`
+  auto march = [&](int s0, const Ops& o, int ahead, Ops& o_next) {
+    // A first look that waits for the faces alone, then the polls: one loop for both would wait, each time, for
+    // every load issued since (the next chunk's operands).
+    auto missing = [&] {
+      return __any(((int)fc.ny & (int)(fc.y == SfBits<T>::kSentinel)) | ((int)fc.nz & (int)(fc.z == SfBits<T>::kSentinel)));
+    };
+    if (missing()) {
+      long spins = 0;
+      do {
+        if (++spins > limit) {
+          if (lane == 0) __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          break;
+        }
+        if ((spins & 255) == 0 && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) break;
+        __builtin_amdgcn_s_sleep(1);
+        face_load(s0, fc);
+      } while (missing());
     }
-    face[0][lane] = SfBits<T>::value(fc.y);
-    face[1][lane] = SfBits<T>::value(fc.z);
+    face[0][lane] = fc.ny ? SfBits<T>::value(fc.y) : T(0);
+    face[1][lane] = fc.nz ? SfBits<T>::value(fc.z) : T(0);
     __syncthreads(); // (one wavefront: orders the LDS accesses)
     T ey[C], ez[C];
 #pragma unroll
     for (int j = 0; j < C; ++j) {
-      ey[j] = face[0][j * kPen + zl];
-      ez[j] = face[1][j * kPen + yl];
+      ey[j] = face_y[j * kPen];
+      ez[j] = face_z[j * kPen];
     }
     face_load(min(s0 + C, S - C), fc);
-    __syncthreads();
+    const long u = (long)step(s0) * kWave, un = (long)step(ahead) * kWave;
+    const int x0 = step(s0) - yl - zl, xn = step(ahead) - yl - zl;
 #pragma unroll
     for (int j = 0; j < C; ++j) {
-      const int s = step(s0 + j), x = s - yl - zl;
-      const bool ok = rowok && x >= 0 && x < g.nx;
-      const bool hasx = UP ? x < g.nx - 1 : x > 0;
-      const T ly = lane_y<UP>(own);
+      const int x = UP ? x0 - j : x0 + j, q = j * dir;
+      // The step's chain: a lane exchange, then a subtraction per neighbour. While the exchange is under way
+      // the operands of a step of the next chunk are asked for.
       const T lz = UP ? __shfl_down(own, kPen, kWave) : __shfl_up(own, kPen, kWave);
-      const T qy = yl == edge ? ey[j] : ly, qz = zl == edge ? ez[j] : lz;
-      const long q = (long)s * kWave;
+      const T ly = lane_y<UP>(own);
+      fetch(un, xn, j, o_next);
+      const bool hasx = UP ? x < g.nx - 1 : x > 0;
+      const T qy = face_lane_y ? ey[j] : ly, qx = hasx ? own : T(0);
+      __builtin_amdgcn_sched_barrier(0);
+      const T qz = face_lane_z ? ez[j] : lz;
       T v;
+      // An absent neighbour's coefficient is +0 and so is its value here: subtracting their product changes
+      // nothing, not even a zero's sign.
       if constexpr (KIND == kPenLower) {
-        v = o.r[j];
-        if (hasz) v = v - o.z[j] * qz;
-        if (hasy) v = v - o.y[j] * qy;
-        if (hasx) v = v - o.x[j] * own;
-        tt[q] = v;
+        v = o.r[j] - o.z[j] * qz;
+        v = v - o.y[j] * qy;
+        v = v - o.x[j] * qx;
+        (tt + u + lane)[q] = v;
       } else if constexpr (UP) {
-        v = o.r[j];
-        if (hasx) v = v - o.x[j] * own;
-        if (hasy) v = v - o.y[j] * qy;
-        if (hasz) v = v - o.z[j] * qz;
+        v = o.r[j] - o.x[j] * qx;
+        v = v - o.y[j] * qy;
+        v = v - o.z[j] * qz;
         v = v / o.d[j];
-        T* to = ok ? out + line + x : tt + q; // a padding step's t is never read
-        *to = v;
       } else {
         const T fz = hasz ? o.z[j] / qz : T(0), fy = hasy ? o.y[j] / qy : T(0), fx = hasx ? o.x[j] / own : T(0);
         v = o.d[j];
         if (hasz) v = v - fz * o.tz[j];
         if (hasy) v = v - fy * o.ty[j];
         if (hasx) v = v - fx * o.tx[j];
-        az[q] = fz;
-        ay[q] = fy;
-        ax[q] = fx;
-        dd[q] = v;
+        (az + u + lane)[q] = fz;
+        (ay + u + lane)[q] = fy;
+        (ax + u + lane)[q] = fx;
+        (dd + u + lane)[q] = v;
       }
       own = v;
-      // the faces' values of the chunk, gathered for one store each
-      if (yl == far) face[0][j * kPen + zl] = v;
-      if (zl == far) face[1][j * kPen + yl] = v;
+      val[j][lane] = v;
     }
-    if (ahead < S) fetch(ahead, o);
     __syncthreads();
     // (steps outside a line leave values there that nothing reads)
-    const long fo = ((long)p * S + step(s0 + fj)) * kPen + fk;
-    if (toy) __hip_atomic_store(hy + fo, SfBits<T>::bits(face[0][lane]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (toz) __hip_atomic_store(hz + fo, SfBits<T>::bits(face[1][lane]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const U vy = SfBits<T>::bits(val[fj][fk * kPen + far]), vz = SfBits<T>::bits(val[fj][far * kPen + fk]);
+    const unsigned fo = (unsigned)step(s0 + fj) * kPen + fk;
+    if (toy) __hip_atomic_store(yto + fo, vy, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (toz) __hip_atomic_store(zto + fo, vz, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if constexpr (UP) {
+      // the chunk's results, 8 consecutive x of 8 lines a store (a lane's own step by step is 64 lines a store):
+      // step fk of the lines (fj, 0 .. 7)
+      const int xs = step(s0 + fk) - fj, xend = b * kPen + fj < g.ny ? g.nx : 0;
+      T* to = out + (((long)c * kPen * g.ny + b * kPen + fj) * g.nx + xs);
+      T* none = tt + (long)(S - 1) * kWave; // a padding step's t is never read
+#pragma unroll
+      for (int m = 0; m < kPen; ++m) {
+        const bool ok = (unsigned)(xs - m) < (unsigned)(c * kPen + m < g.nz ? xend : 0);
+        *(ok ? to : none) = val[fk][m * kPen + fj];
+        to += (long)g.ny * g.nx - 1;
+      }
+    }
     __syncthreads();
   };
 
-  constexpr int D = FAC ? 1 : kPenDepth; // chunks fetched ahead
-  Ops buf[D + 1];
+  // two sets of operands in turn: the chunk's are used where they were loaded, no register is moved
+  // (a copy would wait for its load)
+  Ops even, odd;
 #pragma unroll
-  for (int r = 0; r <= D; ++r)
-    if (r * C < S) fetch(r * C, buf[r]);
+  for (int j = 0; j < C; ++j) fetch((long)step(0) * kWave, step(0) - yl - zl, j, even);
   face_load(0, fc);
-  for (int s0 = 0; s0 < S; s0 += (D + 1) * C) {
-#pragma unroll
-    for (int r = 0; r <= D; ++r)
-      if (s0 + r * C < S) march(s0 + r * C, buf[r], s0 + (r + D + 1) * C);
+  for (int s0 = 0; s0 < S; s0 += 2 * C) {
+    march(s0, even, min(s0 + C, S - C), odd);
+    if (s0 + C >= S) break;
+    march(s0 + C, odd, min(s0 + 2 * C, S - C), even);
   }
 }
 
