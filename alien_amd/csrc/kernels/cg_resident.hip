@@ -14,11 +14,13 @@
 // Every workgroup has to be running: there are no more than compute units, a workgroup fits beside
 // any other kernel's once that ends, and the caller keeps a second such launch of the process off
 // the device (resident_mutex); what else might hold one back too long runs the waits out of polls.
-// Bound by the latency of the sums, about 3 us each. An iteration of Jacobi-CG in FP64 against the
-// graph of launches: 14 x 11 x 9 cells 3.9 us (16), 32^3 5.6 (18), 64^3 8.5 (21), 80^3 (two rows per
-// lane, which spill) 21 (30); FP32 in the mixed solver 9.4 (19) at 64^3; Chebyshev of degree 3 16
-// (39) at 32^3. One sum per workgroup, with a tree of its own, took 7.7 us at 64^3, but its iterates
-// are not the launches'. Exchanging through barriers (stores settled, then a sum, then loads) took 10.4.
+// Bound by the latency of the sums, about 3 us each, and in one workgroup by its instructions. An iteration of
+// Jacobi-CG in FP64 against the graph of launches: 14 x 11 x 9 cells 2.8 us (16), 32^3 5.6 (18), 64^3 8.5 (21), 80^3 (two
+// rows per lane, which spill) 22 (30); FP32 in the mixed solver 7.9 (19) at 64^3; Chebyshev of degree 3 16 (39) at
+// 32^3. Each barrier of a sum costs some 0.1 us: one after the totals are read was spared by a place of their own
+// (64^3 mixed 9.1 -> 8.7 us a solve's iteration), two sets of places in turn, indexed, cost more than they spared (10.3).
+// One sum per workgroup, with a tree of its own, took 7.7 us at 64^3, but its iterates are not the launches'.
+// Exchanging through barriers (stores settled, then a sum, then loads) took 10.4.
 #include "../alien_hip_internal.h"
 #include "../alien/hip/HIPContext.h"
 #include "device_common.h"
@@ -73,19 +75,77 @@ __device__ __forceinline__ bool give_up(const GridSums& g, long spins, int* fail
 }
 struct SumLds {
   double term[2][2][kResBlock]; // by value and round
-  double wave[2][2][kResWaves];
-  double part[2][kResBlock]; // ONE: the partials
+  double wave[2][2][kResWaves], fin[2][kResWaves];
+  double one[2][2][2][kResWaves]; // block_total's, by turn: none of its sums waits for the readers of the last
   int failed;
 };
+// The same within a launch of one workgroup. Its partials, at most 8, lie in the first 64 slots (bundle_walk
+// gives row block l < 64 workgroup 8 l): after one or two barriers every wavefront adds them by the finalize's tree for
+// itself.
+template <int KIND, int NV, int R>
+__device__ __forceinline__ void block_total(unsigned& phase, int n, const double (&term)[NV][R], double (&out)[NV], SumLds& L) {
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wid = tid / kWave;
+  constexpr int W = kRowWaves, G = KIND == kSumRows ? 4 : KIND == kSumPairs ? 2 : 1;
+  static_assert(G * R <= kWave / kXcds && (int)kXcdChunk >= G * R, "row block l is workgroup 8 l");
+  auto& wave = L.one[++phase & 1];
+  if constexpr (KIND == kSumRows) {
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const double s = wave_total(term[0][q]);
+      if (lane == 0) wave[0][q][wid] = s;
+    }
+  } else if constexpr (KIND == kSumPairs) {
+    if (wid & 1)
+#pragma unroll
+      for (int q = 0; q < R; ++q) L.term[0][q][tid] = term[0][q];
+    __syncthreads();
+    if (!(wid & 1))
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        const double s = wave_total(term[0][q] + L.term[0][q][tid + kWave]);
+        if (lane == 0) wave[0][q][wid / 2] = s;
+      }
+  } else {
+#pragma unroll
+    for (int v = 0; v < NV; ++v)
+#pragma unroll
+      for (int q = 0; q < R; ++q) L.term[v][q][tid] = term[v][q];
+    __syncthreads();
+    if (wid < W * NV * R) {
+      const int v = wid / W % NV, q = wid / W / NV;
+      const double* t = L.term[v][q] + tid % kBlock;
+      const double s = wave_total(((t[0] + t[kBlock]) + t[2 * kBlock]) + t[3 * kBlock]);
+      if (lane == 0) wave[v][q][wid % W] = s;
+    }
+  }
+  __syncthreads();
+  const int real = (n + kResBlock / G - 1) / (kResBlock / G);
+  const int l = KIND == kSumStream ? lane : lane % kXcds ? real : lane / kXcds;
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    double acc = 0;
+    if (l < real) {
+      double s = 0;
+#pragma unroll
+      for (int w = 0; w < W; ++w) s += wave[v][l / G][l % G * W + w];
+      acc += s;
+    }
+    out[v] = 0.0 + wave_total(acc);
+  }
+}
 template <int KIND, int NV, bool ONE, int R>
 __device__ __forceinline__ bool grid_sum(GridSums& g, int n, const double (&term)[NV][R], double (&out)[NV], SumLds& L,
                                          bool settle) {
+  if constexpr (ONE) {
+    block_total<KIND, NV, R>(g.phase, n, term, out, L);
+    return true;
+  }
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wid = tid / kWave;
   constexpr int W = kRowWaves; // wavefronts of a launch's workgroup, whose totals are added in turn
   static_assert(R <= 2 && NV <= 2 && W * NV * R <= kResWaves, "");
   static_assert(kRowBlock == kBlock && kBlock * kEPT == kResBlock, "a workgroup holds whole workgroups of the launches");
   ++g.phase;
-  if (settle && !ONE) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if (settle) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   constexpr int G = KIND == kSumRows ? 4 : KIND == kSumPairs ? 2 : 1; // partials per 1024 rows
   const int per = kResBlock / G, real = (n + per - 1) / per;
   constexpr int C = (int)kXcdChunk, XC = kXcds * C;
@@ -137,13 +197,9 @@ __device__ __forceinline__ bool grid_sum(GridSums& g, int n, const double (&term
     for (int w = 0; w < W; ++w) s += L.wave[v][q][k * W + w];
     if (l < real) {
       const int p = slot_of(l);
-      if constexpr (ONE) {
-        L.part[v][p] = s;
-      } else {
-        const Halves h = halves(s);
-        agent_store(set + 2 * v * kResidentSlots + p, tag | h.lo);
-        agent_store(set + (2 * v + 1) * kResidentSlots + p, tag | h.hi);
-      }
+      const Halves h = halves(s);
+      agent_store(set + 2 * v * kResidentSlots + p, tag | h.lo);
+      agent_store(set + (2 * v + 1) * kResidentSlots + p, tag | h.hi);
     }
   }
   __syncthreads();
@@ -152,27 +208,22 @@ __device__ __forceinline__ bool grid_sum(GridSums& g, int n, const double (&term
   for (int v = 0; v < NV; ++v) acc[v] = 0;
   for (int p = tid; p < nslots; p += kResBlock) {
     if (row_order(p) >= real) continue; // a workgroup without rows: + 0
-    if constexpr (ONE) {
+    unsigned long long w[2 * NV];
+    for (long spins = 1;; ++spins) {
+      bool there = true;
 #pragma unroll
-      for (int v = 0; v < NV; ++v) acc[v] += L.part[v][p];
-    } else {
-      unsigned long long w[2 * NV];
-      for (long spins = 1;; ++spins) {
-        bool there = true;
+      for (int k = 0; k < 2 * NV; ++k) w[k] = agent_load(set + k * kResidentSlots + p);
 #pragma unroll
-        for (int k = 0; k < 2 * NV; ++k) w[k] = agent_load(set + k * kResidentSlots + p);
-#pragma unroll
-        for (int k = 0; k < 2 * NV; ++k) there = there && (unsigned)(w[k] >> 32) == g.phase;
-        if (there || give_up(g, spins, &L.failed)) break;
-      }
-#pragma unroll
-      for (int v = 0; v < NV; ++v) acc[v] += whole((unsigned)w[2 * v], (unsigned)w[2 * v + 1]);
+      for (int k = 0; k < 2 * NV; ++k) there = there && (unsigned)(w[k] >> 32) == g.phase;
+      if (there || give_up(g, spins, &L.failed)) break;
     }
+#pragma unroll
+    for (int v = 0; v < NV; ++v) acc[v] += whole((unsigned)w[2 * v], (unsigned)w[2 * v + 1]);
   }
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
     const double s = wave_total(acc[v]);
-    if (lane == 0) L.wave[v][0][wid] = s;
+    if (lane == 0) L.fin[v][wid] = s;
   }
   __syncthreads();
   if (L.failed) return false;
@@ -180,9 +231,9 @@ __device__ __forceinline__ bool grid_sum(GridSums& g, int n, const double (&term
   for (int v = 0; v < NV; ++v) {
     out[v] = 0;
 #pragma unroll
-    for (int w = 0; w < kResWaves; ++w) out[v] += L.wave[v][0][w];
+    for (int w = 0; w < kResWaves; ++w) out[v] += L.fin[v][w];
   }
-  __syncthreads(); // L is free again
+  // (no barrier: the next sum writes term and wave, and fin only behind a barrier of its own)
   return true;
 }
 
@@ -196,9 +247,14 @@ __device__ __forceinline__ bool grid_sum(GridSums& g, int n, const double (&term
 // An entry is cleared by its owner after a sum that all its readers reached by having read it, and
 // written again only after the p.q sum in between, which settles the clearing.
 // ONE: a single workgroup, the exchange vectors in LDS with barriers instead of sentinels (through
-// memory an exchange inside one workgroup costs as much as between two).
-// PQ: the tree of q = A p's p.q on this operand (kSumRows or kSumPairs).
-template <typename T, int R, bool ONE, bool CHEB, int PQ>
+// memory an exchange inside one workgroup costs as much as between two; 14 x 11 x 9: 3.9 us an iteration with the sums of
+// several workgroups and z exchanged, 2.8 with block_total and p). p itself is exchanged, in ex[0]: one
+// barrier more, and neither the copies' registers (two FP64 rows a lane spilled with them) nor their operations.
+// PQ: the tree of q = A p's p.q on this operand (kSumRows or kSumPairs). K: entries of a row at most.
+// Where a row has no j-th entry, ONE (bound by its instructions: 16 wavefronts on one compute unit) multiplies two zeros,
+// the value and the vector's entry past the last, and adds +0 to a sum that is never -0; a wavefront without
+// rows in a round does none of its work.
+template <typename T, int R, int K, bool ONE, bool CHEB, int PQ>
 __global__ void __launch_bounds__(kResBlock) k_cg_resident(int n, RBMat<T> A, const T* __restrict__ invd, T* x, T* r,
                                                             T* z, T* p, T* ex, CGState* st, GridSums g,
                                                             ResidentCheb cb, int iters, int check, double below) {
@@ -213,11 +269,16 @@ __global__ void __launch_bounds__(kResBlock) k_cg_resident(int n, RBMat<T> A, co
   g.phase = (unsigned)g.head[0];
   if (threadIdx.x == 0) lds.failed = 0;
 
-  constexpr int K = kResSlots;
+  const int stride = ONE ? n + 1 : n; // of the exchange vectors
+  // whether this wavefront has rows in round q
+  auto mine = [&](int q) {
+    return !ONE || __builtin_amdgcn_readfirstlane((int)(q * kResBlock + (threadIdx.x & ~(kWave - 1)))) < n;
+  };
   int row[R];
   unsigned on[R];    // bit j: the row has entry j; bit 31: the row exists
   unsigned at[R][K]; // byte offset of entry j's column, or of the row itself where there is none
-  T a[R][K], pc[R][K], xv[R], rv[R], dv[R], zv[R], pv[R];
+  T a[R][K], xv[R], rv[R], dv[R], zv[R], pv[R];
+  T pc[ONE ? 1 : R][ONE ? 1 : K];
   U* const exu = reinterpret_cast<U*>(ONE ? (char*)own_ex : (char*)ex);
 #pragma unroll
   for (int q = 0; q < R; ++q) {
@@ -232,7 +293,7 @@ __global__ void __launch_bounds__(kResBlock) k_cg_resident(int n, RBMat<T> A, co
     for (int j = 0; j < K; ++j) {
       const int s = s0 + min(j, max(w - 1, 0));
       a[q][j] = T(0);
-      at[q][j] = (unsigned)row[q] * (unsigned)sizeof(T);
+      at[q][j] = (unsigned)(ONE ? n : row[q]) * (unsigned)sizeof(T);
       if (j < w) {
         a[q][j] = A.bv[(long)s * kWave + lane];
         if (in && (A.dmask[s] >> lane & 1)) {
@@ -251,14 +312,14 @@ __global__ void __launch_bounds__(kResBlock) k_cg_resident(int n, RBMat<T> A, co
     T acc = 0;
 #pragma unroll
     for (int j = 0; j < K; ++j)
-      if (on[q] >> j & 1) acc = acc + a[q][j] * v[j];
+      if (ONE || (on[q] >> j & 1)) acc = acc + a[q][j] * v[j];
     return acc;
   };
   auto publish = [&](int e, const T (&v)[R]) {
 #pragma unroll
     for (int q = 0; q < R; ++q)
       if (on[q] >> 31) {
-        if constexpr (ONE) exu[e * n + row[q]] = SfBits<T>::bits(v[q]);
+        if constexpr (ONE) exu[e * stride + row[q]] = SfBits<T>::bits(v[q]);
         else agent_store(exu + (size_t)e * n + row[q], SfBits<T>::bits(v[q]));
       }
   };
@@ -274,7 +335,7 @@ __global__ void __launch_bounds__(kResBlock) k_cg_resident(int n, RBMat<T> A, co
     U u[K];
     if constexpr (ONE) {
 #pragma unroll
-      for (int j = 0; j < K; ++j) out[j] = *reinterpret_cast<const T*>(own_ex + e * n * sizeof(T) + at[q][j]);
+      for (int j = 0; j < K; ++j) out[j] = *reinterpret_cast<const T*>(own_ex + e * stride * sizeof(T) + at[q][j]);
       return;
     }
     for (long spins = 1;; ++spins) {
@@ -291,16 +352,19 @@ __global__ void __launch_bounds__(kResBlock) k_cg_resident(int n, RBMat<T> A, co
 #pragma unroll
     for (int j = 0; j < K; ++j) out[j] = SfBits<T>::value(u[j]);
   };
+  if constexpr (!ONE)
 #pragma unroll
-  for (int q = 0; q < R; ++q)
+    for (int q = 0; q < R; ++q)
 #pragma unroll
-    for (int j = 0; j < K; ++j)
-      pc[q][j] = *reinterpret_cast<const T*>(reinterpret_cast<const char*>(p) + at[q][j]);
+      for (int j = 0; j < K; ++j)
+        pc[q][j] = *reinterpret_cast<const T*>(reinterpret_cast<const char*>(p) + at[q][j]);
 
+  if constexpr (ONE)
+    if (threadIdx.x < (CHEB ? 2 + cb.order : 2)) exu[threadIdx.x * stride + n] = 0;
   __syncthreads();
   for (int e = 0; e < (CHEB ? 2 + cb.order : 2); ++e) clear(e);
   if (CHEB) publish(2, rv);
-  else publish(1, zv);
+  else if (!ONE) publish(1, zv);
   double none[1][R] = {}, s1[1];
   if (!grid_sum<kSumStream, 1, ONE, R>(g, n, none, s1, lds, true)) return;
   for (int i = 0;;) {
@@ -314,6 +378,9 @@ __global__ void __launch_bounds__(kResBlock) k_cg_resident(int n, RBMat<T> A, co
         if (ONE && m) __syncthreads();
 #pragma unroll
         for (int q = 0; q < R; ++q) {
+          if (m == 0) cp[q] = y[q] = T(0);
+          xy[0][q] = 0.0;
+          if (!mine(q)) continue;
           T v[K];
           gather(2 + m, q, v);
           const T t = sum(q, v);
@@ -329,7 +396,7 @@ __global__ void __launch_bounds__(kResBlock) k_cg_resident(int n, RBMat<T> A, co
           }
           xy[0][q] = on[q] >> 31 ? 0.0 + (double)rv[q] * (double)y[q] : 0.0;
         }
-        publish(m == cb.order - 1 ? ze : 3 + m, y);
+        if (m < cb.order - 1 || !ONE) publish(m == cb.order - 1 ? ze : 3 + m, y);
       }
       if (!grid_sum<kSumRows, 1, ONE, R>(g, n, xy, s1, lds, false)) return;
       for (int e = 2; e < 2 + cb.order; ++e) clear(e);
@@ -340,14 +407,28 @@ __global__ void __launch_bounds__(kResBlock) k_cg_resident(int n, RBMat<T> A, co
     const T beta = (T)(rho1 / rho);
     T qv[R];
     double pq[1][R];
+    if constexpr (ONE) {
+#pragma unroll
+      for (int q = 0; q < R; ++q) pv[q] = zv[q] + beta * pv[q];
+      publish(0, pv);
+      __syncthreads();
+    }
 #pragma unroll
     for (int q = 0; q < R; ++q) {
+      qv[q] = T(0);
+      pq[0][q] = 0.0;
+      if (!mine(q)) continue;
       T v[K];
-      gather(ze, q, v);
+      if constexpr (ONE) {
+        gather(0, q, v);
+        qv[q] = sum(q, v);
+      } else {
+        gather(ze, q, v);
 #pragma unroll
-      for (int j = 0; j < K; ++j) pc[q][j] = v[j] + beta * pc[q][j];
-      pv[q] = zv[q] + beta * pv[q];
-      qv[q] = sum(q, pc[q]);
+        for (int j = 0; j < K; ++j) pc[q][j] = v[j] + beta * pc[q][j];
+        pv[q] = zv[q] + beta * pv[q];
+        qv[q] = sum(q, pc[q]);
+      }
       pq[0][q] = on[q] >> 31 ? 0.0 + (double)pv[q] * (double)qv[q] : 0.0;
     }
     if (!grid_sum<PQ, 1, ONE, R>(g, n, pq, s1, lds, true)) return;
@@ -370,7 +451,7 @@ __global__ void __launch_bounds__(kResBlock) k_cg_resident(int n, RBMat<T> A, co
       }
     }
     if (CHEB) publish(2, rv);
-    else publish(ze ^ 1, zv);
+    else if (!ONE) publish(ze ^ 1, zv);
     if (!grid_sum<kSumStream, CHEB ? 1 : 2, ONE, R>(g, n, rs, s, lds, false)) return;
     // Iteration::stop and the scalars, as k_finalize's kFinXR / kFinXRDiag
     rho = rho1;
@@ -418,7 +499,7 @@ bool resident_plan(int n, const RBMat<T>& A, int cus, int cheb_order, ResidentPl
   if (rb_blocks(n, A) != bundle_blocks_max(n)) return false;
   P.pairs = A.uni > 0 && A.uni <= kUniPairMaxSlots;
   P.exchange = 2 + cheb_order;
-  P.lds = P.exchange * n * sizeof(T);
+  P.lds = P.exchange * (n + 1) * sizeof(T);
   P.one = n <= 2 * kResBlock && P.lds <= 40 * 1024;
   if (!P.one) P.lds = 0;
   const long blocks = P.one ? 1 : std::min(cus, kResidentMaxBlocks);
@@ -427,10 +508,14 @@ bool resident_plan(int n, const RBMat<T>& A, int cus, int cheb_order, ResidentPl
 }
 
 template <typename T, int R, bool ONE, bool CHEB>
-static const void* resident_kernel(bool pairs) {
+static const void* resident_kernel(bool pairs, int width) {
+  // rows of at most 7 entries (the 7-point stencils) do not pay for the eighth
   if constexpr (sizeof(T) == 4)
-    if (pairs) return (const void*)k_cg_resident<T, R, ONE, CHEB, kSumPairs>;
-  return (const void*)k_cg_resident<T, R, ONE, CHEB, kSumRows>;
+    if (pairs)
+      return width <= 7 ? (const void*)k_cg_resident<T, R, 7, ONE, CHEB, kSumPairs>
+                        : (const void*)k_cg_resident<T, R, kResSlots, ONE, CHEB, kSumPairs>;
+  return width <= 7 ? (const void*)k_cg_resident<T, R, 7, ONE, CHEB, kSumRows>
+                    : (const void*)k_cg_resident<T, R, kResSlots, ONE, CHEB, kSumRows>;
 }
 
 template <typename T>
@@ -442,7 +527,8 @@ bool launch_cg_resident(hipStream_t s, const ResidentPlan& P, int n, RBMat<T> A,
     constexpr int R = decltype(rows)::value;
     constexpr bool ONE = decltype(one)::value;
     if (P.rows == R && P.one == ONE)
-      f = cheb.order > 0 ? resident_kernel<T, R, ONE, true>(P.pairs) : resident_kernel<T, R, ONE, false>(P.pairs);
+      f = cheb.order > 0 ? resident_kernel<T, R, ONE, true>(P.pairs, A.wmax)
+                         : resident_kernel<T, R, ONE, false>(P.pairs, A.wmax);
   };
   pick(std::integral_constant<int, 1>{}, std::false_type{});
   pick(std::integral_constant<int, 2>{}, std::false_type{});
