@@ -472,6 +472,7 @@ class HIPMatrix
   template <typename T>
   void fillDIA(T* bv) {
     hipStream_t st = m_ctx->stream;
+    if (sizeof(T) == 4) m_sym32 = -1;
     if (m_pair)
       alien_hip::launch_rbdia2_fill<T>(st, m_n, d_ro.data(), d_cols.data(), d_vals.data(), d_bo.data(),
                                        d_doff.data(), bv);
@@ -496,6 +497,24 @@ class HIPMatrix
     alien_hip::check_launch("row-bundled fill<float>");
     settle();
   }
+  // Whether the FP32 values may be read as symmetric ones (RBMat::sym), looked up once per set of values: a pass over
+  // them and 10 us. Mixed CG with the learned factor, us an iteration without and with: 96^3 40.6 and 38.9, 128^3 72.6
+  // and 64.8, 160^3 114.7 and 105.3, 256^3 320 and 306; with Jacobi 49.7 and 41.7 at 128^3. Smaller systems, most of
+  // them solved in one launch that holds the values in registers, are not looked at.
+  void findSymmetry32() {
+    if (!m_uni || m_fused_ell || m_sym32 >= 0) return;
+    m_sym32 = 0;
+    if (m_uni != 7 || m_n < kSymMinRows) return;
+    for (int j = 0; j <= 3; ++j)
+      if (m_uoff[j] != -m_uoff[6 - j]) return;
+    const int s = m_ctx->take_slot();
+    ALIEN_HIP_CHECK(hipMemsetAsync(m_ctx->dslot(s), 0, sizeof(int), m_ctx->stream));
+    alien_hip::launch_uniform_symmetric(m_ctx->stream, m_n, m_uoff, d_bv32.data(), reinterpret_cast<int*>(m_ctx->dslot(s)));
+    alien_hip::check_launch("uniform_symmetric");
+    int bad = 1;
+    m_ctx->read_words(m_ctx->dslot(s), &bad, 1);
+    m_sym32 = bad ? 0 : 1;
+  }
   bool isRBDIA() const { return m_rbdia && !m_fused_ell; }
   bool isPairDIA() const { return m_rbdia && m_pair && !m_fused_ell; }
   // FP64 operand: the uniform structure read as an ordinary RB-DIA (its masks skip the padded
@@ -514,6 +533,7 @@ class HIPMatrix
     alien_hip::RBMat<float> a{d_bo.data(), m_rbdia ? nullptr : d_bc.data(), d_bv32.data(),
                               m_rbdia ? d_doff.data() : nullptr, m_rbdia ? d_dmask.data() : nullptr, m_pair ? 1 : 0};
     setUniform(a);
+    a.sym = m_sym32 == 1;
     setWidth(a);
     return a;
   }
@@ -629,6 +649,8 @@ class HIPMatrix
   bool m_rbdia = false;
   int m_uni = 0;     // uniform RB-DIA: slots per bundle (0: not uniform)
   int m_uoff[8] = {}; // and their column offsets
+  int m_sym32 = -1;   // the uniform FP32 values are symmetric (-1: not looked up)
+  static constexpr int kSymMinRows = 1 << 19;
   bool m_pair = false; // RB-DIA in pair mode
   bool m_fused_ell = false; // the fused solvers read the BEllPack arrays
   int m_n = 0, m_nnz = 0;

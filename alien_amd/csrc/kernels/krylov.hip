@@ -202,7 +202,15 @@ __global__ void __launch_bounds__(kRowBlock) k_cg_q(int n, RBMat<T> A, const T* 
         const int row0 = b0 * kBundle + (threadIdx.x & (kWave - 1)), row1 = row0 + kBundle;
         const T p0 = p[min(row0, n - 1)], p1 = p[min(row1, n - 1)];
         T t0, t1;
-        uni_sum2<T>(A, b0, b1, [&](int c) { return p[c]; }, t0, t1);
+        bool done = false;
+        if constexpr (sizeof(T) == 4) {
+          if (A.sym && A.uni == 7) {
+            if (A.uoff[4] == 1) uni_sum2_sym_k<7, true>(A, b0, b1, p0, p1, [&](int c) { return p[c]; }, t0, t1);
+            else uni_sum2_sym_k<7, false>(A, b0, b1, p0, p1, [&](int c) { return p[c]; }, t0, t1);
+            done = true;
+          }
+        }
+        if (!done) uni_sum2<T>(A, b0, b1, [&](int c) { return p[c]; }, t0, t1);
         if (row0 < n) {
           q[row0] = t0;
           s += (double)p0 * (double)t0;

@@ -37,6 +37,9 @@ struct RBMat {
   int uni = 0;
   int nrows = 0;
   int uoff[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  // uniform of an odd number of slots at offsets -o .. 0 .. o: the values are known to be symmetric, a(r, r - o) ==
+  // a(r - o, r) bit for bit, so that a kernel may read the entries below the diagonal at their mirror's place
+  int sym = 0;
   int wmax = 1 << 30; // row-bundled: at least the widest bundle's slots
 };
 constexpr int kUniMaxSlots = 8;

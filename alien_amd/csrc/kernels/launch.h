@@ -73,6 +73,9 @@ void launch_rbdia_struct(hipStream_t, int n, const int* ro, const int* cols, con
 // (host array, the union of the matrix's diagonals), lane masks as in RB-DIA
 void launch_rbdia_uniform_struct(hipStream_t, int n, const int* ro, const int* cols, int k, const int* off, int* bo,
                                  int* doff, unsigned long long* dmask);
+// *bad (0 on entry) is raised unless the values of a uniform RB-DIA of 7 slots at offsets -o .. 0 .. o are symmetric,
+// bit for bit (RBMat::sym)
+void launch_uniform_symmetric(hipStream_t, int n, const int* off, const float* bv, int* bad);
 // values of the pair mode (two planes per slot)
 template <typename T>
 void launch_rbdia2_fill(hipStream_t, int n, const int* ro, const int* cols, const double* vals, const int* bo,

@@ -252,6 +252,71 @@ __device__ __forceinline__ void uni_sum2_k(const RBMat<T, V>& A, int b0, int b1,
   t0 = a0;
   t1 = a1;
 }
+// The value of the lane before (after) this one, `edge` on the wavefront's first (last) lane.
+__device__ __forceinline__ float lane_before(float v, float edge) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(edge), __float_as_int(v), 0x138, 0xf, 0xf, false));
+}
+__device__ __forceinline__ float lane_after(float v, float edge) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(edge), __float_as_int(v), 0x130, 0xf, 0xf, false));
+}
+__device__ __forceinline__ float of_lane(float v, int lane) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+
+// The same for symmetric values (RBMat::sym): the K / 2 entries below the diagonal are read where their
+// mirrors are stored, row - o of slot +o, which the waves before have brought into this XCD's L2: K / 2 + 1
+// values a row come from memory, not K. With the neighbours at -1 and +1 the lanes pass each other their
+// vector elements and that mirror (NEAR). own0, own1: the vector at this lane's two rows. b1 is b0 + 1, or b0 past the
+// end. q = A p at 256^3: 81 us (83 without the lanes' exchange) against 99, 24 bytes a row from memory and not 36. Its
+// loads are unconditional: behind branches for the wave's ends it took 98.
+template <int K, bool NEAR, typename XS>
+__device__ __forceinline__ void uni_sum2_sym_k(const RBMat<float>& A, int b0, int b1, float own0, float own1, XS xs,
+                                               float& t0, float& t1) {
+  constexpr int H = K / 2;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int r0 = b0 * kWave + lane, r1 = b1 * kWave + lane, last = A.nrows - 1;
+  auto at = [&](int row, int u) { return A.bv[((row & ~(kWave - 1)) * K + u * kWave) + (row & (kWave - 1))]; };
+  float v0[K], v1[K], x0[K], x1[K];
+  float xe = 0.f, ve = 0.f; // on the first lane what lies before the wave's rows, on the last what lies after
+  if constexpr (NEAR) {
+    const int before = lane ? r0 : max(r0 - 1, 0);
+    xe = xs(min(lane == kWave - 1 ? r1 + 1 : before, last)); // (rows past the last: any element)
+    ve = at(before, H + 1);
+    ve = r0 > 0 ? ve : 0.f;
+  }
+#pragma unroll
+  for (int u = K - 1; u >= 0; --u) {
+    if (NEAR && u == H - 1) continue;
+    const int o = u < H ? A.uoff[u] : 0, s = u < H ? K - 1 - u : u;
+    const float a0 = at(max(r0 + o, 0), s), a1 = at(max(r1 + o, 0), s);
+    v0[u] = r0 + o >= 0 ? a0 : 0.f;
+    v1[u] = r1 + o >= 0 ? a1 : 0.f;
+  }
+#pragma unroll
+  for (int u = 0; u < K; ++u) {
+    if (u == H || (NEAR && (u == H - 1 || u == H + 1))) continue;
+    x0[u] = xs(min(max(r0 + A.uoff[u], 0), last));
+    x1[u] = xs(min(max(r1 + A.uoff[u], 0), last));
+  }
+  x0[H] = own0;
+  x1[H] = own1;
+  if constexpr (NEAR) {
+    v0[H - 1] = lane_before(v0[H + 1], ve);
+    v1[H - 1] = lane_before(v1[H + 1], of_lane(v0[H + 1], kWave - 1));
+    x0[H - 1] = lane_before(own0, xe);
+    x1[H - 1] = lane_before(own1, of_lane(own0, kWave - 1));
+    x0[H + 1] = lane_after(own0, of_lane(own1, 0));
+    x1[H + 1] = lane_after(own1, xe);
+  }
+  float a0 = 0.f, a1 = 0.f;
+#pragma unroll
+  for (int u = 0; u < K; ++u) {
+    a0 = a0 + v0[u] * x0[u];
+    a1 = a1 + v1[u] * x1[u];
+  }
+  t0 = a0;
+  t1 = a1;
+}
 template <typename T, typename V, typename XS>
 __device__ __forceinline__ void uni_sum2(const RBMat<T, V>& A, int b0, int b1, XS xs, T& t0, T& t1) {
   switch (A.uni) {

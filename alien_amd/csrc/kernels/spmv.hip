@@ -751,6 +751,27 @@ __global__ void __launch_bounds__(kBlock) k_rbdia_uniform_struct(int n, const in
     if (b == nb - 1) bo[nb] = nb * U.k;
   }
 }
+__global__ void __launch_bounds__(kBlock) k_uniform_symmetric(int n, UniOffsets U, const unsigned* __restrict__ bv,
+                                                               int* bad) {
+  const int r = blockIdx.x * kBlock + threadIdx.x;
+  if (r >= n) return;
+  constexpr int K = 7;
+  auto at = [&](int row, int u) { return bv[((long)(row & ~(kWave - 1)) * K + u * kWave) + (row & (kWave - 1))]; };
+  bool same = true;
+#pragma unroll
+  for (int u = 0; u < K / 2; ++u) {
+    const int m = r + U.off[u];
+    same = same && at(r, u) == (m >= 0 ? at(m, K - 1 - u) : 0u);
+  }
+  if (!same) *bad = 1;
+}
+void launch_uniform_symmetric(hipStream_t st, int n, const int* off, const float* bv, int* bad) {
+  UniOffsets U{};
+  U.k = 7;
+  for (int j = 0; j < U.k; ++j) U.off[j] = off[j];
+  hipLaunchKernelGGL(k_uniform_symmetric, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, st, n, U,
+                     reinterpret_cast<const unsigned*>(bv), bad);
+}
 void launch_rbdia_uniform_struct(hipStream_t st, int n, const int* ro, const int* cols, int k, const int* off,
                                  int* bo, int* doff, unsigned long long* dmask) {
   if (n <= 0) return;

@@ -1580,6 +1580,7 @@ void solve_on(alien_hip_ctx* ctx, const alien_hip_solve_params* p, HIPMatrix& A,
     } else {
       // FP32 matrix, preconditioner and Krylov vectors, FP64 dots; FP64 defect correction
       A.ensureRB32();
+      if (!bicg) A.findSymmetry32();
       phase("FP32 matrix");
       DeviceArray<float> invd32(n);
       launch_demote(ctx->stream, n, invd64, invd32.data());
