@@ -47,6 +47,8 @@ BESIDE = ("k_factor_t<float, float, 2>", "k_factor_p<float, float, 2>", "k_cg_up
 # workgroups of the step kernel on a 7-slot uniform RB-DIA at 256^3 (the library's default cap for
 # uniform operators of 6 or more slots): one FP64 partial each
 UNI_WIDE_GRID = 32768
+# rows from which the mixed CG reads a symmetric uniform operator's lower entries at their mirrors
+SYMMETRIC_ROWS = 1 << 19
 # the CSR-family kernel whose bytes are the CSR formula's (RB-CSR stores every CSR column)
 CSR_ROOF, CSR_ROOF_KERNEL = "rbcsr_fp64", "k_spmv_rbcsr<double>"
 PROFILES = os.path.join(ROOT, "profiles")
@@ -105,6 +107,12 @@ def udia_bytes(n, nnz, word):
     """Uniform RB-DIA: the values of the stored entries, x once, y (no descriptors are read; the
     zero padding of absent entries, 0.2% at 256^3, is not credited)."""
     return word * nnz + 2 * word * n
+
+
+def symmetric_udia_bytes(n, nnz, word):
+    """Uniform RB-DIA whose values are symmetric (they are looked at once per solve from SYMMETRIC_ROWS rows on): the
+    diagonal and the entries above it, x once, y."""
+    return word * (nnz + n) // 2 + 2 * word * n
 
 
 def bellpack_bytes(n, nnz, nslices, word):
@@ -1012,13 +1020,16 @@ def main():
     # launch) is reported beside it
     if step_timing and step_timing["launches"] > 0:
         roof_us = step_timing["us_total"] / step_timing["launches"]
+        roof_bytes = spmv[ROOF]["bytes"]
+        if N >= SYMMETRIC_ROWS:  # (the loop of time_spmv runs the general form on the same arrays)
+            roof_bytes = symmetric_udia_bytes(N, nnz, 4) + 8 * UNI_WIDE_GRID
         roof_how = (f"HIP events around each of its {step_timing['launches']} launches inside one extra "
                     f"learned + mixed solve (on the solve stream; that solve launches its iterations directly, not "
                     f"from the captured graph)")
     else:
-        roof_us = spmv[ROOF]["us"]
+        roof_us, roof_bytes = spmv[ROOF]["us"], spmv[ROOF]["bytes"]
         roof_how = "back-to-back launches with its one-workgroup finalize (no learned + mixed solve in this run)"
-    roof_gbs = spmv[ROOF]["bytes"] / roof_us / 1e3
+    roof_gbs = roof_bytes / roof_us / 1e3
     roof_frac = roof_gbs / HBM_PEAK_GBS
     if roof_frac > 1.0:
         raise RuntimeError(f"{ROOF_KERNEL}: {roof_gbs:.0f} GB/s exceeds the HBM peak: bytes or time wrong")
@@ -1048,7 +1059,7 @@ def main():
         "spmv": spmv,
         "roofline": {"bound": "hbm", "achieved": roof_gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": roof_frac, "traffic": profile_traffic(ROOF_KERNEL) if n == 256 else None,
-                     "kernel": ROOF_KERNEL, "bytes_per_launch": spmv[ROOF]["bytes"],
+                     "kernel": ROOF_KERNEL, "bytes_per_launch": roof_bytes,
                      "us_per_launch": roof_us, "measured": roof_how,
                      "us_back_to_back": spmv[ROOF]["us"], "achieved_back_to_back": spmv[ROOF]["gbs"],
                      "us_in_solve_profile": profile_avg_us(ROOF_KERNEL),

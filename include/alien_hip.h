@@ -41,7 +41,7 @@ const char* alien_hip_last_error(void);
 const char* alien_hip_version(void);
 
 /* Context = one HIP stream (NULL = create a private one) plus the workspace
- * used by the reductions. Replaces SYCLInternal::KernelInternal, the queue
+ * used by the reductions and the ILU(0) entry points. Replaces SYCLInternal::KernelInternal, the queue
  * holder of SYCLInternalLinearAlgebra (sycl/algebra/SYCLInternalLinearAlgebra.h:137). */
 int alien_hip_ctx_create(void* stream, alien_hip_ctx** out);
 int alien_hip_ctx_destroy(alien_hip_ctx* ctx);
@@ -323,7 +323,9 @@ int alien_hip_spmv_dot_csr_f64_noalloc(void* stream, int nrows, const int* row_o
  * levels in order: bit-exact with LUFactorisationAlgo::factorize, sequential
  * branch (ILU0Preconditioner.h:71-179, 156-178). level_rows lists the rows of
  * level l in level_ptr[l]..level_ptr[l+1] (built on the host from
- * alien_hip_host_levels with upper = 0). */
+ * alien_hip_host_levels with upper = 0). One launch for all levels, rows waiting for
+ * the rows they read, with a workspace of the context (8 bytes per row, kept); one launch per
+ * level inside a stream capture when that workspace is not there yet. */
 int alien_hip_ilu0_factor_f64(alien_hip_ctx* ctx, int nrows, const int* row_offset, const int* cols,
                               const int* dcol, double* lu, int nlevels, const int* level_ptr_host,
                               const int* level_rows);
@@ -333,7 +335,8 @@ int alien_hip_ilu0_factor_f64(alien_hip_ctx* ctx, int nrows, const int* row_offs
 int alien_hip_filu0_sweep_f64(alien_hip_ctx* ctx, int nrows, const int* row_offset, const int* cols,
                               const int* dcol, const double* vals, const double* prev, double* lu);
 /* L x1 = y then U x = x1 (solveL/solveU, ILU0Preconditioner.h:181-231), level by
- * level; t is an n-vector of workspace. lower/upper schedules as above. */
+ * level; t is an n-vector of workspace. lower/upper schedules as above. One launch per
+ * sweep, as the factorisation's; one per level where t overlaps y or x. */
 int alien_hip_ilu0_solve_f64(alien_hip_ctx* ctx, int nrows, const int* row_offset, const int* cols,
                              const int* dcol, const double* lu, int nlev_l, const int* lptr_host,
                              const int* lrows, int nlev_u, const int* uptr_host, const int* urows,
