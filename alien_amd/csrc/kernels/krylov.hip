@@ -184,8 +184,10 @@ __global__ void __launch_bounds__(kBlock) k_cg_p(int n, const T* __restrict__ z,
 }
 
 // q = A p ; pq = p . q (a zero pq raises the breakdown flag in the finalize)
+// Row-bundled: 7 wavefronts a SIMD (72 registers in FP64; 74 had let 6 run). A Jacobi-CG iteration in FP64 32.9 -> 31.9 us
+// at 82^3, 70.8 -> 69.8 at 128^3, 503 -> 499 at 256^3; eight spill (25 us instead of 13 at 80^3).
 template <typename T, int LAY = kRowBundled>
-__global__ void __launch_bounds__(kRowBlock) k_cg_q(int n, RBMat<T> A, const T* __restrict__ p, T* __restrict__ q,
+__global__ void __launch_bounds__(kRowBlock, LAY == kRowBundled ? 7 : 1) k_cg_q(int n, RBMat<T> A, const T* __restrict__ p, T* __restrict__ q,
                                                      CGState* st, RedWork w) {
   if (st->done) return;
   __shared__ double lds4[kRowBlock / kWave];
