@@ -172,9 +172,15 @@ struct alien_hip_ctx {
   alien_hip::DeviceArray<double> scalars; // device-resident scalar slots
   // zeroed CG state (done = 0, never written): the fused iteration's kernels launched on their own
   alien_hip::DeviceArray<alien_hip::CGState> idle_cg;
-  // slots and head of the grid-wide sums of the resident CG (cg_resident.hip), zeroed on first use
+  // slots and head of the grid-wide sums of the resident CG (cg_resident.hip), zeros at first
   alien_hip::DeviceArray<unsigned long long> grid_slots;
   alien_hip::DeviceArray<int> grid_head;
+  // Zeros again, on the stream: after a launch that gave up, whose words are tagged with phases past the head's, which
+  // the next launch would take for its own.
+  void clear_grid() {
+    ALIEN_HIP_CHECK(hipMemsetAsync(grid_slots.data(), 0, sizeof(unsigned long long) * grid_slots.size(), stream));
+    ALIEN_HIP_CHECK(hipMemsetAsync(grid_head.data(), 0, sizeof(int) * grid_head.size(), stream));
+  }
   // pivots (one per row) and ticket, flag of the ILU(0) kernels of ilu0_sync.hip
   alien_hip::DeviceArray<double> ilu_piv;
   alien_hip::DeviceArray<int> ilu_work;

@@ -42,8 +42,7 @@ alien_hip_ctx* make_ctx(void* stream) {
     ALIEN_HIP_CHECK(hipMemsetAsync(c->idle_cg.data(), 0, sizeof(CGState), c->stream));
     c->grid_slots.resize(kResidentWords);
     c->grid_head.resize(2);
-    ALIEN_HIP_CHECK(hipMemsetAsync(c->grid_slots.data(), 0, sizeof(unsigned long long) * kResidentWords, c->stream));
-    ALIEN_HIP_CHECK(hipMemsetAsync(c->grid_head.data(), 0, 2 * sizeof(int), c->stream));
+    c->clear_grid();
     ALIEN_HIP_CHECK(hipGetDevice(&c->device));
     ALIEN_HIP_CHECK(hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, c->device));
     c->tickets.resize(kTicketWords);

@@ -410,7 +410,7 @@ struct FusedCG {
     if (!cur.done && cur.it == before.it) {
       lost = true;
       resident = false;
-      ALIEN_HIP_CHECK(hipMemsetAsync(ctx->grid_head.data() + 1, 0, sizeof(int), ctx->stream));
+      ctx->clear_grid();
     }
     return cur;
   }

@@ -1,0 +1,134 @@
+// What calls leave in the state of a context: calls that end off the straight path (a wait given up, a stream
+// capture, a second context), followed by ordinary ones on the same context. Prints one JSON object per check on stdout
+// for tests/test_gpu_ctx_state.py. The internal headers give the checks the context's own fields.
+// Usage: ctx_state_check [check ...]  (all of them without an argument)
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <functional>
+#include <map>
+#include <random>
+#include <string>
+#include <vector>
+
+#include "alien/hip/HIPBackEnd.h"
+
+namespace {
+
+struct System {
+  int n = 0;
+  std::vector<int> ro, cols;
+  std::vector<double> vals, b;
+};
+
+// 7-point system, its right-hand side the product with U[0,1) values of `seed`
+System generate(int kind, int nx, int ny, int nz, unsigned seed) {
+  System a;
+  const long nnz = alien_hip_gen_nnz(kind, nx, ny, nz);
+  a.n = nx * ny * nz;
+  a.ro.resize(a.n + 1);
+  a.cols.resize(nnz);
+  a.vals.resize(nnz);
+  const double lognormal[4] = {1, 1, 1, 1};
+  if (alien_hip_gen_csr(kind, nx, ny, nz, kind == ALIEN_HIP_GEN_LOGNORMAL7 ? lognormal : nullptr, seed, a.ro.data(),
+                        a.cols.data(), a.vals.data()) != 0) {
+    std::fprintf(stderr, "gen_csr: %s\n", alien_hip_last_error());
+    std::exit(2);
+  }
+  std::vector<double> x(a.n);
+  alien_hip_fill_uniform01(seed, a.n, x.data());
+  a.b.assign(a.n, 0);
+  for (int i = 0; i < a.n; ++i)
+    for (int k = a.ro[i]; k < a.ro[i + 1]; ++k) a.b[i] += a.vals[k] * x[a.cols[k]];
+  return a;
+}
+
+void call(int rc, const char* what) {
+  if (rc == 0) return;
+  std::fprintf(stderr, "%s: %s\n", what, alien_hip_last_error());
+  std::exit(3);
+}
+
+struct Context {
+  alien_hip_ctx* c = nullptr;
+  Context() { call(alien_hip_ctx_create(nullptr, &c), "ctx_create"); }
+  ~Context() { alien_hip_ctx_destroy(c); }
+  alien_hip_ctx* operator->() const { return c; }
+};
+
+struct Solved {
+  std::vector<double> x;
+  alien_hip_solve_result r{};
+  bool operator==(const Solved& o) const {
+    return r.iterations == o.r.iterations && r.status == o.r.status && r.error == o.r.error &&
+           std::memcmp(x.data(), o.x.data(), sizeof(double) * x.size()) == 0;
+  }
+};
+
+alien_hip_solve_params params(int precond, int mode, double tol) {
+  alien_hip_solve_params p{};
+  p.solver = ALIEN_HIP_CG;
+  p.precond = precond;
+  p.layout = ALIEN_HIP_LAYOUT_RBDIA;
+  p.mode = mode;
+  p.tol = tol;
+  p.max_iter = 2000;
+  p.poll_every = 8;
+  return p;
+}
+
+Solved solve(const Context& c, const System& a, int mode, double tol = 1e-10, int precond = ALIEN_HIP_PREC_DIAG) {
+  Solved s;
+  s.x.assign(a.n, 0.0);
+  const alien_hip_solve_params p = params(precond, mode, tol);
+  call(alien_hip_solve_csr(c.c, &p, a.n, a.ro.data(), a.cols.data(), a.vals.data(), a.b.data(), s.x.data(), &s.r),
+       "solve_csr");
+  return s;
+}
+
+template <typename T>
+std::vector<T> read(const alien_hip::DeviceArray<T>& d) {
+  std::vector<T> h(d.size());
+  ALIEN_HIP_CHECK(hipDeviceSynchronize());
+  ALIEN_HIP_CHECK(hipMemcpy(h.data(), d.data(), sizeof(T) * h.size(), hipMemcpyDeviceToHost));
+  return h;
+}
+
+// After waits given up, the words of the grid-wide sums hold no phase that a later launch will reach, and solves of other
+// systems with the usual number of polls are those of a context that runs no resident launch.
+void after_a_wait_given_up() {
+  const System first = generate(ALIEN_HIP_GEN_LOGNORMAL7, 40, 41, 43, 1);
+  const System second = generate(ALIEN_HIP_GEN_LOGNORMAL7, 44, 37, 45, 2);
+  Context launches, c;
+  launches->cg_resident = false;
+  const long usual = c->resident_spins;
+  int newer = 0, gave_up = 1, same = 1;
+  for (int mode : {ALIEN_HIP_MODE_GRAPH, ALIEN_HIP_MODE_MIXED}) {
+    c->resident_spins = 0;
+    gave_up &= solve(c, first, mode).r.status;
+    const unsigned head = (unsigned)read(c->grid_head)[0];
+    for (unsigned long long w : read(c->grid_slots)) newer += (unsigned)(w >> 32) > head;
+    c->resident_spins = usual;
+    same &= solve(c, second, mode) == solve(launches, second, mode);
+  }
+  std::printf("{\"check\": \"after_a_wait_given_up\", \"status\": %d, \"newer_words\": %d, \"same\": %d}\n", gave_up, newer,
+              same);
+}
+
+const std::map<std::string, std::function<void()>> kChecks = {
+    {"after_a_wait_given_up", after_a_wait_given_up},
+};
+
+} // namespace
+
+int main(int argc, char** argv) {
+  for (const auto& c : kChecks) {
+    bool on = argc == 1;
+    for (int k = 1; k < argc; ++k) on = on || c.first == argv[k];
+    if (!on) continue;
+    std::fprintf(stderr, "check %s\n", c.first.c_str());
+    c.second();
+    std::fflush(stdout);
+  }
+  return 0;
+}

@@ -1,0 +1,27 @@
+"""What calls leave in the state of a context (tests/cxx/ctx_state_check.cpp): each call off the straight path is followed
+by ordinary ones on the same context, whose results are compared bit for bit with those of an untouched one."""
+import json
+import pathlib
+import subprocess
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+CXX = pathlib.Path(__file__).resolve().parent / "cxx"
+
+
+def run(check):
+    exe = CXX / "ctx_state_check"
+    if not exe.exists():
+        subprocess.run(["make", "-s", "-C", str(CXX)], check=True)
+    print("case", check, flush=True)
+    p = subprocess.run([str(exe), check], capture_output=True, text=True, timeout=100)
+    assert p.returncode == 0, p.stderr[-2000:]
+    (out,) = [json.loads(s) for s in p.stdout.splitlines()]
+    assert out.pop("check") == check
+    return out
+
+
+def test_after_a_wait_given_up():
+    assert run("after_a_wait_given_up") == {"status": 1, "newer_words": 0, "same": 1}
