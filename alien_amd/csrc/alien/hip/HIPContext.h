@@ -285,11 +285,12 @@ struct alien_hip_ctx {
     fetch(mail + 2 * s, tag, dslot(s), &v, 2);
     return v;
   }
-  // n 32-bit words (at most kMaxPostWords) of device memory, likewise.
-  void read_words(const void* from, void* to, int n) {
+  // n 32-bit words of device memory, likewise, and one from `also` (at most kMaxPostWords together).
+  void read_words(const void* from, void* to, int n, const int* also = nullptr, int* also_to = nullptr) {
     const alien_hip::HostPost p{mail + 2 * kSlots, new_tag()};
-    alien_hip::launch_post_words(stream, from, n, p);
+    alien_hip::launch_post_words(stream, from, n, p, also);
     fetch(p.to, p.tag, from, to, n);
+    if (also) fetch(p.to + n, p.tag, also, also_to, 1);
   }
 
  private:

@@ -173,8 +173,8 @@ struct ResidentPlan {
 template <typename T>
 bool resident_plan(int n, const RBMat<T>& A, int cus, int cheb_order, ResidentPlan& P);
 // ex: P.exchange vectors of n entries; slots: kResidentWords words and head: two ints, 0 before the
-// first launch and again before the next one after a wait that ran out of polls, when head[1] is set: x, r, z and p may
-// then be a mixture, the state is the one before. spins: polls of a wait. false: not launched.
+// first launch and again before the next one after a wait that ran out of polls, when head[1] is set: rows of x, r, z and
+// p, and the state, may then each be those before the launch or after it. spins: polls of a wait. false: not launched.
 template <typename T>
 bool launch_cg_resident(hipStream_t, const ResidentPlan& P, int n, RBMat<T> A, const T* invd, T* x, T* r, T* z, T* p,
                         T* ex, CGState* st, unsigned long long* slots, int* head, const ResidentCheb& cheb, int iters,

@@ -21,9 +21,9 @@ enum FinOp { kFinStore = 0, kFinRho1 = 1, kFinPQ = 2, kFinXR = 3, kFinXRDiag = 4
 void launch_finalize(hipStream_t, RedWork w, long nblk, int nslot, int op, double* out, CGState* st);
 // one stored total, handed to the host as well
 void launch_finalize_post(hipStream_t, RedWork w, long nblk, double* out, HostPost post);
-// n (at most kMaxPostWords) 32-bit words of device memory to the host
+// n 32-bit words of device memory to the host, and one from `also` behind them (at most kMaxPostWords together)
 constexpr int kMaxPostWords = 64;
-void launch_post_words(hipStream_t, const void* from, int n, HostPost post);
+void launch_post_words(hipStream_t, const void* from, int n, HostPost post, const void* also = nullptr);
 // the same second stage for the BiCGStab state (reduce.hip)
 enum BFinOp { kBFinAlpha = 0, kBFinS = 1, kBFinOmega = 2, kBFinXR = 3 };
 void launch_finalize_bicg(hipStream_t, RedWork w, long nblk, int nslot, int op, BiCGState* st);

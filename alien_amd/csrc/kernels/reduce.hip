@@ -166,15 +166,18 @@ __global__ void __launch_bounds__(kFin) k_finalize_post(RedWork w, int nblk, dou
   out[0] = tot[0];
 }
 // One wavefront: the host polls for the words where a copy and a wait for the stream took it 13 us.
-__global__ void __launch_bounds__(kMaxPostWords) k_post_words(const unsigned* from, int n, HostPost post) {
+__global__ void __launch_bounds__(kMaxPostWords) k_post_words(const unsigned* from, int n, const unsigned* also,
+                                                               HostPost post) {
   if ((int)threadIdx.x < n) post_word(post, threadIdx.x, from[threadIdx.x]);
+  else if ((int)threadIdx.x == n && also) post_word(post, n, *also);
 }
 
 void launch_finalize_post(hipStream_t s, RedWork w, long nblk, double* out, HostPost post) {
   hipLaunchKernelGGL(k_finalize_post, dim3(1), dim3(kFin), 0, s, w, (int)nblk, out, post);
 }
-void launch_post_words(hipStream_t s, const void* from, int n, HostPost post) {
-  hipLaunchKernelGGL(k_post_words, dim3(1), dim3(kMaxPostWords), 0, s, static_cast<const unsigned*>(from), n, post);
+void launch_post_words(hipStream_t s, const void* from, int n, HostPost post, const void* also) {
+  hipLaunchKernelGGL(k_post_words, dim3(1), dim3(kMaxPostWords), 0, s, static_cast<const unsigned*>(from), n,
+                     static_cast<const unsigned*>(also), post);
 }
 void launch_finalize_bicg(hipStream_t s, RedWork w, long nblk, int nslot, int op, BiCGState* st) {
   hipLaunchKernelGGL(k_finalize_bicg, dim3(1), dim3(kFin), 0, s, w, (int)nblk, nslot, op, st);

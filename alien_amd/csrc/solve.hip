@@ -394,9 +394,11 @@ struct FusedCG {
   ResidentPlan res;
   ResidentCheb res_cheb;
   DeviceArray<T> ex;
-  bool lost = false; // a resident launch gave up: x is valid, the recurrence is not (see restart)
+  bool lost = false; // a resident launch gave up: x is any iterate, the recurrence is not valid (see restart)
   // iterations until the device stop flag is raised, or to a multiple of `check` iterations with r.r
-  // below `below`; then the state
+  // below `below`; then the state. A workgroup that gave up has stored nothing, others may have gone on and stored their
+  // rows, the one that stores the state among them: whatever the state says, the launch is lost when the flag is up, and
+  // the count stays where it was (r.r is the launch's, not finite where x may not be).
   CGState advance_resident(T* x, int check, double below) {
     const CGState before = *h_st;
     const std::lock_guard<std::mutex> alone(resident_mutex(ctx->device));
@@ -406,13 +408,16 @@ struct FusedCG {
       resident = false;
       return before;
     }
-    const CGState cur = read_state();
-    if (!cur.done && cur.it == before.it) {
-      lost = true;
-      resident = false;
-      ctx->clear_grid();
-    }
-    return cur;
+    int gave_up = 0;
+    static_assert(sizeof(CGState) + 4 <= 4 * kMaxPostWords, "one post");
+    ctx->read_words(st.data(), h_st, (int)(sizeof(CGState) / 4), ctx->grid_head.data() + 1, &gave_up);
+    if (!gave_up) return *h_st;
+    lost = true;
+    resident = false;
+    ctx->clear_grid();
+    CGState out = before;
+    out.rr = h_st->rr;
+    return out;
   }
   // one launch at most runs this many iterations (tens of milliseconds)
   static constexpr int kResidentIters = 4096;
@@ -753,7 +758,7 @@ MixedResult mixed_reliable_cg(alien_hip_ctx* ctx, int n, RBMat<double> A64, RBMa
   watch.stalled(rr64, 0);
   auto advance = [&]() {
     CGState c = F.advance(x32.data(), graph, k, d2 * rr_last);
-    if (!F.lost) return c;
+    if (!F.lost || !std::isfinite(c.rr)) return c;
     // the increment is kept, its recurrence begun again from the true residual
     launch_fold_increment(s, n, x32.data(), x);
     launch_residual<double>(s, ctx->red(), n, A64, x, b, r64.data(), ctx->dslot(rslot));

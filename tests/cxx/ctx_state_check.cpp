@@ -115,8 +115,28 @@ void after_a_wait_given_up() {
               same);
 }
 
+// With the flag of a wait given up raised, whatever the launch's own state says: the solve goes on from the true residual
+// and the flag is down again.
+void flag_is_read() {
+  const System a = generate(ALIEN_HIP_GEN_LOGNORMAL7, 40, 41, 43, 3);
+  const double tol = 1e-10;
+  Context c;
+  int up = 0, status = 1;
+  double worst = 0;
+  for (int mode : {ALIEN_HIP_MODE_GRAPH, ALIEN_HIP_MODE_MIXED}) {
+    const int one = 1;
+    ALIEN_HIP_CHECK(hipMemcpy(c->grid_head.data() + 1, &one, sizeof(int), hipMemcpyHostToDevice));
+    const Solved s = solve(c, a, mode, tol);
+    status &= s.r.status;
+    worst = std::max(worst, s.r.true_rel_res / tol);
+    up += read(c->grid_head)[1];
+  }
+  std::printf("{\"check\": \"flag_is_read\", \"status\": %d, \"up\": %d, \"residual\": %.17g}\n", status, up, worst);
+}
+
 const std::map<std::string, std::function<void()>> kChecks = {
     {"after_a_wait_given_up", after_a_wait_given_up},
+    {"flag_is_read", flag_is_read},
 };
 
 } // namespace

@@ -25,3 +25,11 @@ def run(check):
 
 def test_after_a_wait_given_up():
     assert run("after_a_wait_given_up") == {"status": 1, "newer_words": 0, "same": 1}
+
+
+def test_flag_is_read():
+    """A resident launch is taken back by its flag, not by its count. The residual that the solve stopped on is updated, not
+    recomputed: a true one of up to 1.05 times the tolerance, as in the tests of the solvers."""
+    out = run("flag_is_read")
+    assert out.pop("residual") <= 1.05
+    assert out == {"status": 1, "up": 0}
