@@ -184,16 +184,20 @@ struct alien_hip_ctx {
   // pivots (one per row) and ticket, flag of the ILU(0) kernels of ilu0_sync.hip
   alien_hip::DeviceArray<double> ilu_piv;
   alien_hip::DeviceArray<int> ilu_work;
-  // room for them; false where that would take an allocation inside a stream capture
+  // Room for them; false inside a stream capture: a graph would hold pointers that a larger system's call frees, and its
+  // replays beside the context's own work would share ticket, flag and pivots with it.
   bool reserve_ilu(size_t rows) {
+    if (capturing()) return false;
     if (ilu_work.size() == 2 && ilu_piv.size() >= rows) return true;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    ALIEN_HIP_CHECK(hipStreamIsCapturing(stream, &cap));
-    if (cap != hipStreamCaptureStatusNone) return false;
     ALIEN_HIP_CHECK(hipStreamSynchronize(stream));
     if (ilu_work.size() != 2) ilu_work.resize(2);
     if (ilu_piv.size() < rows) ilu_piv.resize(rows);
     return true;
+  }
+  bool capturing() const {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    ALIEN_HIP_CHECK(hipStreamIsCapturing(stream, &cap));
+    return cap != hipStreamCaptureStatusNone;
   }
   int device = 0, cus = 0; // the context's device and its compute units
   // resident CG (cg_resident.hip): on / off (ALIEN_HIP_CG_RESIDENT at creation), polls of a wait
@@ -258,9 +262,7 @@ struct alien_hip_ctx {
   // replayed beside the context's own work would leave the counters wrong for good, not for one result.
   alien_hip::RedWork red_once() {
     alien_hip::RedWork w = red();
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    ALIEN_HIP_CHECK(hipStreamIsCapturing(stream, &cap));
-    if (cap == hipStreamCaptureStatusNone) w.ticket = tickets.data();
+    if (!capturing()) w.ticket = tickets.data();
     return w;
   }
   // A fresh device scalar slot (ring of kSlots; callers keep at most a few live).

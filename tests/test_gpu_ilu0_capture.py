@@ -1,0 +1,68 @@
+"""ILU(0) factorisation and sweeps through the C entry points in a captured graph: it holds the caller's arrays only, so it
+replays rightly after a larger system has gone through the context, and after the context is gone."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import alien_amd as aa
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+from gpu_util import dev, empty  # noqa: E402
+from test_gpu_ilu0_sync import CASES  # noqa: E402
+
+
+def ptr(t):
+    return ctypes.c_void_p(t.data_ptr())
+
+
+def system(case):
+    """(run(context), lu, x): factorisation of the case's matrix and one solve, on arrays of their own."""
+    ro, cols, vals = CASES[case]()
+    n = len(ro) - 1
+    dcol = aa.host_dcol(ro, cols)
+    (lp, lr), (up, ur) = (aa.group_by_level(*aa.host_levels(ro, cols, dcol, u)) for u in (False, True))
+    lp, up = (np.ascontiguousarray(a, np.int32) for a in (lp, up))
+    A = [dev(ro), dev(cols), dev(dcol)]
+    v, lr, ur, y = dev(vals), dev(lr.astype(np.int32)), dev(ur.astype(np.int32)), dev(np.random.default_rng(n).random(n))
+    lu, t, x = empty(len(cols)), empty(n), empty(n)
+
+    def run(c):
+        L, a = aa.lib(), [ptr(q) for q in A]
+        aa.check(L.alien_hip_copy_f64(c.h, len(cols), ptr(v), ptr(lu)))
+        aa.check(L.alien_hip_ilu0_factor_f64(c.h, n, *a, ptr(lu), len(lp) - 1, aa._capi.iptr(lp), ptr(lr)))
+        aa.check(L.alien_hip_ilu0_solve_f64(c.h, n, *a, ptr(lu), len(lp) - 1, aa._capi.iptr(lp), ptr(lr), len(up) - 1,
+                                            aa._capi.iptr(up), ptr(ur), ptr(y), ptr(t), ptr(x)))
+
+    return run, lu, x
+
+
+def test_graph_outlives_the_workspace():
+    print("case graph of a small system, eager larger one, context closed", flush=True)
+    (small, lu, x), (large, _, xl) = system("fill"), system("wide")
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        with aa.Context(s.cuda_stream) as c:
+            small(c)
+            s.synchronize()
+            want, want_lu = x.clone(), lu.clone()
+            g = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(g, stream=s):
+                small(c)
+            large(c)
+            s.synchronize()
+            want_large = xl.clone()
+            for _ in range(3):
+                x.zero_()
+                g.replay()
+                large(c)
+                s.synchronize()
+                assert torch.equal(x, want) and torch.equal(lu, want_lu) and torch.equal(xl, want_large)
+        for _ in range(3):
+            x.zero_()
+            lu.zero_()
+            g.replay()
+            s.synchronize()
+            assert torch.equal(x, want) and torch.equal(lu, want_lu)
