@@ -181,17 +181,25 @@ struct alien_hip_ctx {
     ALIEN_HIP_CHECK(hipMemsetAsync(grid_slots.data(), 0, sizeof(unsigned long long) * grid_slots.size(), stream));
     ALIEN_HIP_CHECK(hipMemsetAsync(grid_head.data(), 0, sizeof(int) * grid_head.size(), stream));
   }
-  // pivots (one per row) and ticket, flag of the ILU(0) kernels of ilu0_sync.hip
-  alien_hip::DeviceArray<double> ilu_piv;
+  // pivots (one per row, in the last block) and ticket, flag of the ILU(0) kernels of ilu0_sync.hip
+  std::vector<alien_hip::DeviceArray<double>> ilu_piv;
   alien_hip::DeviceArray<int> ilu_work;
-  // Room for them; false inside a stream capture: a graph would hold pointers that a larger system's call frees, and its
-  // replays beside the context's own work would share ticket, flag and pivots with it.
+  // Room for them, without a wait for the stream: a block that has become too small stays (queued launches may use it)
+  // until the context goes, and each is at least twice the one before, so that all of them are at most twice the last.
+  // False without the memory for it, and inside a stream capture: a graph would outlive the workspace, and its replays
+  // beside the context's own work would share ticket, flag and pivots with it.
   bool reserve_ilu(size_t rows) {
     if (capturing()) return false;
-    if (ilu_work.size() == 2 && ilu_piv.size() >= rows) return true;
-    ALIEN_HIP_CHECK(hipStreamSynchronize(stream));
-    if (ilu_work.size() != 2) ilu_work.resize(2);
-    if (ilu_piv.size() < rows) ilu_piv.resize(rows);
+    const size_t have = ilu_piv.empty() ? 0 : ilu_piv.back().size();
+    if (have >= rows) return true;
+    try {
+      alien_hip::DeviceArray<double> more(std::max(rows, 2 * have));
+      ilu_piv.push_back(std::move(more));
+    } catch (const alien_hip::Error& e) {
+      if (e.code != (int)hipErrorOutOfMemory) throw;
+      (void)hipGetLastError();
+      return false;
+    }
     return true;
   }
   bool capturing() const {

@@ -45,6 +45,7 @@ alien_hip_ctx* make_ctx(void* stream) {
     c->clear_grid();
     ALIEN_HIP_CHECK(hipGetDevice(&c->device));
     ALIEN_HIP_CHECK(hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, c->device));
+    c->ilu_work.resize(2);
     c->tickets.resize(kTicketWords);
     ALIEN_HIP_CHECK(hipMemsetAsync(c->tickets.data(), 0, sizeof(unsigned) * kTicketWords, c->stream));
     ALIEN_HIP_CHECK(hipHostMalloc((void**)&c->mail, sizeof(unsigned long long) * alien_hip_ctx::kMailWords,
@@ -66,7 +67,7 @@ void destroy_ctx(alien_hip_ctx* c) {
   c->idle_cg.reset();
   c->grid_slots.reset();
   c->grid_head.reset();
-  c->ilu_piv.reset();
+  c->ilu_piv.clear();
   c->ilu_work.reset();
   c->tickets.reset();
   if (c->mail) (void)hipHostFree(c->mail);
@@ -960,7 +961,8 @@ int alien_hip_ilu0_factor_f64(alien_hip_ctx* ctx, int n, const int* ro, const in
   REQUIRE(nlevels == 0 || (lptr_host[0] == 0 && lptr_host[nlevels] == n), "ilu0_factor_f64: schedule must cover the rows");
   API_BEGIN
   if (sync_levels(n, nlevels) && ctx->reserve_ilu(n))
-    launch_sync_factor(ctx->stream, n, nlevels, lrows, ro, cols, dcol, lu, ctx->ilu_piv.data(), ctx->ilu_work.data());
+    launch_sync_factor(ctx->stream, n, nlevels, lrows, ro, cols, dcol, lu, ctx->ilu_piv.back().data(),
+                       ctx->ilu_work.data());
   else
     launch_ilu0_factor<double>(ctx->stream, nlevels, lptr_host, lrows, ro, cols, dcol, lu);
   LAUNCHED("ilu0_factor_f64");

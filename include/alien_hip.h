@@ -324,8 +324,10 @@ int alien_hip_spmv_dot_csr_f64_noalloc(void* stream, int nrows, const int* row_o
  * branch (ILU0Preconditioner.h:71-179, 156-178). level_rows lists the rows of
  * level l in level_ptr[l]..level_ptr[l+1] (built on the host from
  * alien_hip_host_levels with upper = 0). One launch for all levels, rows waiting for
- * the rows they read, with a workspace of the context (8 bytes per row, kept); one launch per
- * level inside a stream capture, so that a graph holds the caller's arrays only. */
+ * the rows they read, with a workspace of the context (8 bytes per row of the largest system so
+ * far, up to four times that after growing; allocated without a wait for the stream, kept until the
+ * context is destroyed); one launch per level where there is no memory for it, and inside a stream
+ * capture, so that a graph holds the caller's arrays only. */
 int alien_hip_ilu0_factor_f64(alien_hip_ctx* ctx, int nrows, const int* row_offset, const int* cols,
                               const int* dcol, double* lu, int nlevels, const int* level_ptr_host,
                               const int* level_rows);

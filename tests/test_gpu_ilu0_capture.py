@@ -66,3 +66,30 @@ def test_graph_outlives_the_workspace():
             g.replay()
             s.synchronize()
             assert torch.equal(x, want) and torch.equal(lu, want_lu)
+
+
+def test_larger_system_while_the_stream_is_busy():
+    """The workspace grows without a wait for the stream, under a smaller system's launches that are still to run."""
+    print("case small and larger system behind 400 copies", flush=True)
+    (small, lu, x), (large, _, xl) = system("fill"), system("wide")
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s), aa.Context(s.cuda_stream) as c:
+        with aa.Context(s.cuda_stream) as other:
+            small(other)
+            large(other)
+            s.synchronize()
+            want, want_lu, want_large = x.clone(), lu.clone(), xl.clone()
+        x.zero_()
+        xl.zero_()
+        a = torch.zeros(1 << 28, dtype=torch.float64, device="cuda")
+        b = torch.empty_like(a)
+        s.synchronize()
+        for _ in range(400):  # 2 GiB each: 0.3 s in all
+            b.copy_(a)
+        copied = torch.cuda.Event()
+        copied.record(s)
+        small(c)
+        large(c)
+        assert not copied.query()
+        s.synchronize()
+        assert torch.equal(x, want) and torch.equal(lu, want_lu) and torch.equal(xl, want_large)
