@@ -182,6 +182,9 @@ struct alien_hip_ctx {
     ALIEN_HIP_CHECK(hipMemsetAsync(grid_head.data(), 0, sizeof(int) * grid_head.size(), stream));
   }
   // pivots (one per row, in the last block) and ticket, flag of the ILU(0) kernels of ilu0_sync.hip
+  // Threads that call the entry points on one context take turns to queue a call's launches: the first of them clears
+  // what the others use.
+  std::mutex ilu_turn;
   std::vector<alien_hip::DeviceArray<double>> ilu_piv;
   alien_hip::DeviceArray<int> ilu_work;
   // Room for them, without a wait for the stream: a block that has become too small stays (queued launches may use it)

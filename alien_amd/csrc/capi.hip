@@ -960,6 +960,7 @@ int alien_hip_ilu0_factor_f64(alien_hip_ctx* ctx, int n, const int* ro, const in
           "ilu0_factor_f64: bad arguments");
   REQUIRE(nlevels == 0 || (lptr_host[0] == 0 && lptr_host[nlevels] == n), "ilu0_factor_f64: schedule must cover the rows");
   API_BEGIN
+  const std::lock_guard<std::mutex> turn(ctx->ilu_turn);
   if (sync_levels(n, nlevels) && ctx->reserve_ilu(n))
     launch_sync_factor(ctx->stream, n, nlevels, lrows, ro, cols, dcol, lu, ctx->ilu_piv.back().data(),
                        ctx->ilu_work.data());
@@ -979,6 +980,7 @@ int alien_hip_ilu0_solve_f64(alien_hip_ctx* ctx, int n, const int* ro, const int
   REQUIRE(nl == 0 || (lptr[0] == 0 && lptr[nl] == n), "ilu0_solve_f64: lower schedule must cover the rows");
   REQUIRE(nu == 0 || (uptr[0] == 0 && uptr[nu] == n), "ilu0_solve_f64: upper schedule must cover the rows");
   API_BEGIN
+  const std::lock_guard<std::mutex> turn(ctx->ilu_turn);
   const bool apart = std::abs(y - t) >= n && std::abs(x - t) >= n; // a sweep that overwrites its input goes level by level
   if (apart && sync_levels(n, nl) && sync_levels(n, nu) && ctx->reserve_ilu(0))
     launch_sync_solve(ctx->stream, n, nl, lrows, nu, urows, ro, cols, dcol, lu, y, t, x, ctx->ilu_work.data());

@@ -1,6 +1,8 @@
-"""ILU(0) factorisation and sweeps through the C entry points in a captured graph: it holds the caller's arrays only, so it
-replays rightly after a larger system has gone through the context, and after the context is gone."""
+"""The context's workspace of the ILU(0) entry points. A captured graph holds the caller's arrays only, so it replays rightly
+after a larger system has gone through the context, and after the context is gone; the workspace grows under queued work; two
+threads may call on one context."""
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -93,3 +95,34 @@ def test_larger_system_while_the_stream_is_busy():
         assert not copied.query()
         s.synchronize()
         assert torch.equal(x, want) and torch.equal(lu, want_lu) and torch.equal(xl, want_large)
+
+
+def test_two_threads_on_one_context():
+    """Calls of two threads on one context: its stream runs them whole, one after the other."""
+    print("case two threads, one context", flush=True)
+    systems = [system("fill"), system("wide")]
+    with aa.Context() as c:
+        want = []
+        for run, lu, x in systems:
+            run(c)
+            c.synchronize()
+            want.append((lu.clone(), x.clone()))
+        torch.cuda.synchronize()
+        same = [True, True]
+
+        def work(k):
+            run, lu, x = systems[k]
+            s = torch.cuda.Stream()
+            for _ in range(20):
+                run(c)
+                c.synchronize()
+                with torch.cuda.stream(s):
+                    same[k] = same[k] and torch.equal(lu, want[k][0]) and torch.equal(x, want[k][1])
+                s.synchronize()
+
+        threads = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert same == [True, True]
