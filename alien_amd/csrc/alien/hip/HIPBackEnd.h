@@ -500,19 +500,20 @@ class HIPMatrix
   // Whether the FP32 values may be read as symmetric ones (RBMat::sym), looked up once per set of values: a pass over
   // them and 10 us. Mixed CG with the learned factor, us an iteration without and with: 96^3 40.6 and 38.9, 128^3 72.6
   // and 64.8, 160^3 114.7 and 105.3, 256^3 320 and 306; with Jacobi 49.7 and 41.7 at 128^3. Smaller systems, most of
-  // them solved in one launch that holds the values in registers, are not looked at.
-  void findSymmetry32() {
+  // them solved in one launch that holds the values in registers, are not looked at. ctx: the solve's, not the matrix's
+  // own, which another thread may be using (its scalar slots and posted words are one thread's).
+  void findSymmetry32(alien_hip_ctx* ctx) {
     if (!m_uni || m_fused_ell || m_sym32 >= 0) return;
     m_sym32 = 0;
     if (m_uni != 7 || m_n < kSymMinRows) return;
     for (int j = 0; j <= 3; ++j)
       if (m_uoff[j] != -m_uoff[6 - j]) return;
-    const int s = m_ctx->take_slot();
-    ALIEN_HIP_CHECK(hipMemsetAsync(m_ctx->dslot(s), 0, sizeof(int), m_ctx->stream));
-    alien_hip::launch_uniform_symmetric(m_ctx->stream, m_n, m_uoff, d_bv32.data(), reinterpret_cast<int*>(m_ctx->dslot(s)));
+    const int s = ctx->take_slot();
+    ALIEN_HIP_CHECK(hipMemsetAsync(ctx->dslot(s), 0, sizeof(int), ctx->stream));
+    alien_hip::launch_uniform_symmetric(ctx->stream, m_n, m_uoff, d_bv32.data(), reinterpret_cast<int*>(ctx->dslot(s)));
     alien_hip::check_launch("uniform_symmetric");
     int bad = 1;
-    m_ctx->read_words(m_ctx->dslot(s), &bad, 1);
+    ctx->read_words(ctx->dslot(s), &bad, 1);
     m_sym32 = bad ? 0 : 1;
   }
   bool isRBDIA() const { return m_rbdia && !m_fused_ell; }

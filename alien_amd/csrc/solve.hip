@@ -1595,7 +1595,7 @@ void solve_on(alien_hip_ctx* ctx, const alien_hip_solve_params* p, HIPMatrix& A,
     } else {
       // FP32 matrix, preconditioner and Krylov vectors, FP64 dots; FP64 defect correction
       A.ensureRB32();
-      if (!bicg) A.findSymmetry32();
+      if (!bicg) A.findSymmetry32(ctx);
       phase("FP32 matrix");
       DeviceArray<float> invd32(n);
       launch_demote(ctx->stream, n, invd64, invd32.data());

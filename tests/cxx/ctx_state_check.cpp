@@ -134,9 +134,32 @@ void flag_is_read() {
   std::printf("{\"check\": \"flag_is_read\", \"status\": %d, \"up\": %d, \"residual\": %.17g}\n", status, up, worst);
 }
 
+// A kept matrix solved through another context than the one it was made on leaves that one's scalar slots alone (another
+// thread may be solving there), with the same result.
+void matrix_of_another_context() {
+  const System a = generate(ALIEN_HIP_GEN_LOGNORMAL7, 81, 81, 81, 4);
+  Context own, other;
+  Solved got[2];
+  int moved = 0;
+  for (const Context* c : {&other, &own}) {
+    alien_hip_matrix* m = nullptr;
+    call(alien_hip_matrix_create(own.c, a.n, a.ro.data(), a.cols.data(), a.vals.data(), &m), "matrix_create");
+    const int slot = own->next_slot;
+    Solved& s = got[c == &own];
+    s.x.assign(a.n, 0.0);
+    alien_hip_solve_params p = params(ALIEN_HIP_PREC_DIAG, ALIEN_HIP_MODE_MIXED, 1e-8);
+    p.max_iter = 40;
+    call(alien_hip_solve(c->c, &p, m, a.b.data(), s.x.data(), &s.r), "solve");
+    if (c == &other) moved = own->next_slot != slot;
+    alien_hip_matrix_destroy(m);
+  }
+  std::printf("{\"check\": \"matrix_of_another_context\", \"moved\": %d, \"same\": %d}\n", moved, got[0] == got[1]);
+}
+
 const std::map<std::string, std::function<void()>> kChecks = {
     {"after_a_wait_given_up", after_a_wait_given_up},
     {"flag_is_read", flag_is_read},
+    {"matrix_of_another_context", matrix_of_another_context},
 };
 
 } // namespace

@@ -33,3 +33,7 @@ def test_flag_is_read():
     out = run("flag_is_read")
     assert out.pop("residual") <= 1.05
     assert out == {"status": 1, "up": 0}
+
+
+def test_matrix_of_another_context():
+    assert run("matrix_of_another_context") == {"moved": 0, "same": 1}
