@@ -156,8 +156,37 @@ void matrix_of_another_context() {
   std::printf("{\"check\": \"matrix_of_another_context\", \"moved\": %d, \"same\": %d}\n", moved, got[0] == got[1]);
 }
 
+// A dot product into a future, captured: the future gives the last replay's value, not the first one's.
+void captured_dot() {
+  Context c;
+  const int n = 5000;
+  Alien::HIPInternalLinearAlgebra alg(c.c);
+  Alien::HIPVector x(Alien::HIPResource{n, c.c});
+  const std::vector<double> ones(n, 1.0);
+  x.setValues(ones.data());
+  double v = 0;
+  Alien::HIPFuture f(v);
+  hipGraph_t g;
+  hipGraphExec_t e;
+  ALIEN_HIP_CHECK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
+  alg.dot(x, x, f);
+  ALIEN_HIP_CHECK(hipStreamEndCapture(c->stream, &g));
+  ALIEN_HIP_CHECK(hipGraphInstantiate(&e, g, nullptr, nullptr, 0));
+  for (int k = 1; k <= 3; ++k) {
+    const std::vector<double> h(n, (double)k);
+    x.setValues(h.data());
+    ALIEN_HIP_CHECK(hipGraphLaunch(e, c->stream));
+    ALIEN_HIP_CHECK(hipStreamSynchronize(c->stream));
+  }
+  const double got = f.get(), eager = alg.dot(x, x);
+  ALIEN_HIP_CHECK(hipGraphExecDestroy(e));
+  ALIEN_HIP_CHECK(hipGraphDestroy(g));
+  std::printf("{\"check\": \"captured_dot\", \"value\": %.17g, \"eager\": %.17g}\n", got, eager);
+}
+
 const std::map<std::string, std::function<void()>> kChecks = {
     {"after_a_wait_given_up", after_a_wait_given_up},
+    {"captured_dot", captured_dot},
     {"flag_is_read", flag_is_read},
     {"matrix_of_another_context", matrix_of_another_context},
 };

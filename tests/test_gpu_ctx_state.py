@@ -37,3 +37,7 @@ def test_flag_is_read():
 
 def test_matrix_of_another_context():
     assert run("matrix_of_another_context") == {"moved": 0, "same": 1}
+
+
+def test_captured_dot():
+    assert run("captured_dot") == {"value": 9 * 5000, "eager": 9 * 5000}
