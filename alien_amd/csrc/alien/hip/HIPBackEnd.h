@@ -677,8 +677,8 @@ class HIPMatrix
 };
 
 // Future of a device-resident scalar: dot(x, y, f) leaves the result on the
-// device; get() copies it back and synchronises (SYCLInternal::Future,
-// sycl/algebra/SYCLKernelInternal.h:32-84).
+// device; get() reads it back behind everything queued by then, so that it synchronises with a caller's
+// own work on the stream too (SYCLInternal::Future, sycl/algebra/SYCLKernelInternal.h:32-84).
 class HIPFuture {
  public:
   explicit HIPFuture(double& v) : m_value(v) {}
@@ -815,10 +815,12 @@ class HIPInternalLinearAlgebra
     alien_hip::check_launch("dot");
     return m_ctx->read_slot(s);
   }
+  // (not posted by the dot itself: what a caller queues behind it would not be waited for, and in a captured graph every
+  // replay would post under one tag)
   void dot(const Vector& x, const Vector& y, FutureType& f) const {
     const int s = m_ctx->take_slot();
     alien_hip::launch_dot<double>(stream(), m_ctx->red_once(), x.scalarizedLocalSize(), x.data(), y.data(),
-                                  m_ctx->dslot(s), m_ctx->post_slot(s));
+                                  m_ctx->dslot(s));
     alien_hip::check_launch("dot(future)");
     f.attach(m_ctx, s);
   }

@@ -27,13 +27,11 @@ class Iteration {
  public:
   typedef AlgebraT AlgebraType;
   typedef typename AlgebraType::Vector VectorType;
-  typedef typename AlgebraType::FutureType FutureType;
   typedef double ValueType;
 
   Iteration(AlgebraType& alg, const VectorType& b, ValueType tol, int max_iter, ITraceMng* = nullptr)
-  : m_alg(alg), m_max_it(max_iter), m_tol(tol), m_future(m_value) {
-    m_alg.dot(b, b, m_future);
-    m_nrm2_b = m_future.get();
+  : m_alg(alg), m_max_it(max_iter), m_tol(tol) {
+    m_nrm2_b = m_alg.dot(b, b);
     m_criteria = m_tol * m_tol * m_nrm2_b;
     m_sqrt_nrm2_b = std::sqrt(m_nrm2_b);
     m_value = m_criteria + 1;
@@ -44,8 +42,8 @@ class Iteration {
   // iter >= max: stop without a dot; else status = (r,r) < tol^2 (b,b)
   bool stop(const VectorType& r) {
     if (m_iter >= m_max_it) return true;
-    m_alg.dot(r, r, m_future);
-    m_status = m_future.get() < m_criteria;
+    m_value = m_alg.dot(r, r); // (needed at once: a future's get() would wait for the stream besides)
+    m_status = m_value < m_criteria;
     return m_status;
   }
   void operator++() { ++m_iter; }
@@ -68,7 +66,6 @@ class Iteration {
   ValueType m_tol = 0;
   int m_iter = 0;
   ValueType m_value = 0;
-  FutureType m_future;
   ValueType m_criteria = 0, m_nrm2_b = 0, m_sqrt_nrm2_b = 0;
   bool m_status = false;
 };

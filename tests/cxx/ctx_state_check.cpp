@@ -184,10 +184,36 @@ void captured_dot() {
   std::printf("{\"check\": \"captured_dot\", \"value\": %.17g, \"eager\": %.17g}\n", got, eager);
 }
 
+// A future's get() returns when what was queued behind the dot is done too. (An event tells: the stream itself may not yet
+// be idle, the launch that handed the value over being its last.)
+void future_synchronises() {
+  Context c;
+  const int n = 5000;
+  Alien::HIPInternalLinearAlgebra alg(c.c);
+  Alien::HIPVector x(Alien::HIPResource{n, c.c});
+  const std::vector<double> ones(n, 1.0);
+  x.setValues(ones.data());
+  const size_t bytes = size_t(1) << 30;
+  alien_hip::DeviceArray<char> a(bytes), b(bytes);
+  double v = 0;
+  Alien::HIPFuture f(v);
+  alg.dot(x, x, f);
+  for (int k = 0; k < 100; ++k)  // 40 ms
+    ALIEN_HIP_CHECK(hipMemcpyAsync(a.data(), b.data(), bytes, hipMemcpyDeviceToDevice, c->stream));
+  hipEvent_t copied;
+  ALIEN_HIP_CHECK(hipEventCreate(&copied));
+  ALIEN_HIP_CHECK(hipEventRecord(copied, c->stream));
+  const double got = f.get();
+  const bool done = hipEventQuery(copied) == hipSuccess;
+  ALIEN_HIP_CHECK(hipEventDestroy(copied));
+  std::printf("{\"check\": \"future_synchronises\", \"value\": %.17g, \"done\": %d}\n", got, done);
+}
+
 const std::map<std::string, std::function<void()>> kChecks = {
     {"after_a_wait_given_up", after_a_wait_given_up},
     {"captured_dot", captured_dot},
     {"flag_is_read", flag_is_read},
+    {"future_synchronises", future_synchronises},
     {"matrix_of_another_context", matrix_of_another_context},
 };
 

@@ -41,3 +41,7 @@ def test_matrix_of_another_context():
 
 def test_captured_dot():
     assert run("captured_dot") == {"value": 9 * 5000, "eager": 9 * 5000}
+
+
+def test_future_synchronises():
+    assert run("future_synchronises") == {"value": 5000, "done": 1}
