@@ -162,7 +162,7 @@ class ILU0Preconditioner<HIPInternalLinearAlgebra> {
     m_pencil = false;
     d_lu.reset();
     if (!alien_hip::g_ilu_sync_free || !alien_hip::pencil_grid(n, m_A.kcol(), m_A.cols(), g)) return false;
-    const int zero[alien_hip::kPencilWork] = {0, 0, 0};
+    const int zero[alien_hip::kPencilWork] = {};
     int bad[alien_hip::kPencilWork];
     d_penwork.upload(zero, alien_hip::kPencilWork, st);
     alien_hip::launch_pencil_check(st, n, g, m_A.d_ro.data(), m_A.d_cols.data(), d_penwork.data());

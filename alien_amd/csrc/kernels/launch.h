@@ -230,7 +230,7 @@ struct PencilGrid {
     return ((long)(z / 8 * py + y / 8) * steps + x + yl + zl) * 64 + zl * 8 + yl;
   }
 };
-constexpr int kPencilWork = 3; // tickets of the two sweeps, error flag
+constexpr int kPencilWork = 4; // tickets of the two sweeps, flags of a lower (or the factorisation) and an upper one that gave up
 template <typename T>
 struct PencilFactor {
   PencilGrid g;
@@ -254,7 +254,7 @@ void launch_pencil_factor(hipStream_t, const PencilFactor<double>& F, const int*
 void launch_pencil_demote(hipStream_t, const PencilFactor<double>& F, float* base);
 // the factor in CSR order; lu: A's values on entry
 void launch_pencil_to_csr(hipStream_t, int n, const PencilFactor<double>& F, const int* ro, double* lu);
-// x = (LU)^-1 y; returns early once *done; may be captured
+// x = (LU)^-1 y (x may be y); returns early once *done; may be captured
 template <typename T>
 void launch_pencil_apply(hipStream_t, const PencilFactor<T>& F, const T* y, T* x, const int* done = nullptr);
 

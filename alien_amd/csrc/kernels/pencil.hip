@@ -158,7 +158,8 @@ __device__ __forceinline__ double lane_y(double v) {
 // one load per face and chunk, issued a chunk ahead and polled again only if it came too early.
 // Two sets of faces and tickets: the lower sweep uses set 0 and clears set 1, the upper sweep and
 // the factorisation the other way round, so neither needs a clearing launch before it. Waits are
-// bounded (limit polls); one that runs out raises work[2] and the redo kernel follows.
+// bounded (limit polls); one that runs out raises work[2], in the upper sweep work[3], and the redo kernel
+// follows. The upper sweep stores nothing after a lower one that gave up: `out` may be `in`, which the redo then reads.
 // Bound by the instructions and waits of a lone wavefront, 0.12 us a lower step and 0.17 an upper one (a lane
 // exchange, three dependent subtractions, the upper's division), and per trip between pencils by 15 steps of skew
 // and chunk and 1.6 us from store to load. Operands of a step of the next chunk are loaded during each lane exchange, at
@@ -180,7 +181,7 @@ __global__ void __launch_bounds__(kWave) k_pencil_sweep(PencilFactor<T> F, const
   const int np = g.pencils(), S = g.steps;
   const int lane = threadIdx.x, yl = lane % kPen, zl = lane / kPen;
   __shared__ T face[3][kWave], val[C][kWave]; // face[2]: zeros
-  int* err = F.work + 2;
+  int* err = F.work + (UP ? 3 : 2);
 
   int tk = 0;
   if (lane == 0) tk = __hip_atomic_fetch_add(F.work + set, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -213,6 +214,7 @@ __global__ void __launch_bounds__(kWave) k_pencil_sweep(PencilFactor<T> F, const
     }
     if (tk == 0 && lane == 0) F.work[1 - set] = 0;
   }
+  if (UP && __hip_atomic_load(F.work + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
   const bool fromy = UP ? b < g.py - 1 : b > 0, fromz = UP ? c < g.pz - 1 : c > 0; // a pencil feeds this one
   const bool toy = UP ? b > 0 : b < g.py - 1, toz = UP ? c > 0 : c < g.pz - 1;     // this one feeds a pencil
   constexpr int edge = UP ? kPen - 1 : 0, far = kPen - 1 - edge; // lines fed by, and feeding, another pencil
@@ -372,13 +374,14 @@ __global__ void __launch_bounds__(kWave) k_pencil_sweep(PencilFactor<T> F, const
 }
 
 // A sweep pair (or a factorisation) with a wait that ran out of polls, again, by one workgroup and
-// plane by plane of x + y + z; then the flag is cleared. Without the flag it returns at once.
+// plane by plane of x + y + z, from the sweep that gave up; then the flags are cleared. Without a flag it returns at once.
 constexpr int kPenRedoBlock = 1024;
 template <typename T, bool FAC>
 __global__ void __launch_bounds__(kPenRedoBlock) k_pencil_redo(PencilFactor<T> F, const double* trans, const T* in,
                                                                 T* out, const int* __restrict__ done) {
   if (done && *done) return;
-  if (__hip_atomic_load(F.work + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) return;
+  const bool lower = __hip_atomic_load(F.work + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+  if (!lower && __hip_atomic_load(F.work + 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) return;
   const PencilGrid& g = F.g;
   const long np = g.positions();
   const int planes = g.nx + g.ny + g.nz - 2, lines = g.ny * g.nz;
@@ -390,7 +393,7 @@ __global__ void __launch_bounds__(kPenRedoBlock) k_pencil_redo(PencilFactor<T> F
     }
     __syncthreads();
   };
-  for (int d = 0; d < planes; ++d)
+  for (int d = 0; lower && d < planes; ++d)
     each(d, [&](int x, int y, int z, long q) {
       const T* from = FAC ? dd : F.t;
       const T vz = z > 0 ? from[g.position(x, y, z - 1)] : T(0), vy = y > 0 ? from[g.position(x, y - 1, z)] : T(0),
@@ -419,7 +422,7 @@ __global__ void __launch_bounds__(kPenRedoBlock) k_pencil_redo(PencilFactor<T> F
         if (z < g.nz - 1) v = v - uz[q] * out[i + (long)g.nx * g.ny];
         out[i] = v / dd[q];
       });
-  if (threadIdx.x == 0) __hip_atomic_store(F.work + 2, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (threadIdx.x < 2) __hip_atomic_store(F.work + 2 + threadIdx.x, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 void launch_pencil_check(hipStream_t st, int n, const PencilGrid& g, const int* ro, const int* cols, int* bad) {

@@ -1,5 +1,5 @@
-// What calls leave in the state of a context: calls that end off the straight path (a wait given up, a stream
-// capture, a second context), followed by ordinary ones on the same context. Prints one JSON object per check on stdout
+// What calls leave in the state of a context: calls off the straight path (a wait given up, a stream capture, a second
+// context, a result in its operand's place), followed by ordinary ones on the same context. Prints one JSON object per check on stdout
 // for tests/test_gpu_ctx_state.py. The internal headers give the checks the context's own fields.
 // Usage: ctx_state_check [check ...]  (all of them without an argument)
 #include <cstdio>
@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "alien/hip/HIPBackEnd.h"
+#include "alien/hip/krylov/HIPILU0Preconditioner.h"
 
 namespace {
 
@@ -209,12 +210,40 @@ void future_synchronises() {
   std::printf("{\"check\": \"future_synchronises\", \"value\": %.17g, \"done\": %d}\n", got, done);
 }
 
+// ILU(0) in pencils, the result in the right-hand side's place, with every wait given up and with none: as apart.
+void pencils_in_place() {
+  const System a = generate(ALIEN_HIP_GEN_CONVDIFF7, 21, 18, 19, 5);
+  Context c;
+  Alien::HIPInternalLinearAlgebra alg(c.c);
+  Alien::HIPMatrix A(static_cast<const Alien::MultiMatrixImpl*>(nullptr));
+  A.build(c.c, Alien::CSRHostView{a.n, a.ro.data(), a.cols.data(), a.vals.data()}, Alien::kLayoutCSR);
+  const long usual = alien_hip::g_ilu_sf_spins;
+  std::vector<double> x[3];
+  bool pencils = true;
+  for (int k = 0; k < 3; ++k) { // apart; in place; in place, given up
+    alien_hip::g_ilu_sf_spins = usual;
+    Alien::ILU0Preconditioner<Alien::HIPInternalLinearAlgebra> P(alg, A);
+    P.init();
+    pencils = pencils && P.pencils();
+    Alien::HIPVector y(A.resource()), z(A.resource());
+    y.setValues(a.b.data());
+    alien_hip::g_ilu_sf_spins = k == 2 ? 0 : usual;
+    P.solve(alg, y, k == 0 ? z : y);
+    x[k].resize(a.n);
+    (k == 0 ? z : y).copyValuesTo(x[k].data());
+  }
+  alien_hip::g_ilu_sf_spins = usual;
+  std::printf("{\"check\": \"pencils_in_place\", \"pencils\": %d, \"in_place\": %d, \"given_up\": %d}\n", pencils,
+              x[1] == x[0], x[2] == x[0]);
+}
+
 const std::map<std::string, std::function<void()>> kChecks = {
     {"after_a_wait_given_up", after_a_wait_given_up},
     {"captured_dot", captured_dot},
     {"flag_is_read", flag_is_read},
     {"future_synchronises", future_synchronises},
     {"matrix_of_another_context", matrix_of_another_context},
+    {"pencils_in_place", pencils_in_place},
 };
 
 } // namespace

@@ -45,3 +45,7 @@ def test_captured_dot():
 
 def test_future_synchronises():
     assert run("future_synchronises") == {"value": 5000, "done": 1}
+
+
+def test_pencils_in_place():
+    assert run("pencils_in_place") == {"pencils": 1, "in_place": 1, "given_up": 1}
