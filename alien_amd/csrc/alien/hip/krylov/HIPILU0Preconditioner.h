@@ -36,6 +36,7 @@ class ILU0Preconditioner<HIPInternalLinearAlgebra> {
   void init() {
     const int n = m_A.getNRows();
     hipStream_t st = m_alg.stream();
+    m_pencil = false; // (of an init() before a colour schedule)
     if (!m_colours.empty()) {
       const int nc = (int)m_colours.size() - 1;
       m_nl = m_nu = nc;
@@ -159,7 +160,6 @@ class ILU0Preconditioner<HIPInternalLinearAlgebra> {
   bool buildPencils(hipStream_t st) {
     const int n = m_A.getNRows();
     alien_hip::PencilGrid g;
-    m_pencil = false;
     d_lu.reset();
     if (!alien_hip::g_ilu_sync_free || !alien_hip::pencil_grid(n, m_A.kcol(), m_A.cols(), g)) return false;
     const int zero[alien_hip::kPencilWork] = {};

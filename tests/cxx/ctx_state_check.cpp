@@ -237,9 +237,39 @@ void pencils_in_place() {
               x[1] == x[0], x[2] == x[0]);
 }
 
+// init() again with a colour schedule and new values on a preconditioner that had taken pencils: the new factor's sweeps.
+void colours_after_pencils() {
+  const System a = generate(ALIEN_HIP_GEN_CONVDIFF7, 10, 8, 8, 6);
+  Context c;
+  Alien::HIPInternalLinearAlgebra alg(c.c);
+  Alien::HIPMatrix A(static_cast<const Alien::MultiMatrixImpl*>(nullptr));
+  A.build(c.c, Alien::CSRHostView{a.n, a.ro.data(), a.cols.data(), a.vals.data()}, Alien::kLayoutCSR);
+  Alien::ILU0Preconditioner<Alien::HIPInternalLinearAlgebra> P(alg, A), fresh(alg, A);
+  P.init();
+  const bool pencils = P.pencils();
+  std::vector<double> vals(a.vals), x[2];
+  for (size_t k = 0; k < vals.size(); ++k) vals[k] *= 1.0 + 0.01 * (k % 7);
+  A.updateValues(vals.data());
+  std::vector<int> colours(a.n + 1); // each row a colour of its own
+  for (int i = 0; i <= a.n; ++i) colours[i] = i;
+  P.setColourSchedule(colours);
+  P.init();
+  fresh.init();
+  Alien::HIPVector y(A.resource()), z(A.resource());
+  y.setValues(a.b.data());
+  for (int k = 0; k < 2; ++k) {
+    (k == 0 ? P : fresh).solve(alg, y, z);
+    x[k].resize(a.n);
+    z.copyValuesTo(x[k].data());
+  }
+  std::printf("{\"check\": \"colours_after_pencils\", \"pencils\": [%d, %d], \"same\": %d}\n", pencils, P.pencils(),
+              x[0] == x[1]);
+}
+
 const std::map<std::string, std::function<void()>> kChecks = {
     {"after_a_wait_given_up", after_a_wait_given_up},
     {"captured_dot", captured_dot},
+    {"colours_after_pencils", colours_after_pencils},
     {"flag_is_read", flag_is_read},
     {"future_synchronises", future_synchronises},
     {"matrix_of_another_context", matrix_of_another_context},

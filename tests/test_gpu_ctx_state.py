@@ -49,3 +49,7 @@ def test_future_synchronises():
 
 def test_pencils_in_place():
     assert run("pencils_in_place") == {"pencils": 1, "in_place": 1, "given_up": 1}
+
+
+def test_colours_after_pencils():
+    assert run("colours_after_pencils") == {"pencils": [1, 0], "same": 1}
