@@ -12,8 +12,8 @@
 // trees (lanes, wavefronts, workgroups and finalize of the launches), so the iterates are the
 // launches' bit for bit.
 // Every workgroup has to be running: there are no more than compute units, a workgroup fits beside
-// any other kernel's once that ends, and the caller keeps a second such launch of the process off
-// the device (resident_mutex); what else might hold one back too long runs the waits out of polls.
+// any other kernel's once that ends, and the caller lets such launches of the process run together only where
+// the compute units hold them all (ResidentTurn); what else might hold one back too long runs the waits out of polls.
 // Bound by the latency of the sums, about 3 us each, and in one workgroup by its instructions. An iteration of
 // Jacobi-CG in FP64 against the graph of launches: 14 x 11 x 9 cells 2.8 us (16), 32^3 5.6 (18), 64^3 8.5 (21), 80^3 (two
 // rows per lane, which spill) 22 (30); FP32 in the mixed solver 7.9 (19) at 64^3; Chebyshev of degree 3 16 (39) at
@@ -504,6 +504,7 @@ bool resident_plan(int n, const RBMat<T>& A, int cus, int cheb_order, ResidentPl
   if (!P.one) P.lds = 0;
   const long blocks = P.one ? 1 : std::min(cus, kResidentMaxBlocks);
   P.rows = n <= blocks * kResBlock ? 1 : 2;
+  P.blocks = (n + kResBlock * P.rows - 1) / (kResBlock * P.rows);
   return n <= blocks * kResBlock * P.rows && (P.rows == 1 || P.one || cheb_order == 0);
 }
 
@@ -537,8 +538,7 @@ bool launch_cg_resident(hipStream_t s, const ResidentPlan& P, int n, RBMat<T> A,
   GridSums g{slots, head, 0, spins};
   ResidentCheb cb = cheb;
   void* args[] = {&n, &A, &invd, &x, &r, &z, &p, &ex, &st, &g, &cb, &iters, &check, &below};
-  const long per = (long)kResBlock * P.rows;
-  if (hipLaunchKernel(f, dim3((unsigned)((n + per - 1) / per)), dim3(kResBlock), args, P.lds, s) != hipSuccess) {
+  if (hipLaunchKernel(f, dim3((unsigned)P.blocks), dim3(kResBlock), args, P.lds, s) != hipSuccess) {
     (void)hipGetLastError();
     return false;
   }

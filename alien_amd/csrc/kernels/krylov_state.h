@@ -166,6 +166,7 @@ struct ResidentPlan {
   int rows = 0;            // per lane
   bool pairs = false;      // p.q is summed over pairs of bundles
   bool one = false;        // one workgroup, its exchange in LDS
+  int blocks = 0;          // workgroups, each on a compute unit
   size_t lds = 0;
   int exchange = 0; // vectors of workspace (none of memory with `one`)
 };

@@ -9,7 +9,6 @@
 #include <cmath>
 #include <cstring>
 #include <memory>
-#include <mutex>
 #include <numeric>
 #include <type_traits>
 #include <vector>
@@ -23,6 +22,7 @@
 #include "kernels/gnn.h"
 #include "kernels/krylov_state.h"
 #include "kernels/launch.h"
+#include "kernels/resident_turn.h"
 
 namespace alien_hip {
 
@@ -342,13 +342,6 @@ struct ProgressWatch {
   }
 };
 
-// One resident launch at a time per device: two that each hold half of the compute units would wait
-// for each other. Held from the launch to the read of the state.
-std::mutex& resident_mutex(int device) {
-  static std::mutex m[64];
-  return m[device & 63];
-}
-
 template <typename T>
 struct FusedCG {
   alien_hip_ctx* ctx;
@@ -401,7 +394,8 @@ struct FusedCG {
   // the count stays where it was (r.r is the launch's, not finite where x may not be).
   CGState advance_resident(T* x, int check, double below) {
     const CGState before = *h_st;
-    const std::lock_guard<std::mutex> alone(resident_mutex(ctx->device));
+    // (from the launch to the read of the state; one workgroup waits for none)
+    const ResidentTurn turn(resident_gate(ctx->device), res.one ? 0 : res.blocks, ctx->cus);
     if (!launch_cg_resident<T>(ctx->stream, res, n, A, invd, x, r.data(), z.data(), p.data(), ex.data(),
                                st.data(), ctx->grid_slots.data(), ctx->grid_head.data(), res_cheb,
                                kResidentIters, check, below, ctx->resident_spins)) {
@@ -1166,6 +1160,12 @@ double true_residual(Alg& alg, const HIPMatrix& A, const HIPVector& b, const HIP
 } // namespace alien_hip
 
 namespace alien_hip {
+
+ResidentGate& resident_gate(int device) {
+  static ResidentGate g[64];
+  return g[device & 63];
+}
+
 namespace {
 
 // Parameter checks shared by the solve entry points.

@@ -13,6 +13,7 @@
 
 #include "alien/hip/HIPBackEnd.h"
 #include "alien/hip/krylov/HIPILU0Preconditioner.h"
+#include "kernels/resident_turn.h"
 
 namespace {
 
@@ -266,6 +267,20 @@ void colours_after_pencils() {
               x[0] == x[1]);
 }
 
+// Solves of one workgroup go on while another launch holds every compute unit, of a few workgroups while the others are held.
+void small_solves_take_their_share() {
+  const System one = generate(ALIEN_HIP_GEN_LOGNORMAL7, 14, 11, 9, 7), few = generate(ALIEN_HIP_GEN_LOGNORMAL7, 21, 18, 19, 8);
+  Context c;
+  int status = 0;
+  {
+    const alien_hip::ResidentTurn all(alien_hip::resident_gate(c->device), c->cus, c->cus);
+    status += solve(c, one, ALIEN_HIP_MODE_GRAPH).r.status;
+  }
+  const alien_hip::ResidentTurn rest(alien_hip::resident_gate(c->device), c->cus - 8, c->cus);
+  status += solve(c, few, ALIEN_HIP_MODE_GRAPH).r.status;
+  std::printf("{\"check\": \"small_solves_take_their_share\", \"solved\": %d}\n", status);
+}
+
 const std::map<std::string, std::function<void()>> kChecks = {
     {"after_a_wait_given_up", after_a_wait_given_up},
     {"captured_dot", captured_dot},
@@ -274,6 +289,7 @@ const std::map<std::string, std::function<void()>> kChecks = {
     {"future_synchronises", future_synchronises},
     {"matrix_of_another_context", matrix_of_another_context},
     {"pencils_in_place", pencils_in_place},
+    {"small_solves_take_their_share", small_solves_take_their_share},
 };
 
 } // namespace

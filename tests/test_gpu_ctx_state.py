@@ -53,3 +53,7 @@ def test_pencils_in_place():
 
 def test_colours_after_pencils():
     assert run("colours_after_pencils") == {"pencils": [1, 0], "same": 1}
+
+
+def test_small_solves_take_their_share():
+    assert run("small_solves_take_their_share") == {"solved": 2}
