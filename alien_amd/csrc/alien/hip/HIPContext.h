@@ -220,6 +220,7 @@ struct alien_hip_ctx {
   static constexpr int kMailWords = 2 * 64 + alien_hip::kMaxPostWords;
   unsigned last_tag = 0, slot_tag[64] = {}; // tag of the post that fills a slot's words (0: none under way)
   unsigned waits = 0;
+  unsigned polls = 32768; // of posted words before a wait for the stream; none where the program asked for blocking waits
   alien_hip::DeviceArray<unsigned> tickets; // counters of the reductions finished in their own launch, zeros
   // Pinned 512-byte blocks for the fused solvers' host state mirrors, allocated once per context
   // (pinned allocation and release cost far more than a solve's own host work); a solver takes a
@@ -311,7 +312,8 @@ struct alien_hip_ctx {
  private:
   unsigned new_tag() { return last_tag += last_tag == ~0u ? 2 : 1; }
   // The words posted with this tag. The host polls memory: a stored word reaches it in about 2 us, where a
-  // copy and a wait for the stream took 13 to 20. A word that the finished stream has not posted is copied.
+  // copy and a wait for the stream took 13 to 20. After about 1 ms, where those no longer matter, it waits for the
+  // stream and leaves its core to others. A word that the finished stream has not posted is copied.
   void fetch(const unsigned long long* from, unsigned tag, const void* dev, void* to, int n) {
     alien_hip::check_launch("post");
     unsigned* out = static_cast<unsigned*>(to);
@@ -323,15 +325,12 @@ struct alien_hip_ctx {
       }
       return true;
     };
-    for (unsigned spin = 1; !arrived(); ++spin) {
-      __builtin_ia32_pause();
-      if (spin % 32768) continue; // (about 1 ms: a query queues a marker, which delays the kernels behind it)
-      const hipError_t e = hipStreamQuery(stream);
-      if (e == hipErrorNotReady) {
-        (void)hipGetLastError();
+    for (unsigned spin = 0; !arrived(); ++spin) {
+      if (spin < polls) {
+        __builtin_ia32_pause();
         continue;
       }
-      ALIEN_HIP_CHECK(e);
+      ALIEN_HIP_CHECK(hipStreamSynchronize(stream));
       if (arrived()) break;
       ALIEN_HIP_CHECK(hipMemcpyAsync(to, dev, sizeof(unsigned) * n, hipMemcpyDeviceToHost, stream));
       ALIEN_HIP_CHECK(hipStreamSynchronize(stream));

@@ -45,6 +45,10 @@ alien_hip_ctx* make_ctx(void* stream) {
     c->clear_grid();
     ALIEN_HIP_CHECK(hipGetDevice(&c->device));
     ALIEN_HIP_CHECK(hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, c->device));
+    unsigned flags = 0;
+    ALIEN_HIP_CHECK(hipGetDeviceFlags(&flags));
+    flags &= hipDeviceScheduleMask;
+    if (flags == hipDeviceScheduleBlockingSync || flags == hipDeviceScheduleYield) c->polls = 0;
     c->ilu_work.resize(2);
     c->tickets.resize(kTicketWords);
     ALIEN_HIP_CHECK(hipMemsetAsync(c->tickets.data(), 0, sizeof(unsigned) * kTicketWords, c->stream));

@@ -1,10 +1,11 @@
 // What calls leave in the state of a context: calls off the straight path (a wait given up, a stream capture, a second
 // context, a result in its operand's place), followed by ordinary ones on the same context. Prints one JSON object per check on stdout
 // for tests/test_gpu_ctx_state.py. The internal headers give the checks the context's own fields.
-// Usage: ctx_state_check [check ...]  (all of them without an argument)
+// Usage: ctx_state_check [check ...]  (all of them without an argument; blocking_wait has to come first)
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <ctime>
 #include <functional>
 #include <map>
 #include <random>
@@ -281,8 +282,34 @@ void small_solves_take_their_share() {
   std::printf("{\"check\": \"small_solves_take_their_share\", \"solved\": %d}\n", status);
 }
 
+// A program that asked for blocking waits (before anything else on the device) gets them from a read-back too.
+void blocking_wait() {
+  ALIEN_HIP_CHECK(hipSetDeviceFlags(hipDeviceScheduleBlockingSync));
+  Context c;
+  const int n = 5000;
+  Alien::HIPInternalLinearAlgebra alg(c.c);
+  Alien::HIPVector x(Alien::HIPResource{n, c.c});
+  const std::vector<double> ones(n, 1.0);
+  x.setValues(ones.data());
+  const size_t bytes = size_t(1) << 30;
+  alien_hip::DeviceArray<char> a(bytes), b(bytes);
+  double v = alg.dot(x, x);
+  for (int k = 0; k < 200; ++k)  // 90 ms
+    ALIEN_HIP_CHECK(hipMemcpyAsync(a.data(), b.data(), bytes, hipMemcpyDeviceToDevice, c->stream));
+  auto now = [](clockid_t id) {
+    timespec t;
+    clock_gettime(id, &t);
+    return t.tv_sec + 1e-9 * t.tv_nsec;
+  };
+  const double wall = now(CLOCK_MONOTONIC), cpu = now(CLOCK_THREAD_CPUTIME_ID);
+  v = alg.dot(x, x);
+  std::printf("{\"check\": \"blocking_wait\", \"value\": %.17g, \"wall_s\": %.4f, \"cpu_s\": %.4f}\n", v,
+              now(CLOCK_MONOTONIC) - wall, now(CLOCK_THREAD_CPUTIME_ID) - cpu);
+}
+
 const std::map<std::string, std::function<void()>> kChecks = {
     {"after_a_wait_given_up", after_a_wait_given_up},
+    {"blocking_wait", blocking_wait},
     {"captured_dot", captured_dot},
     {"colours_after_pencils", colours_after_pencils},
     {"flag_is_read", flag_is_read},

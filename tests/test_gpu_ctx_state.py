@@ -57,3 +57,11 @@ def test_colours_after_pencils():
 
 def test_small_solves_take_their_share():
     assert run("small_solves_take_their_share") == {"solved": 2}
+
+
+def test_blocking_wait():
+    """A wait of some 90 ms takes less than half of its time from the core."""
+    out = run("blocking_wait")
+    print(out, flush=True)
+    assert out["value"] == 5000
+    assert out["wall_s"] > 0.02 and out["cpu_s"] < 0.5 * out["wall_s"]
