@@ -34,7 +34,6 @@
 
 namespace alien_hip {
 
-constexpr int kResSlots = kResidentMaxSlots;
 
 template <typename T>
 __device__ __forceinline__ T agent_load(const T* p) {
@@ -250,15 +249,16 @@ __device__ __forceinline__ bool grid_sum(GridSums& g, int n, const double (&term
 // memory an exchange inside one workgroup costs as much as between two; 14 x 11 x 9: 3.9 us an iteration with the sums of
 // several workgroups and z exchanged, 2.8 with block_total and p). p itself is exchanged, in ex[0]: one
 // barrier more, and neither the copies' registers (two FP64 rows a lane spilled with them) nor their operations.
-// PQ: the tree of q = A p's p.q on this operand (kSumRows or kSumPairs). K: entries of a row at most.
+// PQ: the tree of q = A p's p.q on this operand (kSumRows or kSumPairs).
 // Where a row has no j-th entry, ONE (bound by its instructions: 16 wavefronts on one compute unit) multiplies two zeros,
 // the value and the vector's entry past the last, and adds +0 to a sum that is never -0; a wavefront without
 // rows in a round does none of its work.
-template <typename T, int R, int K, bool ONE, bool CHEB, int PQ>
+template <typename T, int R, bool ONE, bool CHEB, int PQ>
 __global__ void __launch_bounds__(kResBlock) k_cg_resident(int n, RBMat<T> A, const T* __restrict__ invd, T* x, T* r,
                                                             T* z, T* p, T* ex, CGState* st, GridSums g,
                                                             ResidentCheb cb, int iters, int check, double below) {
   typedef typename SfBits<T>::U U;
+  constexpr int K = kResidentMaxSlots;
   __shared__ SumLds lds;
   extern __shared__ char own_ex[];
   if (st->done) return;
@@ -509,14 +509,10 @@ bool resident_plan(int n, const RBMat<T>& A, int cus, int cheb_order, ResidentPl
 }
 
 template <typename T, int R, bool ONE, bool CHEB>
-static const void* resident_kernel(bool pairs, int width) {
-  // rows of at most 7 entries (the 7-point stencils) do not pay for the eighth
+static const void* resident_kernel(bool pairs) {
   if constexpr (sizeof(T) == 4)
-    if (pairs)
-      return width <= 7 ? (const void*)k_cg_resident<T, R, 7, ONE, CHEB, kSumPairs>
-                        : (const void*)k_cg_resident<T, R, kResSlots, ONE, CHEB, kSumPairs>;
-  return width <= 7 ? (const void*)k_cg_resident<T, R, 7, ONE, CHEB, kSumRows>
-                    : (const void*)k_cg_resident<T, R, kResSlots, ONE, CHEB, kSumRows>;
+    if (pairs) return (const void*)k_cg_resident<T, R, ONE, CHEB, kSumPairs>;
+  return (const void*)k_cg_resident<T, R, ONE, CHEB, kSumRows>;
 }
 
 template <typename T>
@@ -528,8 +524,7 @@ bool launch_cg_resident(hipStream_t s, const ResidentPlan& P, int n, RBMat<T> A,
     constexpr int R = decltype(rows)::value;
     constexpr bool ONE = decltype(one)::value;
     if (P.rows == R && P.one == ONE)
-      f = cheb.order > 0 ? resident_kernel<T, R, ONE, true>(P.pairs, A.wmax)
-                         : resident_kernel<T, R, ONE, false>(P.pairs, A.wmax);
+      f = cheb.order > 0 ? resident_kernel<T, R, ONE, true>(P.pairs) : resident_kernel<T, R, ONE, false>(P.pairs);
   };
   pick(std::integral_constant<int, 1>{}, std::false_type{});
   pick(std::integral_constant<int, 2>{}, std::false_type{});

@@ -152,7 +152,7 @@ void launch_factor_apply(hipStream_t, RedWork w, int n, RBMat<T> G, RBMat<T> GT,
                          CGState* st);
 // CG iterations in one launch (cg_resident.hip), for systems of row-bundled diagonal offsets whose
 // rows the compute units hold in registers; Diag preconditioner, or Chebyshev of an order > 0.
-constexpr int kResidentMaxSlots = 7;    // entries per row
+constexpr int kResidentMaxSlots = 7;    // entries per row: the 7-point stencils'; wider rows are left to the launches
 constexpr int kResidentMaxBlocks = 256; // workgroups, one per compute unit
 constexpr int kResidentMaxRows = kResidentMaxBlocks * 2048;
 constexpr int kResidentSlots = kResidentMaxRows / 256; // workgroups of a row kernel, whose partials are summed

@@ -2,6 +2,7 @@
 // context, a result in its operand's place), followed by ordinary ones on the same context. Prints one JSON object per check on stdout
 // for tests/test_gpu_ctx_state.py. The internal headers give the checks the context's own fields.
 // Usage: ctx_state_check [check ...]  (all of them without an argument; blocking_wait has to come first)
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -307,6 +308,35 @@ void blocking_wait() {
               now(CLOCK_MONOTONIC) - wall, now(CLOCK_THREAD_CPUTIME_ID) - cpu);
 }
 
+// Which rows' systems run in one launch: the phase in the context's head tells. Rows of 6 to 9 entries, in one workgroup and
+// in several.
+void widths_in_one_launch() {
+  std::printf("{\"check\": \"widths_in_one_launch\", \"taken\": [");
+  for (int width = 6; width <= 9; ++width)
+    for (int n : {1000, 5000}) {
+      System a;
+      a.n = n;
+      a.ro.push_back(0);
+      a.b.assign(n, 1.0);
+      const std::vector<int> offsets = {0, -1, 1, -5, 5, -37, 37, -41, 41};
+      for (int i = 0; i < n; ++i) {
+        std::vector<int> c;
+        for (int k = 0; k < width; ++k)
+          if (i + offsets[k] >= 0 && i + offsets[k] < n) c.push_back(i + offsets[k]);
+        std::sort(c.begin(), c.end());
+        for (int j : c) {
+          a.cols.push_back(j);
+          a.vals.push_back(j == i ? 9.0 : -1.0);
+        }
+        a.ro.push_back((int)a.cols.size());
+      }
+      Context c;
+      solve(c, a, ALIEN_HIP_MODE_GRAPH);
+      std::printf("%s%d", width == 6 && n == 1000 ? "" : ", ", read(c->grid_head)[0] != 0);
+    }
+  std::printf("]}\n");
+}
+
 const std::map<std::string, std::function<void()>> kChecks = {
     {"after_a_wait_given_up", after_a_wait_given_up},
     {"blocking_wait", blocking_wait},
@@ -317,6 +347,7 @@ const std::map<std::string, std::function<void()>> kChecks = {
     {"matrix_of_another_context", matrix_of_another_context},
     {"pencils_in_place", pencils_in_place},
     {"small_solves_take_their_share", small_solves_take_their_share},
+    {"widths_in_one_launch", widths_in_one_launch},
 };
 
 } // namespace

@@ -65,3 +65,8 @@ def test_blocking_wait():
     print(out, flush=True)
     assert out["value"] == 5000
     assert out["wall_s"] > 0.02 and out["cpu_s"] < 0.5 * out["wall_s"]
+
+
+def test_widths_in_one_launch():
+    """Rows of up to 7 entries (6 and 7 of 6 to 9, each in one workgroup and in several)."""
+    assert run("widths_in_one_launch") == {"taken": [1, 1, 1, 1, 0, 0, 0, 0]}

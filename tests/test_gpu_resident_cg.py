@@ -1,5 +1,5 @@
 """CG whose iterations run in one launch with the system in registers, against the same solve from launches, bit for
-bit: at the edges of its forms (one workgroup, four and eight rows per lane, and past the last)."""
+bit: at the edges of its forms (one workgroup, one and two rows per lane, and past the last)."""
 import threading
 
 import numpy as np

@@ -1,5 +1,5 @@
-"""Iterations in one launch: rows of 6 to 9 entries (7 and 8 have kernels of their own, 9 is left to the launches), some
-of them missing, in one workgroup and in several, against the same solve from launches, bit for bit."""
+"""Iterations in one launch: rows of 6 to 9 entries (8 and 9 are left to the launches, on either side), some of them
+missing, in one workgroup and in several, against the same solve from launches, bit for bit."""
 import os
 
 import numpy as np
