@@ -285,10 +285,10 @@ struct alien_hip_ctx {
     return s;
   }
   double* dslot(int s) { return scalars.data() + s; }
-  // Where the kernel that writes slot s posts it too, for a read_slot that follows; nowhere inside a stream capture: each
-  // replay would post under the same tag, and a read would take the first replay's value for the last one's.
+  // Where the kernel that writes slot s posts it too, for a read_slot that follows at once. (Nothing that a stream
+  // capture may record posts by itself: each replay would post under the same tag, and a read would take the first
+  // replay's value for the last one's.)
   alien_hip::HostPost post_slot(int s) {
-    if (capturing()) return {};
     slot_tag[s] = new_tag();
     return alien_hip::HostPost{mail + 2 * s, slot_tag[s]};
   }
