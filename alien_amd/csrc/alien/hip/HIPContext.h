@@ -130,6 +130,17 @@ class DeviceArray {
     }
     m_n = n;
   }
+  // The same for workspace that its user can do without: false, and empty, where there is no memory for it.
+  bool try_resize(size_t n) {
+    try {
+      resize(n);
+    } catch (const Error& e) {
+      if (e.code != (int)hipErrorOutOfMemory) throw;
+      (void)hipGetLastError();
+      return false;
+    }
+    return true;
+  }
   void reset() {
     if (m_p && !BlockCache::get().give(m_dev, m_p, m_n * sizeof(T))) (void)hipFree(m_p);
     m_p = nullptr;
@@ -195,14 +206,9 @@ struct alien_hip_ctx {
     if (capturing()) return false;
     const size_t have = ilu_piv.empty() ? 0 : ilu_piv.back().size();
     if (have >= rows) return true;
-    try {
-      alien_hip::DeviceArray<double> more(std::max(rows, 2 * have));
-      ilu_piv.push_back(std::move(more));
-    } catch (const alien_hip::Error& e) {
-      if (e.code != (int)hipErrorOutOfMemory) throw;
-      (void)hipGetLastError();
-      return false;
-    }
+    alien_hip::DeviceArray<double> more;
+    if (!more.try_resize(std::max(rows, 2 * have))) return false;
+    ilu_piv.push_back(std::move(more));
     return true;
   }
   bool capturing() const {

@@ -56,19 +56,7 @@ class ILU0Preconditioner<HIPInternalLinearAlgebra> {
       buildLevelSweeps(st, false); // the colour classes as the levels
       return;
     }
-    if (buildPencils(st)) return;
-    std::vector<int> level(n);
-    m_nl = alien_hip::host_levels(n, m_A.kcol(), m_A.cols(), m_A.dcol(), 0, level.data());
-    m_lptr.resize(m_nl + 1);
-    std::vector<int> rows(n);
-    alien_hip::group_by_level(n, level.data(), m_nl, m_lptr.data(), rows.data());
-    d_lrows.upload(rows.data(), rows.size(), st);
-    m_nu = alien_hip::host_levels(n, m_A.kcol(), m_A.cols(), m_A.dcol(), 1, level.data());
-    m_uptr.resize(m_nu + 1);
-    alien_hip::group_by_level(n, level.data(), m_nu, m_uptr.data(), rows.data());
-    d_urows.upload(rows.data(), rows.size(), st);
-    factorize(st);
-    buildLevelSweeps(st, true);
+    if (!buildPencils(st)) buildLevels(st);
   }
   void update() {}
   void solve(AlgebraType& alg, const VectorType& y, VectorType& x) const {
@@ -142,18 +130,23 @@ class ILU0Preconditioner<HIPInternalLinearAlgebra> {
   // (kernels/pencil.hip); no level sets are built then
   bool pencils() const { return m_pencil; }
   const alien_hip::PencilFactor<double>& pencilFactor() const { return m_pen; }
-  // the same factor in FP32, with its own faces and tickets
-  alien_hip::PencilFactor<float> pencilF32(hipStream_t st, alien_hip::DeviceArray<float>& vals,
-                                           alien_hip::DeviceArray<int>& work) const {
+  // the same factor in FP32, with its own faces and tickets; false where there is no memory for it
+  bool pencilF32(hipStream_t st, alien_hip::DeviceArray<float>& vals, alien_hip::DeviceArray<int>& work,
+                 alien_hip::PencilFactor<float>& F) const {
     const alien_hip::PencilGrid& g = m_pen.g;
-    vals.resize(8 * g.positions() + 2 * g.halo());
+    if (!vals.try_resize(8 * g.positions() + 2 * g.halo())) return false;
     work.resize(alien_hip::kPencilWork);
-    alien_hip::PencilFactor<float> F{g, vals.data(), vals.data() + 7 * g.positions(),
-                                     vals.data() + 8 * g.positions(), d_order.data(), work.data()};
+    F = {g, vals.data(), vals.data() + 7 * g.positions(), vals.data() + 8 * g.positions(), d_order.data(), work.data()};
     alien_hip::launch_pencil_init<float>(st, F);
     alien_hip::launch_pencil_demote(st, m_pen, F.base);
     alien_hip::check_launch("ilu0 pencils (FP32)");
-    return F;
+    return true;
+  }
+  // the factor and its sweeps over level sets after all (they take less memory on thin grids)
+  void leavePencils() {
+    m_pencil = false;
+    d_pen.reset();
+    buildLevels(m_alg.stream());
   }
 
  private:
@@ -175,10 +168,13 @@ class ILU0Preconditioner<HIPInternalLinearAlgebra> {
     if (bad[0]) return false;
     const std::vector<int> order = alien_hip::pencil_order(g);
     d_order.upload(order.data(), order.size(), st);
-    d_pen.resize(8 * g.positions() + 2 * g.halo());
+    alien_hip::DeviceArray<double> trans;
+    if (!d_pen.try_resize(8 * g.positions() + 2 * g.halo()) || !trans.try_resize(3 * g.positions())) {
+      d_pen.reset();
+      return false;
+    }
     m_pen = {g, d_pen.data(), d_pen.data() + 7 * g.positions(), d_pen.data() + 8 * g.positions(), d_order.data(),
              d_penwork.data()};
-    alien_hip::DeviceArray<double> trans(3 * g.positions());
     alien_hip::launch_pencil_init<double>(st, m_pen);
     alien_hip::launch_pencil_factor(st, m_pen, m_A.d_ro.data(), m_A.d_vals.data(), trans.data(), false);
     alien_hip::check_launch("ilu0 pencils factor");
@@ -189,6 +185,21 @@ class ILU0Preconditioner<HIPInternalLinearAlgebra> {
     m_pencil = true;
     return true;
   }
+  void buildLevels(hipStream_t st) {
+    const int n = m_A.getNRows();
+    std::vector<int> level(n);
+    m_nl = alien_hip::host_levels(n, m_A.kcol(), m_A.cols(), m_A.dcol(), 0, level.data());
+    m_lptr.resize(m_nl + 1);
+    std::vector<int> rows(n);
+    alien_hip::group_by_level(n, level.data(), m_nl, m_lptr.data(), rows.data());
+    d_lrows.upload(rows.data(), rows.size(), st);
+    m_nu = alien_hip::host_levels(n, m_A.kcol(), m_A.cols(), m_A.dcol(), 1, level.data());
+    m_uptr.resize(m_nu + 1);
+    alien_hip::group_by_level(n, level.data(), m_nu, m_uptr.data(), rows.data());
+    d_urows.upload(rows.data(), rows.size(), st);
+    factorize(st);
+    buildLevelSweeps(st, true);
+  }
   void factorize(hipStream_t st) {
     d_lptr.upload(m_lptr.data(), m_lptr.size(), st);
     d_uptr.upload(m_uptr.data(), m_uptr.size(), st);
@@ -198,8 +209,7 @@ class ILU0Preconditioner<HIPInternalLinearAlgebra> {
     const int n = m_A.getNRows();
     alien_hip::DeviceArray<double> piv;
     alien_hip::DeviceArray<int> work;
-    if (alien_hip::sync_levels(n, m_nl)) {
-      piv.resize(n);
+    if (alien_hip::sync_levels(n, m_nl) && piv.try_resize(n)) {
       work.resize(2);
       alien_hip::launch_sync_factor(st, n, m_nl, d_lrows.data(), m_A.d_ro.data(), m_A.d_cols.data(),
                                     m_A.d_dcol.data(), d_lu.data(), piv.data(), work.data());

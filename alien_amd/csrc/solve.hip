@@ -379,7 +379,7 @@ struct FusedCG {
       std::copy_n(P.a.begin(), P.order, res_cheb.a);
       std::copy_n(P.b.begin(), P.order, res_cheb.b);
     }
-    if (resident && !res.one) ex.resize((size_t)n * res.exchange);
+    if (resident && !res.one) resident = ex.try_resize((size_t)n * res.exchange);
   }
   // Small and middle-sized systems: the iterations run in one launch (cg_resident.hip) instead of
   // being launched one by one or from a graph
@@ -1381,10 +1381,10 @@ void solve_on(alien_hip_ctx* ctx, const alien_hip_solve_params* p, HIPMatrix& A,
       phase("ILU0 level-set factorisation");
       ps.kind = kPrecILU0Level;
       LevelILU& L = ps.lev;
+      if (mixed && ilu->pencils() && !ilu->pencilF32(ctx->stream, lev_l32, lev_work32, L.pen32)) ilu->leavePencils();
       L.pencils = ilu->pencils();
       if (L.pencils) {
         L.pen64 = ilu->pencilFactor();
-        if (mixed) L.pen32 = ilu->pencilF32(ctx->stream, lev_l32, lev_work32);
       } else {
         L.nl = ilu->lowerLevels();
         L.nu = ilu->upperLevels();

@@ -1,7 +1,10 @@
 // What calls leave in the state of a context: calls off the straight path (a wait given up, a stream capture, a second
-// context, a result in its operand's place), followed by ordinary ones on the same context. Prints one JSON object per check on stdout
-// for tests/test_gpu_ctx_state.py. The internal headers give the checks the context's own fields.
+// context, a result in its operand's place, a device without memory), followed by ordinary ones on the same context.
+// Prints one JSON object per check on stdout for tests/test_gpu_ctx_state.py. The internal headers give the checks the
+// context's own fields.
 // Usage: ctx_state_check [check ...]  (all of them without an argument; blocking_wait has to come first)
+#include <dlfcn.h>
+
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
@@ -16,6 +19,17 @@
 #include "alien/hip/HIPBackEnd.h"
 #include "alien/hip/krylov/HIPILU0Preconditioner.h"
 #include "kernels/resident_turn.h"
+
+// Device allocations of `refuse` bytes end as those of a device without memory (this definition comes before the runtime's).
+static size_t refuse = 0;
+static int refused = 0;
+extern "C" hipError_t hipMalloc(void** p, size_t bytes) {
+  typedef hipError_t (*Malloc)(void**, size_t);
+  static const Malloc real = (Malloc)dlsym(RTLD_NEXT, "hipMalloc");
+  if (bytes != refuse || bytes == 0) return real(p, bytes);
+  ++refused;
+  return real(p, size_t(1) << 46);
+}
 
 namespace {
 
@@ -337,6 +351,60 @@ void widths_in_one_launch() {
   std::printf("]}\n");
 }
 
+// Without the memory for a faster form's workspace, calls run in the form that needs none, to the same bits.
+void without_memory() {
+  int failed = 0, same = 1;
+  auto without = [&](size_t bytes, auto f) {
+    refuse = bytes;
+    refused = 0;
+    auto r = f();
+    failed += refused > 0;
+    refuse = 0;
+    return r;
+  };
+  const System a = generate(ALIEN_HIP_GEN_CONVDIFF7, 21, 18, 19, 9), s = generate(ALIEN_HIP_GEN_LOGNORMAL7, 21, 18, 19, 9);
+  { // the ILU(0) entry points' pivots
+    std::vector<int> dcol(a.n), level(a.n), rows(a.n);
+    alien_hip::host_dcol(a.n, a.ro.data(), a.cols.data(), dcol.data());
+    const int nl = alien_hip::host_levels(a.n, a.ro.data(), a.cols.data(), dcol.data(), 0, level.data());
+    std::vector<int> ptr(nl + 1);
+    alien_hip::group_by_level(a.n, level.data(), nl, ptr.data(), rows.data());
+    auto factor = [&] {
+      Context c;
+      alien_hip::DeviceArray<int> ro, cols, d, r;
+      alien_hip::DeviceArray<double> lu;
+      ro.upload(a.ro.data(), a.ro.size(), c->stream);
+      cols.upload(a.cols.data(), a.cols.size(), c->stream);
+      d.upload(dcol.data(), dcol.size(), c->stream);
+      r.upload(rows.data(), rows.size(), c->stream);
+      lu.upload(a.vals.data(), a.vals.size(), c->stream);
+      call(alien_hip_ilu0_factor_f64(c.c, a.n, ro.data(), cols.data(), d.data(), lu.data(), nl, ptr.data(), r.data()),
+           "ilu0_factor");
+      return read(lu);
+    };
+    same &= without(sizeof(double) * a.n, factor) == factor();
+  }
+  auto bicg = [&](int mode) {
+    Context c;
+    Solved r;
+    r.x.assign(a.n, 0.0);
+    alien_hip_solve_params p = params(ALIEN_HIP_PREC_ILU0, mode, 1e-10);
+    p.solver = ALIEN_HIP_BICGS;
+    call(alien_hip_solve_csr(c.c, &p, a.n, a.ro.data(), a.cols.data(), a.vals.data(), a.b.data(), r.x.data(), &r.r),
+         "solve_csr");
+    return r;
+  };
+  alien_hip::PencilGrid g;
+  same &= alien_hip::pencil_grid(a.n, a.ro.data(), a.cols.data(), g);
+  const size_t words = 8 * g.positions() + 2 * g.halo();
+  same &= without(sizeof(double) * words, [&] { return bicg(ALIEN_HIP_MODE_GRAPH); }) == bicg(ALIEN_HIP_MODE_GRAPH);
+  same &= without(sizeof(double) * 3 * g.positions(), [&] { return bicg(ALIEN_HIP_MODE_GRAPH); }) == bicg(ALIEN_HIP_MODE_GRAPH);
+  same &= without(sizeof(float) * words, [&] { return bicg(ALIEN_HIP_MODE_MIXED); }) == bicg(ALIEN_HIP_MODE_MIXED);
+  Context c; // the exchange vectors of CG in one launch
+  same &= without(sizeof(double) * 2 * s.n, [&] { return solve(c, s, ALIEN_HIP_MODE_GRAPH); }) == solve(c, s, ALIEN_HIP_MODE_GRAPH);
+  std::printf("{\"check\": \"without_memory\", \"refused\": %d, \"same\": %d}\n", failed, same);
+}
+
 const std::map<std::string, std::function<void()>> kChecks = {
     {"after_a_wait_given_up", after_a_wait_given_up},
     {"blocking_wait", blocking_wait},
@@ -348,6 +416,7 @@ const std::map<std::string, std::function<void()>> kChecks = {
     {"pencils_in_place", pencils_in_place},
     {"small_solves_take_their_share", small_solves_take_their_share},
     {"widths_in_one_launch", widths_in_one_launch},
+    {"without_memory", without_memory},
 };
 
 } // namespace

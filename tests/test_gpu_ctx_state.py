@@ -70,3 +70,8 @@ def test_blocking_wait():
 def test_widths_in_one_launch():
     """Rows of up to 7 entries (6 and 7 of 6 to 9, each in one workgroup and in several)."""
     assert run("widths_in_one_launch") == {"taken": [1, 1, 1, 1, 0, 0, 0, 0]}
+
+
+def test_without_memory():
+    """Factorisation entry point, FP64 and FP32 pencils and their set-up, resident CG: each refused its workspace once."""
+    assert run("without_memory") == {"refused": 5, "same": 1}
