@@ -49,10 +49,15 @@ __device__ __forceinline__ int csr_block() {
 // makes every load of a wavefront touch 64 rows and waits for each entry in turn. Bound by HBM:
 // the 7-point 160^3 matrix (424 MB) takes 78 us, 5.5 TB/s (walk: 221 us, 1.9 TB/s); FP32 60 us.
 // kCsrStageRow: runs of more than this many entries a row on average keep the walk: with rows that
-// long a tile holds few of them, so most lanes would wait while a few add.
+// long a tile holds few of them, so most lanes would wait while a few add. Runs of up to kCsrWalkRow a row keep it too:
+// each of their loads is coalesced as it is. In between, a run of up to half a tile takes as many rounds as it has
+// entries for (with all of them, clamped, it was slower than the walk up to four entries a row). 2,000,000 rows of a band,
+// FP64, us, walk / all rounds / now: 1 entry a row 11.1 / 26.3 / 11.1, 2 17.5 / 27.6 / 15.2, 3 23.4 / 29.9 / 20.8,
+// 4 29.6 / 32.1 / 23.0; FP32 8.5 / 14.5 / 8.6, 13.7 / 15.3 / 11.7, 18.3 / 17.1 / 15.4, 27.9 / 18.6 / 17.4.
 constexpr int kCsrUnroll = 8;
 constexpr int kCsrTile = kCsrUnroll * kBlock;
 constexpr int kCsrStageRow = 64;
+constexpr int kCsrWalkRow = 1;
 
 // Row sum of row r0 + threadIdx.x (r0: the workgroup's first row, < n). Every lane of the
 // workgroup calls it.
@@ -64,8 +69,30 @@ __device__ __forceinline__ T csr_row_sum(unsigned n, unsigned r0, const int* __r
   const unsigned kb = ro[min(r0 + tid, n)], ke = ro[min(r0 + tid + 1, n)];
   const unsigned first = ro[r0], last = ro[min(r0 + kBlock, n)];
   T acc = 0;
-  if (last - first > kCsrStageRow * kBlock) {
+  auto walk = [&] {
     for (unsigned k = kb; k < ke; ++k) acc = acc + vals[k] * x[cols[k]];
+    return acc;
+  };
+  if (last - first > kCsrStageRow * kBlock) return walk();
+  if (last - first <= kCsrTile / 2) {
+    auto pass = [&](auto rounds) {
+      constexpr int R = decltype(rounds)::value;
+      int c[R];
+      T v[R];
+#pragma unroll
+      for (int u = 0; u < R; ++u) {
+        const unsigned k = min(first + u * kBlock + tid, last - 1);
+        c[u] = stream_load(cols + k);
+        v[u] = stream_load(vals + k);
+      }
+#pragma unroll
+      for (int u = 0; u < R; ++u) prod[u * kBlock + tid] = v[u] * x[c[u]];
+    };
+    if (last - first <= kCsrWalkRow * kBlock) return walk();
+    if (last - first <= kCsrTile / 4) pass(std::integral_constant<int, kCsrUnroll / 4>{});
+    else pass(std::integral_constant<int, kCsrUnroll / 2>{});
+    __syncthreads();
+    for (unsigned k = kb; k < ke; ++k) acc = acc + prod[k - first];
     return acc;
   }
   for (unsigned t0 = first; t0 < last; t0 += kCsrTile) {
@@ -421,7 +448,10 @@ struct Vec4<float> { typedef float4 type; typedef float2 half; };
 // (32 bytes a lane in FP64), and each lane adds its own scalar row's products in the reference's
 // order (block by block, column 0 then 1): the sequential sum bit for bit. Bound by HBM: 97 x 93 x
 // 101 cells, 7 blocks a row (260 MB), 46 us, 5.6 TB/s (one lane a block row walking: 133 us, 2.0 TB/s). Runs of more than
-// kBsrStageRow blocks a block row keep the walk, one lane a block row.
+// kBsrStageRow blocks a block row keep the walk, one lane a block row. Short runs as in csr_row_sum; with one or two blocks a
+// block row on 300,000 of them or more the walk would still be faster (900,973, FP64: 10.7 against 15.8 us with one, 17.0
+// against 20.0 with two; FP32 5.0 against 9.0, 10.9 against 11.5): the wavefronts, two for each of its one, take that long to
+// start. Twice the rows a workgroup, which has no more wavefronts than the walk, took 49 us for the grid above.
 constexpr int kBsrRows = kBlock / 2;
 constexpr int kBsrUnroll = 4;
 constexpr int kBsrTile = kBsrUnroll * kBlock;
@@ -434,6 +464,15 @@ __global__ void __launch_bounds__(kBlock) k_spmv_bsr2(int nb, const int* __restr
   typedef typename Vec4<T>::type V4;
   typedef typename Vec4<T>::half V2;
   __shared__ V2 prod[2 * kBsrTile]; // block k of the tile: scalar row 0's products at 2 k, row 1's at 2 k + 1
+  auto stage = [&](unsigned at, const V4& m, const V2& xv) {
+    V2 p0, p1;
+    p0.x = m.x * xv.x;
+    p0.y = m.z * xv.y;
+    p1.x = m.y * xv.x;
+    p1.y = m.w * xv.y;
+    prod[2 * at] = p0;
+    prod[2 * at + 1] = p1;
+  };
   const unsigned n = nb, r0 = (unsigned)csr_block() * kBsrRows;
   if (r0 >= n) return;
   const unsigned tid = threadIdx.x;
@@ -461,6 +500,34 @@ __global__ void __launch_bounds__(kBlock) k_spmv_bsr2(int nb, const int* __restr
   const unsigned i = r0 + tid / 2, half = tid & 1;
   const unsigned kb = ro[min(i, n)], ke = ro[min(i + 1, n)];
   T acc = 0;
+  if (last - first <= kBsrTile / 2) {
+    // short runs, as in csr_row_sum
+    auto pass = [&](auto rounds) {
+      constexpr int R = decltype(rounds)::value;
+      int c[R];
+      V4 m[R];
+#pragma unroll
+      for (int u = 0; u < R; ++u) {
+        const unsigned k = min(first + u * kBlock + tid, last - 1);
+        c[u] = stream_load(cols + k);
+        m[u] = reinterpret_cast<const V4*>(vals)[k];
+      }
+#pragma unroll
+      for (int u = 0; u < R; ++u) stage(u * kBlock + tid, m[u], reinterpret_cast<const V2*>(x)[c[u]]);
+    };
+    if (last > first) {
+      if (last - first <= kBsrTile / 4) pass(std::integral_constant<int, kBsrUnroll / 4>{});
+      else pass(std::integral_constant<int, kBsrUnroll / 2>{});
+    }
+    __syncthreads();
+    for (unsigned k = kb; k < ke; ++k) {
+      const V2 p = prod[2 * (k - first) + half];
+      acc = acc + p.x;
+      acc = acc + p.y;
+    }
+    if (i < n) y[2 * (size_t)i + half] = acc;
+    return;
+  }
   for (unsigned t0 = first; t0 < last; t0 += kBsrTile) {
     int c[kBsrUnroll];
     V4 m[kBsrUnroll];
@@ -471,16 +538,7 @@ __global__ void __launch_bounds__(kBlock) k_spmv_bsr2(int nb, const int* __restr
       m[u] = reinterpret_cast<const V4*>(vals)[k];
     }
 #pragma unroll
-    for (int u = 0; u < kBsrUnroll; ++u) {
-      const V2 xv = reinterpret_cast<const V2*>(x)[c[u]];
-      V2 p0, p1;
-      p0.x = m[u].x * xv.x;
-      p0.y = m[u].z * xv.y;
-      p1.x = m[u].y * xv.x;
-      p1.y = m[u].w * xv.y;
-      prod[2 * (u * kBlock + tid)] = p0;
-      prod[2 * (u * kBlock + tid) + 1] = p1;
-    }
+    for (int u = 0; u < kBsrUnroll; ++u) stage(u * kBlock + tid, m[u], reinterpret_cast<const V2*>(x)[c[u]]);
     __syncthreads();
     const unsigned e = min(ke, t0 + kBsrTile);
     for (unsigned k = max(kb, t0); k < e; ++k) {
