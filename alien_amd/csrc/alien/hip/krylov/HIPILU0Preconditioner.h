@@ -210,7 +210,7 @@ class ILU0Preconditioner<HIPInternalLinearAlgebra> {
     alien_hip::DeviceArray<double> piv;
     alien_hip::DeviceArray<int> work;
     if (alien_hip::sync_levels(n, m_nl) && piv.try_resize(n)) {
-      work.resize(2);
+      work.resize(alien_hip::kSyncWork);
       alien_hip::launch_sync_factor(st, n, m_nl, d_lrows.data(), m_A.d_ro.data(), m_A.d_cols.data(),
                                     m_A.d_dcol.data(), d_lu.data(), piv.data(), work.data());
     } else {

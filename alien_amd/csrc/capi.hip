@@ -55,7 +55,7 @@ alien_hip_ctx* make_ctx(void* stream) {
                                   hipHostMallocCoherent));
     std::fill_n(c->mail, alien_hip_ctx::kMailWords, 0ull);
     // (last: taken before the tickets it moved them to where a hand-written step of 101 x 99 x 103 took 57.2 us, not 56.4)
-    c->ilu_work.resize(2);
+    c->ilu_work.resize(kSyncWork);
     ALIEN_HIP_CHECK(hipStreamSynchronize(c->stream));
   } catch (...) {
     destroy_ctx(c);

@@ -9,12 +9,14 @@
 // 4.69 -> 1.21 ms. Waiting for a row's entries in turn, and looking its matches up after the wait,
 // took 2.9 and 19 us per level.
 // Waits are bounded; one that runs out raises a flag, and a wavefront then does in order what is
-// left.
+// left. Matrices whose rows update more than their pivots are factorised a wavefront per row (k_sync_factor_rows).
 #include "../alien_hip_internal.h"
 #include "../alien/hip/HIPContext.h"
 #include "device_common.h"
 #include "launch.h"
 #include "sync_free.h"
+
+#include <algorithm>
 
 namespace alien_hip {
 
@@ -122,10 +124,36 @@ __device__ __forceinline__ void look_up(ShortFactor& f, int i, int rb, int di, i
   }
 }
 
+// As k_sync_fill before a factorisation; work[2]: whether more than an eighth of 256 rows spread over the matrix are not
+// plain ones. It chooses between two kernels that take any row (a host that chose would have to read the matrix back).
+constexpr int kSyncSample = kBlock;
+__global__ void __launch_bounds__(kBlock) k_sync_factor_start(int n, const int* __restrict__ ro,
+                                                               const int* __restrict__ cols, const int* __restrict__ dcol,
+                                                               const double* __restrict__ lu, double* piv, int* work) {
+  for (long i = (long)blockIdx.x * kBlock + threadIdx.x; i < n; i += (long)gridDim.x * kBlock)
+    reinterpret_cast<U*>(piv)[i] = B::kSentinel;
+  if (blockIdx.x != 0) return;
+  const int sample = min(n, kSyncSample);
+  bool other = false;
+  if ((int)threadIdx.x < sample) {
+    const int i = (int)((long)threadIdx.x * n / sample), rb = ro[i], di = dcol[i];
+    int col[kSyncSlots];
+#pragma unroll
+    for (int s = 0; s < kSyncSlots; ++s) col[s] = rb + s < di ? cols[rb + s] : -1;
+    ShortFactor f;
+    look_up(f, i, rb, di, ro[i + 1], ro, cols, dcol, lu, col);
+    other = !f.plain;
+  }
+  const int others = __syncthreads_count(other);
+  if (threadIdx.x < 2) work[threadIdx.x] = 0;
+  if (threadIdx.x == 2) work[2] = 8 * others > sample;
+}
+
 __global__ void __launch_bounds__(kBlock) k_sync_factor(int n, const int* __restrict__ rows,
                                                          const int* __restrict__ ro, const int* __restrict__ cols,
                                                          const int* __restrict__ dcol, double* lu, double* piv,
                                                          int* work, long limit) {
+  if (work[2]) return;
   const int lane = threadIdx.x & (kWave - 1);
   const U* pv = reinterpret_cast<const U*>(piv);
   for (int c; (long)(c = next_chunk(work)) * kWave < n;) {
@@ -179,6 +207,85 @@ __global__ void __launch_bounds__(kBlock) k_sync_factor(int n, const int* __rest
         }
       }
       if (wait_over(spins, limit, work + 1)) open = false;
+    }
+  }
+}
+
+// A row by a wavefront, an entry per lane, for matrices whose rows are mostly not plain: a lane that merges the rows of one
+// of its own alone takes 150 us a row of 27 entries, as in the level kernels, and the lanes of a wavefront whose rows
+// become ready at different times take turns at that. Per lower entry, in order: the entries to its right of
+// that column's row, found by comparing columns across the lanes (the next such row's are asked for meanwhile), and
+// one trip for their values. `per` rows a ticket. Rows of more entries than lanes are left to one lane (factor_row).
+// Bound by that chain, about 1 us a lower entry. Launches per level, lanes as in k_sync_factor, this: 27-point 40^3 45.6,
+// 63.5, 4.8 ms; 9-point 400 x 400 22.6, 26.9, 5.4; 20,000 rows of 41 entries, 1000 levels, 267, 4760 (waits given up), 29.
+__device__ __forceinline__ double of_lane(double v, int lane) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const unsigned lo = __builtin_amdgcn_readlane((int)(unsigned)b, lane), hi = __builtin_amdgcn_readlane((int)(unsigned)(b >> 32), lane);
+  return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
+}
+__global__ void __launch_bounds__(kBlock) k_sync_factor_rows(int n, int per, const int* __restrict__ rows,
+                                                              const int* __restrict__ ro, const int* __restrict__ cols,
+                                                              const int* __restrict__ dcol, double* lu, double* piv,
+                                                              int* work, long limit) {
+  if (!work[2]) return;
+  const int lane = threadIdx.x & (kWave - 1);
+  const U* pv = reinterpret_cast<const U*>(piv);
+  U* lv = reinterpret_cast<U*>(lu);
+  for (int c; (long)(c = next_chunk(work)) * per < n;) {
+    const long end = min((long)n, ((long)c + 1) * per);
+    for (long q = (long)c * per; q < end; ++q) {
+      const int i = rows[q], rb = ro[i], di = dcol[i], re = ro[i + 1];
+      bool there = true;
+      for (int k0 = rb; k0 < di && there; k0 += kWave) {
+        const bool on = k0 + lane < di;
+        const int col = on ? cols[k0 + lane] : 0;
+        long spins = 0;
+        while (there && __any(on && agent_load(pv + col) == B::kSentinel)) there = !wait_over(spins, limit, work + 1);
+      }
+      if (!there) continue; // given up, not touched
+      if (re - rb > kWave) {
+        if (lane == 0) factor_row(i, ro, cols, dcol, lu, piv);
+        continue;
+      }
+      const int low = di - rb, j = rb + lane;
+      const bool has = j < re;
+      const int cj = has ? cols[j] : -1;
+      double v = has ? lu[j] : 0.0;
+      int ub = 0, ue = 0; // of a lower entry's lane: the entries of its column's row beyond the diagonal
+      double pk = 1.0;    // and that row's pivot
+      if (lane < low) {
+        ub = dcol[cj] + 1;
+        ue = ro[cj + 1];
+        pk = B::value(agent_load(pv + cj));
+      }
+      auto column = [&](int t, int p0) { // this lane's of those entries, from p0 on
+        const int p = p0 + lane;
+        return p < __builtin_amdgcn_readlane(ue, t) ? cols[p] : -2;
+      };
+      bool touched = false;
+      int cp = low > 0 ? column(0, __builtin_amdgcn_readlane(ub, 0)) : -2;
+      for (int t = 0; t < low; ++t) {
+        const int b = __builtin_amdgcn_readlane(ub, t), e = __builtin_amdgcn_readlane(ue, t);
+        const double a = of_lane(v, t) / of_lane(pk, t);
+        if (lane == t) v = a;
+        int at = -1;
+        for (int p0 = b; p0 < e; p0 += kWave) {
+          if (p0 > b) cp = column(t, p0);
+          const int m = min(e - p0, kWave);
+          for (int u = 0; u < m; ++u)
+            if (lane > t && cj == __builtin_amdgcn_readlane(cp, u)) at = p0 + u;
+        }
+        if (t + 1 < low) cp = column(t + 1, __builtin_amdgcn_readlane(ub, t + 1));
+        if (at >= 0) {
+          v = v - a * B::value(agent_load(lv + at));
+          touched = true;
+        }
+      }
+      if (has && lane <= low) lu[j] = v;
+      const bool out = has && lane > low && touched;
+      if (out) agent_store(lv + j, B::bits(v));
+      if (__any(out)) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      if (lane == low) agent_store(reinterpret_cast<U*>(piv) + i, B::bits(v));
     }
   }
 }
@@ -270,6 +377,10 @@ __global__ void __launch_bounds__(kWave) k_sync_sweep_rest(int n, const int* row
     }
 }
 
+// Polls of a wait here: a row may wait for all of the thousands taken before it, each taking as long as its
+// entries make it (with the level-ordered sweeps' number of polls 20,000 rows of 41 entries gave up and took 4.8 s).
+static long sync_spins() { return 64 * g_ilu_sf_spins; }
+
 // Lanes for about ten levels' rows (a row's entries are looked up ahead of its turn), 64 to 256
 // workgroups, never more waves than chunks; ALIEN_HIP_ILU_SF_BLOCKS overrides. Factorisation and solve
 // of the 7-point 96^3 matrix: 2.58 ms with 48 workgroups, 2.31 with 64, 2.12 with 128, 2.22 with 192;
@@ -282,16 +393,26 @@ static dim3 sync_grid(int n, int nlevels) {
   return dim3((unsigned)std::max(1L, std::min(blocks, (chunks + waves - 1) / waves)));
 }
 
-// Levels of more rows than this on average are launched one by one (few, and each fills the device).
+// Levels of more rows than this on average are launched one by one (few, and each fills the device). 2,000,000 rows of
+// three entries, a launch each and one launch, us, by rows a level: 12,000 factorisation 621 and 410, solve 1007 and 770;
+// 16,000 470 and 409, 752 and 771; 20,000 386 and 407, 611 and 767; 32,000 254 and 406, 398 and 764.
+constexpr long kSyncAvgRows = 16384;
 bool sync_levels(int n, int nlevels) {
-  return g_ilu_sync_free && nlevels > 2 && n > 0 && n <= g_ilu_sf_avg_rows * nlevels;
+  return g_ilu_sync_free && nlevels > 2 && n > 0 && n <= std::min(g_ilu_sf_avg_rows, kSyncAvgRows) * nlevels;
 }
 
 void launch_sync_factor(hipStream_t st, int n, int nlevels, const int* rows, const int* ro, const int* cols,
                         const int* dcol, double* lu, double* piv, int* work) {
-  hipLaunchKernelGGL(k_sync_fill, dim3(grid_for(n, 4)), dim3(kBlock), 0, st, n, piv, work);
+  hipLaunchKernelGGL(k_sync_factor_start, dim3(grid_for(n, 4)), dim3(kBlock), 0, st, n, ro, cols, dcol, (const double*)lu,
+                     piv, work);
   hipLaunchKernelGGL(k_sync_factor, sync_grid(n, nlevels), dim3(kBlock), 0, st, n, rows, ro, cols, dcol, lu, piv, work,
-                     g_ilu_sf_spins);
+                     sync_spins());
+  // a wavefront per row of about ten levels, 256 to 2048 of them
+  const long avg = n / std::max(1, nlevels), waves = kBlock / kWave;
+  const int per = (int)std::min(16L, std::max(1L, avg / 2048));
+  const long blocks = std::min((10 * avg / per + waves - 1) / waves, 512L), most = ((long)n / per + waves) / waves;
+  hipLaunchKernelGGL(k_sync_factor_rows, dim3((unsigned)std::max(1L, std::min(std::max(blocks, 64L), most))), dim3(kBlock), 0,
+                     st, n, per, rows, ro, cols, dcol, lu, piv, work, sync_spins());
   hipLaunchKernelGGL(k_sync_factor_rest, dim3(1), dim3(kWave), 0, st, n, rows, ro, cols, dcol, lu, piv, work);
 }
 
@@ -300,7 +421,7 @@ static void sync_sweep(hipStream_t st, int n, int nlevels, const int* rows, cons
                        const int* dcol, const double* lu, const double* in, double* out, int* work) {
   hipLaunchKernelGGL(k_sync_fill, dim3(grid_for(n, 4)), dim3(kBlock), 0, st, n, out, work);
   hipLaunchKernelGGL(k_sync_sweep<UPPER>, sync_grid(n, nlevels), dim3(kBlock), 0, st, n, rows, ro, cols, dcol, lu, in,
-                     out, work, g_ilu_sf_spins);
+                     out, work, sync_spins());
   hipLaunchKernelGGL(k_sync_sweep_rest<UPPER>, dim3(1), dim3(kWave), 0, st, n, rows, ro, cols, dcol, lu, in, out, work);
 }
 

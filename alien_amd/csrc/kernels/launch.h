@@ -208,8 +208,9 @@ void launch_ilu0_solve_lev(hipStream_t, int nl, const int* lptr_host, const int*
                            const int* uptr_host, const int* uptr_dev, LevelSweep<T> U, const T* y, T* t, T* x,
                            const int* done = nullptr, int* sf_work = nullptr);
 // ILU(0) over CSR arrays and level schedules in one launch each (ilu0_sync.hip), where sync_levels
-// says so: small levels. piv: n doubles, work: two ints of workspace. The sweeps write their results
+// says so: small levels. piv: n doubles, work: kSyncWork ints of workspace. The sweeps write their results
 // over sentinels, so a sweep's output may not be its input (x may be y).
+constexpr int kSyncWork = 3; // ticket, flag of a wait given up, which kernel factorises
 bool sync_levels(int n, int nlevels);
 void launch_sync_factor(hipStream_t, int n, int nlevels, const int* rows, const int* ro, const int* cols,
                         const int* dcol, double* lu, double* piv, int* work);
