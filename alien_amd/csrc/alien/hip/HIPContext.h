@@ -307,6 +307,14 @@ struct alien_hip_ctx {
     fetch(mail + 2 * s, tag, dslot(s), &v, 2);
     return v;
   }
+  // The same in two halves: the words asked for (one such question at a time); looked at; waited for.
+  alien_hip::HostPost ask_words(const void* from, int n) {
+    const alien_hip::HostPost p{mail + 2 * kSlots, new_tag()};
+    alien_hip::launch_post_words(stream, from, n, p);
+    return p;
+  }
+  bool peek_words(const alien_hip::HostPost& p, void* to, int n) const { return arrived(p.to, p.tag, static_cast<unsigned*>(to), n); }
+  void take_words(const alien_hip::HostPost& p, const void* from, void* to, int n) { fetch(p.to, p.tag, from, to, n); }
   // n 32-bit words of device memory, likewise, and one from `also` (at most kMaxPostWords together).
   void read_words(const void* from, void* to, int n, const int* also = nullptr, int* also_to = nullptr) {
     const alien_hip::HostPost p{mail + 2 * kSlots, new_tag()};
@@ -316,6 +324,14 @@ struct alien_hip_ctx {
   }
 
  private:
+  static bool arrived(const unsigned long long* from, unsigned tag, unsigned* out, int n) {
+    for (int i = 0; i < n; ++i) {
+      const unsigned long long w = __atomic_load_n(from + i, __ATOMIC_ACQUIRE);
+      if ((unsigned)(w >> 32) != tag) return false;
+      out[i] = (unsigned)w;
+    }
+    return true;
+  }
   unsigned new_tag() { return last_tag += last_tag == ~0u ? 2 : 1; }
   // The words posted with this tag. The host polls memory: a stored word reaches it in about 2 us, where a
   // copy and a wait for the stream took 13 to 20. After about 1 ms, where those no longer matter, it waits for the
@@ -323,21 +339,13 @@ struct alien_hip_ctx {
   void fetch(const unsigned long long* from, unsigned tag, const void* dev, void* to, int n) {
     alien_hip::check_launch("post");
     unsigned* out = static_cast<unsigned*>(to);
-    auto arrived = [&] {
-      for (int i = 0; i < n; ++i) {
-        const unsigned long long w = __atomic_load_n(from + i, __ATOMIC_ACQUIRE);
-        if ((unsigned)(w >> 32) != tag) return false;
-        out[i] = (unsigned)w;
-      }
-      return true;
-    };
-    for (unsigned spin = 0; !arrived(); ++spin) {
+    for (unsigned spin = 0; !arrived(from, tag, out, n); ++spin) {
       if (spin < polls) {
         __builtin_ia32_pause();
         continue;
       }
       ALIEN_HIP_CHECK(hipStreamSynchronize(stream));
-      if (arrived()) break;
+      if (arrived(from, tag, out, n)) break;
       ALIEN_HIP_CHECK(hipMemcpyAsync(to, dev, sizeof(unsigned) * n, hipMemcpyDeviceToHost, stream));
       ALIEN_HIP_CHECK(hipStreamSynchronize(stream));
       return;

@@ -821,6 +821,8 @@ struct FusedBiCG {
   DeviceArray<T> r, r0, p, phat, v, sv, shat, t, tmp, tmp2, cp;
   DeviceArray<BiCGState> st;
   BiCGState* h_st = nullptr; // pinned
+  static constexpr int kStateWords = sizeof(BiCGState) / 4;
+  static_assert(kStateWords <= kMaxPostWords, "one post");
 
   FusedBiCG(alien_hip_ctx* c, int n_, RBMat<T> A_, const T* invd_, const PrecondSpec& P_)
   : ctx(c), n(n_), A(A_), invd(invd_), P(P_) {
@@ -884,8 +886,7 @@ struct FusedBiCG {
                       st.data());
   }
   BiCGState read_state() {
-    static_assert(sizeof(BiCGState) <= 4 * kMaxPostWords, "one post");
-    ctx->read_words(st.data(), h_st, (int)(sizeof(BiCGState) / 4));
+    ctx->read_words(st.data(), h_st, kStateWords);
     return *h_st;
   }
   // (the mirror is written again only after a read_state, which waits for this copy)
@@ -903,27 +904,42 @@ struct FusedBiCG {
     ge = nullptr;
     g = nullptr;
   }
-  void capture(T* x, int k) {
+  // the graph of k steps; none when `off` says during its capture that it will not be needed
+  template <typename F>
+  void capture(T* x, int k, F off) {
     if (ge && g_x == x && g_k == k) return;
     release_graph();
+    bool want = true;
     ALIEN_HIP_CHECK(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-    for (int i = 0; i < k; ++i) step(x);
+    for (int i = 0; i < k && want; ++i) {
+      step(x);
+      want = !off();
+    }
     ALIEN_HIP_CHECK(hipStreamEndCapture(ctx->stream, &g));
+    if (!want) {
+      release_graph();
+      return;
+    }
     ALIEN_HIP_CHECK(hipGraphInstantiate(&ge, g, nullptr, nullptr, 0));
     g_x = x;
     g_k = k;
   }
   // The first block, launched directly; the graph of k steps is captured while it runs (a graph of its own, captured,
-  // instantiated and destroyed for one step, left the device idle for 0.9 ms of a 128^3 solve's 6.5 with ILU(0)).
+  // instantiated and destroyed for one step, left the device idle for 0.9 ms of a 128^3 solve's 6.5 with ILU(0)), as long as
+  // its state has not come back as done (20 x 20 cells solved by the first block: 345 us with a graph of one step, 434 to
+  // 600 with the whole graph captured all the same, 360 now).
   BiCGState first_step(T* x, bool graph, int k) {
     step(x);
     check_launch("fused BiCGStab first step");
-    if (graph) capture(x, k);
-    return read_state();
+    if (!graph) return read_state();
+    const HostPost p = ctx->ask_words(st.data(), kStateWords);
+    capture(x, k, [&] { return ctx->peek_words(p, h_st, kStateWords) && h_st->done; });
+    ctx->take_words(p, st.data(), h_st, kStateWords);
+    return *h_st;
   }
   BiCGState advance(T* x, bool graph, int k) {
     if (graph) {
-      capture(x, k);
+      capture(x, k, [] { return false; });
       ALIEN_HIP_CHECK(hipGraphLaunch(ge, ctx->stream));
     } else {
       for (int i = 0; i < k; ++i) step(x);
