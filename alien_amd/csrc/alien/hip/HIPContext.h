@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cstddef>
 #include <map>
 #include <mutex>
@@ -226,7 +227,7 @@ struct alien_hip_ctx {
   static constexpr int kMailWords = 2 * 64 + alien_hip::kMaxPostWords;
   unsigned last_tag = 0, slot_tag[64] = {}; // tag of the post that fills a slot's words (0: none under way)
   unsigned waits = 0;
-  unsigned polls = 32768; // of posted words before a wait for the stream; none where the program asked for blocking waits
+  double poll_s = 4e-3; // a read polls its posted words as long before it waits for the stream; 0: the program asked for blocking waits
   alien_hip::DeviceArray<unsigned> tickets; // counters of the reductions finished in their own launch, zeros
   // Pinned 512-byte blocks for the fused solvers' host state mirrors, allocated once per context
   // (pinned allocation and release cost far more than a solve's own host work); a solver takes a
@@ -334,13 +335,15 @@ struct alien_hip_ctx {
   }
   unsigned new_tag() { return last_tag += last_tag == ~0u ? 2 : 1; }
   // The words posted with this tag. The host polls memory: a stored word reaches it in about 2 us, where a
-  // copy and a wait for the stream took 13 to 20. After about 1 ms, where those no longer matter, it waits for the
+  // copy and a wait for the stream took 13 to 20. After 4 ms, where those no longer matter, it waits for the
   // stream and leaves its core to others. A word that the finished stream has not posted is copied.
   void fetch(const unsigned long long* from, unsigned tag, const void* dev, void* to, int n) {
     alien_hip::check_launch("post");
     unsigned* out = static_cast<unsigned*>(to);
-    for (unsigned spin = 0; !arrived(from, tag, out, n); ++spin) {
-      if (spin < polls) {
+    const auto now = std::chrono::steady_clock::now;
+    const auto until = now() + std::chrono::duration<double>(poll_s);
+    for (unsigned spin = 1; !arrived(from, tag, out, n); ++spin) {
+      if (poll_s > 0 && (spin % 64 || now() < until)) {
         __builtin_ia32_pause();
         continue;
       }

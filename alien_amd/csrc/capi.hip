@@ -48,7 +48,7 @@ alien_hip_ctx* make_ctx(void* stream) {
     unsigned flags = 0;
     ALIEN_HIP_CHECK(hipGetDeviceFlags(&flags));
     flags &= hipDeviceScheduleMask;
-    if (flags == hipDeviceScheduleBlockingSync || flags == hipDeviceScheduleYield) c->polls = 0;
+    if (flags == hipDeviceScheduleBlockingSync || flags == hipDeviceScheduleYield) c->poll_s = 0;
     c->tickets.resize(kTicketWords);
     ALIEN_HIP_CHECK(hipMemsetAsync(c->tickets.data(), 0, sizeof(unsigned) * kTicketWords, c->stream));
     ALIEN_HIP_CHECK(hipHostMalloc((void**)&c->mail, sizeof(unsigned long long) * alien_hip_ctx::kMailWords,
