@@ -125,24 +125,24 @@ __device__ __forceinline__ void look_up(ShortFactor& f, int i, int rb, int di, i
 }
 
 // As k_sync_fill before a factorisation; work[2]: whether more than an eighth of 256 rows spread over the matrix are not
-// plain ones. It chooses between two kernels that take any row (a host that chose would have to read the matrix back).
+// plain ones, by the nearest row that each reads. It chooses between two kernels that take any row (a host that chose
+// would have to read the matrix back).
 constexpr int kSyncSample = kBlock;
 __global__ void __launch_bounds__(kBlock) k_sync_factor_start(int n, const int* __restrict__ ro,
                                                                const int* __restrict__ cols, const int* __restrict__ dcol,
-                                                               const double* __restrict__ lu, double* piv, int* work) {
+                                                               double* piv, int* work) {
   for (long i = (long)blockIdx.x * kBlock + threadIdx.x; i < n; i += (long)gridDim.x * kBlock)
     reinterpret_cast<U*>(piv)[i] = B::kSentinel;
   if (blockIdx.x != 0) return;
   const int sample = min(n, kSyncSample);
   bool other = false;
   if ((int)threadIdx.x < sample) {
-    const int i = (int)((long)threadIdx.x * n / sample), rb = ro[i], di = dcol[i];
-    int col[kSyncSlots];
-#pragma unroll
-    for (int s = 0; s < kSyncSlots; ++s) col[s] = rb + s < di ? cols[rb + s] : -1;
-    ShortFactor f;
-    look_up(f, i, rb, di, ro[i + 1], ro, cols, dcol, lu, col);
-    other = !f.plain;
+    const int i = (int)((long)threadIdx.x * n / sample), rb = ro[i], di = dcol[i], re = ro[i + 1];
+    const int near = di > rb ? cols[di - 1] : -1;
+    other = di - rb > kSyncSlots;
+    if (near >= 0)
+      for (int p = dcol[near] + 1, pe = ro[near + 1]; p < pe; ++p)
+        for (int j = di + 1, c = cols[p]; j < re; ++j) other = other || cols[j] == c;
   }
   const int others = __syncthreads_count(other);
   if (threadIdx.x < 2) work[threadIdx.x] = 0;
@@ -403,8 +403,8 @@ bool sync_levels(int n, int nlevels) {
 
 void launch_sync_factor(hipStream_t st, int n, int nlevels, const int* rows, const int* ro, const int* cols,
                         const int* dcol, double* lu, double* piv, int* work) {
-  hipLaunchKernelGGL(k_sync_factor_start, dim3(grid_for(n, 4)), dim3(kBlock), 0, st, n, ro, cols, dcol, (const double*)lu,
-                     piv, work);
+  hipLaunchKernelGGL(k_sync_factor_start, dim3(grid_for(n, 4)), dim3(kBlock), 0, st, n, ro, cols, dcol, piv,
+                     work);
   hipLaunchKernelGGL(k_sync_factor, sync_grid(n, nlevels), dim3(kBlock), 0, st, n, rows, ro, cols, dcol, lu, piv, work,
                      sync_spins());
   // a wavefront per row of about ten levels, 256 to 2048 of them
