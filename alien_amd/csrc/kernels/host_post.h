@@ -1,4 +1,4 @@
-// Words a kernel hands to a host thread that polls for them (alien_hip_ctx::wait_post).
+// Words a kernel hands to a host thread that polls for them (alien_hip_ctx::fetch).
 #pragma once
 
 namespace alien_hip {

@@ -46,7 +46,7 @@ bool pencil_grid(int n, const int* ro, const int* cols, PencilGrid& g) {
   g.py = (g.ny + kPen - 1) / kPen;
   g.pz = (g.nz + kPen - 1) / kPen;
   g.steps = (g.nx + kPenSkew + kPenChunk - 1) / kPenChunk * kPenChunk;
-  // thin grids whose padding would cost more memory than the level sets' lists are left to those
+  // thin grids are left to the level sets: at 8 positions a row the arrays take 0.5 KB a row, theirs 0.16
   return g.positions() <= 8L * n && g.positions() <= 0x7fffffffL;
 }
 
